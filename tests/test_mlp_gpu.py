@@ -61,6 +61,21 @@ def test_gradient_matches_oracle(h):
         assert err < 1e-6                    # measured <= 9e-8: FP32 accumulation only
 
 
+@pytest.mark.parametrize("n", [1, 32, 255, 256, 257, 544])
+def test_bias_gradients_at_the_edges_of_the_row_tiles(h, n):
+    # the bias gradients are column sums over the batch, taken 256 rows at a time; an
+    # activation that rounds to the neighbouring BF16 value moves outputs, and with them the
+    # gradients, by ~1e-4 (test_forward_matches_oracle's bound)
+    h.mlp_init(6)
+    w = h.mlp_params().astype(np.float64)
+    X, T, rank = _data(n, 2)
+    loss, g = h.mlp_loss_grad(X, T, rank)
+    lo, go = m.loss_grad(w, X, T, rank, bf16=True)
+    assert loss == pytest.approx(lo, rel=1e-4)
+    for a, b in ((BLOCKS[1], BLOCKS[2]), (BLOCKS[3], BLOCKS[4]), (BLOCKS[5], BLOCKS[6])):
+        assert P.rel_err(g[a:b].astype(np.float64), go[a:b]) < 5e-4
+
+
 def test_harvested_features_match_oracle(h):
     dims, R = [12, 10, 8], 3
     X, _ = o.make_tensor(dims, R, seed=3, snr_db=30.0)
