@@ -530,6 +530,23 @@ def test_als_other_constraints(h, cons):
                 assert np.allclose(ratio, ratio[0:1, :], rtol=1e-12)
 
 
+@pytest.mark.parametrize("R", [1, 2, 3, 15, 16, 17, 32, 33, 63, 64])
+def test_orthogonal_update_is_the_polar_factor_at_every_padded_rank(h, R):
+    """One update of mode 0 under the orthogonality constraint, A = M (M^T M)^-1/2, against the
+    SVD's polar factor of the same MTTKRP: even and odd ranks at the edges of the padded sizes.
+    The condition of this M^T M is at most 510 (R = 64), so some hundred roundings of 1.1e-16
+    leave the factor within 1e-11."""
+    rng = np.random.default_rng(R)
+    dims = [200, 9, 11]
+    X, init = rng.standard_normal(dims), [rng.standard_normal((I, R)) for I in dims]
+    h.set_tensor(X)
+    F, _, _ = h.cpd(R, init, max_iter=1, threshold_error=0.0, normalization=0, constraints=[2, 4, 4])
+    U, _, Wt = np.linalg.svd(h.mttkrp(init, 0), full_matrices=False)
+    say("rank", R, np.abs(F[0] - U @ Wt).max())
+    assert np.abs(F[0] - U @ Wt).max() <= 1e-11
+    assert np.abs(F[0].T @ F[0] - np.eye(R)).max() <= 1e-11
+
+
 @pytest.mark.parametrize("dims,R", [([6, 5, 7, 4, 5], 3), ([4, 5, 3, 4, 3, 4], 3), ([3, 4, 3, 2, 3, 2, 3], 2),
                                     ([3, 2, 3, 2, 2, 3, 2, 3], 2)])
 def test_dimtree_higher_orders(h, dims, R):
