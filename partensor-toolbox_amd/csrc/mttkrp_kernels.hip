@@ -23,6 +23,9 @@ namespace ptn {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
+// 16-byte loads at element alignment (a fibre may start at any element)
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 namespace {
 
@@ -192,9 +195,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_cm_f64(const TX *__restrict__ X
 // ---------------------------------------------------------------------------
 // gemm_ck: a wave owns 64 fibers (4 MFMA row tiles) and the whole contraction.
 // Within a 16-wide k-block, lane group g supplies a = kb + 4g + t at MFMA step t,
-// so each lane reads 4 consecutive elements of its fiber.
+// so each lane reads 4 consecutive elements of its fiber: 32 bytes of FP64 (two 16-byte
+// loads) or 16 of FP32 (one), at whatever element the fiber starts.  Reading them one by
+// one where the fiber length is not a multiple of 4, and the FP32 tensor always so, left
+// the kernel waiting on scattered 8-byte loads with nothing in flight behind them
+// (501 x 403 x 307, R = 33 node 423 -> 213 us, 190 x 155 x 61 x 24, R = 12 292 -> 139 us).
 // ---------------------------------------------------------------------------
-template <typename TX, int NT, bool VEC>
+template <typename TX, int NT>
 __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gemm_ck_f64(const TX *__restrict__ X, int64_t L, int64_t C, KrArgs w,
                                                      int ldr, double *__restrict__ T) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -233,38 +240,44 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gemm_ck_f64(const TX *
       for (int u = 0; u < NT; ++u) b[u] = j == 0 ? row[16 * u + f] : b[u] * row[16 * u + f];
     }
   };
-  auto mma16 = [&](const double (&x)[4][4], const double (&b)[4][NT]) {
+  auto mma16 = [&](const TX (&x)[4][4], const double (&b)[4][NT]) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int u = 0; u < NT; ++u)
-          acc[s][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[s][t], b[t][u], acc[s][u], 0, 0, 0);
+          acc[s][u] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x[s][t], b[t][u], acc[s][u], 0, 0, 0);
   };
   int64_t kb = 0;
-  if constexpr (VEC) {
-    // L % 4 == 0 and FP64 data: a lane's four elements a = kb + 4g .. kb + 4g + 3 of a fiber
-    // are one aligned 32-byte chunk (two 16-byte loads).  Full 16-wide blocks are
-    // software-pipelined over two register buffers: block j+1's Khatri-Rao rows and tensor
-    // loads are issued before block j's MFMAs.
+  {
+    // Full 16-wide blocks are software-pipelined over two register buffers: block j+1's
+    // Khatri-Rao rows and tensor loads are issued before block j's MFMAs.  A fiber past C
+    // reads fiber 0; its sums are never stored.
     const int64_t nblk = L / 16;
-    auto load_blk = [&](double (&x)[4][4], double (&b)[4][NT]) {
+    auto load_blk = [&](TX (&x)[4][4], double (&b)[4][NT]) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) kr_row(kb + 4 * g + t, true, b[t]);
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const f64x2 *q = (const f64x2 *)(xp[s] + kb + 4 * g);
-        const f64x2 lo = __builtin_nontemporal_load(q), hi = __builtin_nontemporal_load(q + 1);
-        x[s][0] = lo[0];                            // a fiber past C reads fiber 0; its
-        x[s][1] = lo[1];                            // sums are never stored
-        x[s][2] = hi[0];
-        x[s][3] = hi[1];
+        if constexpr (sizeof(TX) == 8) {
+          const f64x2u *q = (const f64x2u *)(xp[s] + kb + 4 * g);
+          const f64x2u lo = __builtin_nontemporal_load(q), hi = __builtin_nontemporal_load(q + 1);
+          x[s][0] = lo[0];
+          x[s][1] = lo[1];
+          x[s][2] = hi[0];
+          x[s][3] = hi[1];
+        } else {
+          const f32x4u v = __builtin_nontemporal_load((const f32x4u *)(xp[s] + kb + 4 * g));
+#pragma unroll
+          for (int j = 0; j < 4; ++j) x[s][j] = v[j];
+        }
       }
       kb += 16;
     };
     if (nblk > 0) {
-      double x0[4][4], b0[4][NT], x1[4][4], b1[4][NT];
+      TX x0[4][4], x1[4][4];                       // (FP32 elements widen where they are multiplied)
+      double b0[4][NT], b1[4][NT];
       load_blk(x0, b0);
       int64_t j = 0;
       for (; j + 2 < nblk; j += 2) {               // no branch between a load and its use
@@ -283,14 +296,14 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gemm_ck_f64(const TX *
     }
   }
   for (; kb < L; kb += 16) {
-    double x[4][4];
+    TX x[4][4];
     double b[4][NT];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int64_t a = kb + 4 * g + t;
       const bool av = a < L;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) x[s][t] = (av && cv[s]) ? ld(xp[s] + a) : 0.0;
+      for (int s = 0; s < 4; ++s) x[s][t] = (av && cv[s]) ? __builtin_nontemporal_load(xp[s] + a) : (TX)0;
       kr_row(a, av, b[t]);
     }
     mma16(x, b);
@@ -534,13 +547,11 @@ void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, 
   KrArgs a = to_args(w);
   dim3 grid((unsigned)((C + 255) / 256));
   const int NT = ldr / 16;
-  const bool vec = x64 && L % 4 == 0;         // aligned 32-byte chunks of every fiber
-#define PTN_CK(NTV)                                                                          \
-  if (NT == NTV) {                                                                           \
-    if (vec) k_gemm_ck_f64<double, NTV, true><<<grid, 256, 0, s>>>(x64, L, C, a, ldr, T);     \
-    else if (x64) k_gemm_ck_f64<double, NTV, false><<<grid, 256, 0, s>>>(x64, L, C, a, ldr, T); \
-    else     k_gemm_ck_f64<float, NTV, false><<<grid, 256, 0, s>>>(x32, L, C, a, ldr, T);     \
-    return;                                                                                  \
+#define PTN_CK(NTV)                                                                \
+  if (NT == NTV) {                                                                 \
+    if (x64) k_gemm_ck_f64<double, NTV><<<grid, 256, 0, s>>>(x64, L, C, a, ldr, T); \
+    else     k_gemm_ck_f64<float, NTV><<<grid, 256, 0, s>>>(x32, L, C, a, ldr, T);  \
+    return;                                                                        \
   }
   PTN_CK(1) PTN_CK(2) PTN_CK(3) PTN_CK(4)
 #undef PTN_CK

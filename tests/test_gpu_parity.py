@@ -530,6 +530,24 @@ def test_als_other_constraints(h, cons):
                 assert np.allclose(ratio, ratio[0:1, :], rtol=1e-12)
 
 
+@pytest.mark.parametrize("R", [5, 17, 33, 64])
+@pytest.mark.parametrize("I0", [1, 3, 15, 16, 17, 31, 33, 50, 97])
+def test_fibre_contraction_at_unaligned_lengths(h, I0, R):
+    """X x_0 A_0 on the FP64 matrix cores reads each fibre in 16-element blocks wherever it starts:
+    every residue class of the fibre length, more fibres than one block holds, each column
+    tile count, FP64 and FP32 tensors (the values are FP32 numbers, so both are exact), against
+    numpy in FP64.  Sums of up to 97 x 31 products of order 1: 1e-13 relative."""
+    rng = np.random.default_rng(I0 + 100 * R)
+    X = rng.standard_normal((I0, 9, 31)).astype(np.float32).astype(np.float64)
+    A = [rng.standard_normal((I, R)) for I in X.shape]
+    h.set_tensor(X, storage=P.TENSOR_BOTH)
+    T = np.tensordot(A[0], X, axes=(0, 0))                       # R x I1 x I2
+    want = {1: np.einsum("rjk,kr->jr", T, A[2]), 2: np.einsum("rjk,jr->kr", T, A[1])}
+    for arith in (P.ARITH_F64, P.ARITH_F32_F64):
+        for mode in (1, 2):
+            assert P.rel_err(h.mttkrp(A, mode, arith=arith), want[mode]) <= 1e-13
+
+
 @pytest.mark.parametrize("R", [1, 2, 3, 15, 16, 17, 32, 33, 63, 64])
 def test_orthogonal_update_is_the_polar_factor_at_every_padded_rank(h, R):
     """One update of mode 0 under the orthogonality constraint, A = M (M^T M)^-1/2, against the
