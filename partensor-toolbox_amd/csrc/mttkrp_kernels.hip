@@ -193,43 +193,49 @@ __global__ __launch_bounds__(256, 2) void k_gemm_cm_f64(const TX *__restrict__ X
 }
 
 // ---------------------------------------------------------------------------
-// gemm_ck: a wave owns 64 fibers (4 MFMA row tiles) and the whole contraction.
-// Within a 16-wide k-block, lane group g supplies a = kb + 4g + t at MFMA step t,
-// so each lane reads 4 consecutive elements of its fiber: 32 bytes of FP64 (two 16-byte
-// loads) or 16 of FP32 (one), at whatever element the fiber starts.  Reading them one by
-// one where the fiber length is not a multiple of 4, and the FP32 tensor always so, left
-// the kernel waiting on scattered 8-byte loads with nothing in flight behind them
-// (501 x 403 x 307, R = 33 node 423 -> 213 us, 190 x 155 x 61 x 24, R = 12 292 -> 139 us).
+// gemm_ck: a wave (a block of its own) owns 16 S fibers (S MFMA row tiles) and the whole
+// contraction.  Within a 16-wide k-block, lane group g supplies a = kb + 4g + t at MFMA
+// step t, so each lane reads 4 consecutive elements of its fiber: 32 bytes of FP64 (two
+// 16-byte loads) or 16 of FP32 (one), at whatever element the fiber starts.  Reading them
+// one by one where the fiber length is not a multiple of 4, and the FP32 tensor always so,
+// left the kernel waiting on scattered 8-byte loads with nothing in flight behind them.
+// The elements past the last whole block are the end of the block that ends with the fiber
+// (wide loads again; the elements that an earlier block had are zeroed): element by element
+// under a mask they cost as much as a third of the fiber.
+// The loads are cached ones: the two halves of a lane's 32 bytes, and the lines that a block
+// of an unaligned fiber shares with the next, are in two loads each, and non-temporal loads
+// fetched them twice (800^3 R = 32 node 986 -> 803 us, 5.3 TB/s; 501 x 403 x 307 R = 33, FP64
+// tensor 207 -> 156, of 423 at the start; 190 x 155 x 1464 R = 12 127 -> 81).
+// S: a Khatri-Rao fragment serves S tiles, so 4 where the fibers fill the chip all the same
+// (800^3 R = 32 803 us against 922 at S = 2; 123 721 fibers 156 against 163), 2 below 65 536
+// fibers (30 750: 21.4 us against 27.8 at S = 4) and for FP32 tensors, whose conversions take
+// the registers of a wave (245 000 fibers 44 against 52 us), 1 below 16 384 (10 000: 5.8 us
+// against 6.2 and 7.9).
 // ---------------------------------------------------------------------------
-template <typename TX, int NT>
-__global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gemm_ck_f64(const TX *__restrict__ X, int64_t L, int64_t C, KrArgs w,
-                                                     int ldr, double *__restrict__ T) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+template <typename TX, int NT, int S>
+__global__ __launch_bounds__(64, NT * S <= 8 ? 2 : 1) void k_gemm_ck_f64(const TX *__restrict__ X, int64_t L,
+                                                                         int64_t C, KrArgs w, int ldr,
+                                                                         double *__restrict__ T) {
+  const int lane = threadIdx.x;
   const int g = lane >> 4, f = lane & 15;
-  const int64_t cb = ((int64_t)blockIdx.x * 4 + wave) * 64;
-  if (cb >= C) return;
+  const int64_t cb = (int64_t)blockIdx.x * (16 * S);
 
-  f64x4 acc[4][NT];
+  f64x4 acc[S][NT];
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
+  for (int s = 0; s < S; ++s)
 #pragma unroll
     for (int u = 0; u < NT; ++u) acc[s][u] = f64x4{0.0, 0.0, 0.0, 0.0};
 
-  bool cv[4];
-  const TX *xp[4];
+  const TX *xp[S];                              // a fiber past C reads fiber 0; its sums are never stored
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    int64_t c = cb + 16 * s + f;
-    cv[s] = c < C;
-    xp[s] = X + L * (cv[s] ? c : 0);
+  for (int s = 0; s < S; ++s) {
+    const int64_t c = cb + 16 * s + f;
+    xp[s] = X + L * (c < C ? c : 0);
   }
   // the Khatri-Rao row of the contracted modes at a (lowest mode fastest), NT fragments
   // (the product runs over the digits as they are split off, so no array of row pointers
   // is indexed at run time: such an array lives in scratch memory)
-  auto kr_row = [&](int64_t a, bool av, double (&b)[NT]) {
-#pragma unroll
-    for (int u = 0; u < NT; ++u) b[u] = 0.0;
-    if (!av) return;
+  auto kr_row = [&](int64_t a, double (&b)[NT]) {
     uint32_t rem = (uint32_t)a;                   // a < L: the last digit is what remains
     for (int j = 0; j < w.nm; ++j) {
       const bool lastd = j + 1 == w.nm;
@@ -240,81 +246,92 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gemm_ck_f64(const TX *
       for (int u = 0; u < NT; ++u) b[u] = j == 0 ? row[16 * u + f] : b[u] * row[16 * u + f];
     }
   };
-  auto mma16 = [&](const TX (&x)[4][4], const double (&b)[4][NT]) {
+  struct Buf {
+    TX x[S][4];                                   // (FP32 elements widen where they are multiplied)
+    double b[4][NT];
+  };
+  auto mma16 = [&](const Buf &B) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int u = 0; u < NT; ++u)
-          acc[s][u] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x[s][t], b[t][u], acc[s][u], 0, 0, 0);
+          acc[s][u] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)B.x[s][t], B.b[t][u], acc[s][u], 0, 0, 0);
   };
-  int64_t kb = 0;
-  {
-    // Full 16-wide blocks are software-pipelined over two register buffers: block j+1's
-    // Khatri-Rao rows and tensor loads are issued before block j's MFMAs.  A fiber past C
-    // reads fiber 0; its sums are never stored.
-    const int64_t nblk = L / 16;
-    auto load_blk = [&](TX (&x)[4][4], double (&b)[4][NT]) {
+  auto load_blk = [&](int64_t kb, Buf &B) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) kr_row(kb + 4 * g + t, true, b[t]);
+    for (int t = 0; t < 4; ++t) kr_row(kb + 4 * g + t, B.b[t]);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        if constexpr (sizeof(TX) == 8) {
-          const f64x2u *q = (const f64x2u *)(xp[s] + kb + 4 * g);
-          const f64x2u lo = __builtin_nontemporal_load(q), hi = __builtin_nontemporal_load(q + 1);
-          x[s][0] = lo[0];
-          x[s][1] = lo[1];
-          x[s][2] = hi[0];
-          x[s][3] = hi[1];
-        } else {
-          const f32x4u v = __builtin_nontemporal_load((const f32x4u *)(xp[s] + kb + 4 * g));
-#pragma unroll
-          for (int j = 0; j < 4; ++j) x[s][j] = v[j];
-        }
-      }
-      kb += 16;
-    };
-    if (nblk > 0) {
-      TX x0[4][4], x1[4][4];                       // (FP32 elements widen where they are multiplied)
-      double b0[4][NT], b1[4][NT];
-      load_blk(x0, b0);
-      int64_t j = 0;
-      for (; j + 2 < nblk; j += 2) {               // no branch between a load and its use
-        load_blk(x1, b1);
-        mma16(x0, b0);
-        load_blk(x0, b0);
-        mma16(x1, b1);
-      }
-      if (j + 1 < nblk) {
-        load_blk(x1, b1);
-        mma16(x0, b0);
-        mma16(x1, b1);
+    for (int s = 0; s < S; ++s) {
+      if constexpr (sizeof(TX) == 8) {
+        const f64x2u *q = (const f64x2u *)(xp[s] + kb + 4 * g);
+        const f64x2u lo = q[0], hi = q[1];
+        B.x[s][0] = lo[0];
+        B.x[s][1] = lo[1];
+        B.x[s][2] = hi[0];
+        B.x[s][3] = hi[1];
       } else {
-        mma16(x0, b0);
+        const f32x4u v = *(const f32x4u *)(xp[s] + kb + 4 * g);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) B.x[s][j] = v[j];
       }
     }
-  }
-  for (; kb < L; kb += 16) {
-    TX x[4][4];
-    double b[4][NT];
+  };
+  // zero the block's entries outside [lo, L)
+  auto keep_from = [&](int64_t kb, int64_t lo, Buf &B) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int64_t a = kb + 4 * g + t;
-      const bool av = a < L;
+      const bool in = a >= lo && a < L;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) x[s][t] = (av && cv[s]) ? __builtin_nontemporal_load(xp[s] + a) : (TX)0;
-      kr_row(a, av, b[t]);
+      for (int s = 0; s < S; ++s) B.x[s][t] = in ? B.x[s][t] : (TX)0;
+#pragma unroll
+      for (int u = 0; u < NT; ++u) B.b[t][u] = in ? B.b[t][u] : 0.0;
     }
-    mma16(x, b);
+  };
+  Buf b0, b1;
+  if (L >= 16) {
+    // Blocks are software-pipelined over two register buffers: block j+1's Khatri-Rao rows
+    // and tensor loads are issued before block j's MFMAs, with no branch between a load and
+    // its use in the loop.
+    const int64_t nblk = (L + 15) / 16, lo = 16 * (nblk - 1);
+    auto start = [&](int64_t j) { return 16 * j < L - 16 ? 16 * j : L - 16; };
+    load_blk(0, b0);
+    int64_t j = 0;
+    for (; j + 2 < nblk; j += 2) {
+      load_blk(start(j + 1), b1);
+      mma16(b0);
+      load_blk(start(j + 2), b0);
+      mma16(b1);
+    }
+    if (j + 1 < nblk) {
+      load_blk(start(j + 1), b1);
+      mma16(b0);
+      keep_from(start(j + 1), lo, b1);
+      mma16(b1);
+    } else {
+      keep_from(start(j), lo, b0);
+      mma16(b0);
+    }
+  } else {                                        // a fiber shorter than a block: clamped element loads
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int64_t a = 4 * g + t, ac = a < L ? a : L - 1;
+      kr_row(ac, b0.b[t]);
+#pragma unroll
+      for (int s = 0; s < S; ++s) b0.x[s][t] = __builtin_nontemporal_load(xp[s] + ac);
+    }
+    keep_from(0, 0, b0);
+    mma16(b0);
   }
   // the node leaves with non-temporal stores (a leaf reads it after the other streams' work;
   // 800^3 R = 32 right node 1.020 -> 0.993 ms)
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
+  for (int s = 0; s < S; ++s)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      int64_t c = cb + 16 * s + g + 4 * v;
+      const int64_t c = cb + 16 * s + g + 4 * v;
       if (c < C) {
 #pragma unroll
         for (int u = 0; u < NT; ++u) __builtin_nontemporal_store(acc[s][u][v], &T[c * ldr + 16 * u + f]);
@@ -545,16 +562,24 @@ void gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mro
 void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, int64_t C, const KrSpec &w, int ldr,
                  double *T) {
   KrArgs a = to_args(w);
-  dim3 grid((unsigned)((C + 255) / 256));
   const int NT = ldr / 16;
-#define PTN_CK(NTV)                                                                \
-  if (NT == NTV) {                                                                 \
-    if (x64) k_gemm_ck_f64<double, NTV><<<grid, 256, 0, s>>>(x64, L, C, a, ldr, T); \
-    else     k_gemm_ck_f64<float, NTV><<<grid, 256, 0, s>>>(x32, L, C, a, ldr, T);  \
-    return;                                                                        \
+  // Fibers per wave: many share each Khatri-Rao fragment, few leave more waves for the 1024
+  // SIMDs (k_gemm_ck_f64)
+  const int S = C >= 65536 && x64 ? 4 : C >= 16384 ? 2 : 1;
+  const unsigned grid = (unsigned)((C + 16 * S - 1) / (16 * S));
+#define PTN_CKS(NTV, SV)                                                          \
+  if (x64) k_gemm_ck_f64<double, NTV, SV><<<grid, 64, 0, s>>>(x64, L, C, a, ldr, T); \
+  else     k_gemm_ck_f64<float, NTV, SV><<<grid, 64, 0, s>>>(x32, L, C, a, ldr, T);
+#define PTN_CK(NTV)              \
+  if (NT == NTV) {               \
+    if (S == 4) { PTN_CKS(NTV, 4) } \
+    else if (S == 2) { PTN_CKS(NTV, 2) } \
+    else { PTN_CKS(NTV, 1) }     \
+    return;                      \
   }
   PTN_CK(1) PTN_CK(2) PTN_CK(3) PTN_CK(4)
 #undef PTN_CK
+#undef PTN_CKS
 }
 
 void contract_rows(hipStream_t s, const double *T64, const float *T32, int64_t ldt, const KrSpec &spec, int outmode,

@@ -548,6 +548,22 @@ def test_fibre_contraction_at_unaligned_lengths(h, I0, R):
             assert P.rel_err(h.mttkrp(A, mode, arith=arith), want[mode]) <= 1e-13
 
 
+@pytest.mark.parametrize("R", [16, 33, 64])
+@pytest.mark.parametrize("dims", [(19, 127, 129), (16, 129, 128), (35, 131, 127), (16, 256, 256), (21, 257, 257)])
+def test_fibre_contraction_at_the_tile_counts_edges(h, dims, R):
+    """The same contraction with just below and above 16384 and 65536 fibres, where a wave's share
+    goes from 1 to 2 to 4 tiles of 16 fibres, whole and ragged.  Sums of up to 35 x 257 products
+    of order 1: 1e-13 relative."""
+    rng = np.random.default_rng(R)
+    X = rng.standard_normal(dims).astype(np.float32).astype(np.float64)
+    A = [rng.standard_normal((I, R)) for I in dims]
+    h.set_tensor(X, storage=P.TENSOR_BOTH)
+    T = np.tensordot(A[0], X, axes=(0, 0))
+    want = np.einsum("rjk,kr->jr", T, A[2])
+    for arith in (P.ARITH_F64, P.ARITH_F32_F64):
+        assert P.rel_err(h.mttkrp(A, 1, arith=arith), want) <= 1e-13
+
+
 @pytest.mark.parametrize("R", [1, 2, 3, 15, 16, 17, 32, 33, 63, 64])
 def test_orthogonal_update_is_the_polar_factor_at_every_padded_rank(h, R):
     """One update of mode 0 under the orthogonality constraint, A = M (M^T M)^-1/2, against the
