@@ -160,7 +160,10 @@ __global__ __launch_bounds__(256, NT >= 4 || MODE == kGemmFp32 ? 2 : 1) void k_g
   const int64_t mb = ((int64_t)blockIdx.x * 4 + wave) * 64;
   if (mb >= M) return;                                   // no block-wide barrier below
   const int64_t kbeg = (int64_t)blockIdx.y * kchunk;
-  const int64_t kend = kbeg + kchunk < K ? kbeg + kchunk : K;
+  // (chunks are rounded up to 16 columns, so the last splits of many can lie past K: empty
+  // ranges, whose partial sums are zero)
+  const int64_t kstop = kbeg + kchunk < K ? kbeg + kchunk : K;
+  const int64_t kend = kstop > kbeg ? kstop : kbeg;
 
   f32x16 acc[2][NT];
 #pragma unroll

@@ -530,6 +530,29 @@ def test_als_other_constraints(h, cons):
                 assert np.allclose(ratio, ratio[0:1, :], rtol=1e-12)
 
 
+@pytest.mark.parametrize("dims", [(100, 100, 100), (60, 127, 128), (40, 50, 61, 85)])
+def test_fp32_products_with_splits_past_the_last_column(h, dims):
+    """k chunks are rounded up to 16 columns, so the last of many splits can start past the end
+    (100^3, mode 0: 39 splits of 272 of 10000 columns); they add zero.  The tensor's memory is
+    followed by that of a larger one, so a read past its end is not a read of zeros.  FP32 sums
+    in splits of at most 272 products of order 1: 1e-5 relative."""
+    rng = np.random.default_rng(5)
+    h.set_tensor(rng.standard_normal((160, 160, 160)), storage=P.TENSOR_F32)
+    X = rng.standard_normal(dims)
+    A = [rng.standard_normal((I, 10)) for I in dims]
+    h.set_tensor(X, storage=P.TENSOR_F32)
+    want = X.reshape(dims[0], -1, order="F") @ np.array(
+        [np.prod(v, axis=0) for v in _rows_of_khatri_rao(A[1:])])
+    got = h.mttkrp(A, 0, arith=P.ARITH_F32), h.mttkrp_dimtree(A, arith=P.ARITH_F32)[0]
+    for M in got:
+        assert P.rel_err(M, want) <= 1e-5
+
+
+def _rows_of_khatri_rao(A):
+    for i in np.ndindex(*[a.shape[0] for a in A[::-1]]):
+        yield [a[j] for a, j in zip(A, i[::-1])]
+
+
 @pytest.mark.parametrize("R", [5, 17, 33, 64])
 @pytest.mark.parametrize("I0", [1, 3, 15, 16, 17, 31, 33, 50, 97])
 def test_fibre_contraction_at_unaligned_lengths(h, I0, R):
