@@ -58,6 +58,11 @@ struct ptn_handle_s {
   double frob_host = 0.0;
   BatchSet *batch = nullptr;
   MlpState *mlp = nullptr;    // the warm-start network, its training set and work buffers
+  // device memory the current call has finished with: its kernels may still be queued, so it
+  // goes back to the device's pool when the call has waited for its streams
+  std::vector<std::pair<void *, size_t>> spent;
+  void *readback[2] = {nullptr, nullptr};    // page-locked sweep readbacks (two sweep parities), kept between calls
+  bool pooled = false;                       // counted among the pool's handles
 };
 
 // Device scratch of ptn_nesterov_mnls_noalloc: a file-scope device array, one copy per GPU,
@@ -87,6 +92,108 @@ struct Fail {
     }                                                                                     \
   } while (0)
 
+// Device memory between calls.  A call's work buffers (some thirty, from a few bytes to the
+// gigabytes of a node) come from a pool per GPU, shared by its handles, and return to it when
+// the call has waited for its streams, so a block in the pool has no work pending.  hipMalloc,
+// hipFree and a memset for each of them were most of every short call and of every call
+// with a large node: MTTKRP of 37 x 23 x 41 189 -> 65 us, of 501 x 403 x 307 at
+// R = 33 759 -> 268 us, the order-4 tree at 200^4, R = 64 from between 7 and 95 ms to 5.3 ms.
+// The pool holds at most kPoolMax bytes (the oldest blocks are freed first), gives
+// everything back when an allocation fails or the GPU's last handle is destroyed, and is
+// guarded by a mutex.
+constexpr size_t kPoolMax = (size_t)8 << 30;
+struct DevicePool {
+  std::mutex mu;
+  std::vector<std::pair<void *, size_t>> blocks;   // oldest first
+  size_t held = 0;
+  int handles = 0;
+};
+DevicePool pools[kNoallocMaxDevices];
+
+// sizes rounded so that buffers of one call fit those of the next: powers of two up to 1 MB,
+// then whole 2 MB pages
+size_t pool_size(size_t bytes) {
+  if (bytes > ((size_t)1 << 20)) return (bytes + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
+  size_t s = 4096;
+  while (s < bytes) s *= 2;
+  return s;
+}
+
+// frees the oldest blocks until at most `keep` bytes are held
+void pool_trim(DevicePool &P, size_t keep) {
+  size_t n = 0;
+  while (n < P.blocks.size() && P.held > keep) {
+    (void)hipFree(P.blocks[n].first);
+    P.held -= P.blocks[n].second;
+    ++n;
+  }
+  P.blocks.erase(P.blocks.begin(), P.blocks.begin() + (std::ptrdiff_t)n);
+}
+
+// hipMalloc that gives the pool's memory back before it reports that there is none
+hipError_t device_malloc(int device, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  DevicePool &P = pools[device];
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    pool_trim(P, 0);
+  }
+  return hipMalloc(p, bytes);
+}
+
+// a block of at least `size` (a pool_size) bytes; a larger one serves while less than a
+// quarter of it would lie idle
+hipError_t pool_take(int device, size_t size, void **p, size_t *got) {
+  DevicePool &P = pools[device];
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    size_t best = P.blocks.size();
+    for (size_t i = 0; i < P.blocks.size(); ++i) {
+      const size_t b = P.blocks[i].second;
+      if (b >= size && b - size <= b / 4 && (best == P.blocks.size() || b < P.blocks[best].second)) best = i;
+    }
+    if (best < P.blocks.size()) {
+      *p = P.blocks[best].first;
+      *got = P.blocks[best].second;
+      P.held -= *got;
+      P.blocks.erase(P.blocks.begin() + (std::ptrdiff_t)best);
+      return hipSuccess;
+    }
+  }
+  *got = size;
+  return device_malloc(device, p, size);
+}
+
+void pool_give(int device, void *p, size_t bytes) {
+  DevicePool &P = pools[device];
+  std::lock_guard<std::mutex> lock(P.mu);
+  if (bytes <= kPoolMax) {
+    pool_trim(P, kPoolMax - bytes);
+    try {
+      P.blocks.emplace_back(p, bytes);
+      P.held += bytes;
+      return;
+    } catch (const std::bad_alloc &) {
+    }
+  }
+  (void)hipFree(p);
+}
+
+// the end of a call: what it has finished with returns to the pool once its streams are idle
+void give_back_spent(ptn_handle h) {
+  if (h->spent.empty()) return;
+  bool idle = true;
+  for (hipStream_t s : {h->stream, h->side, h->aux})
+    if (s && hipStreamSynchronize(s) != hipSuccess) idle = false;
+  for (const auto &b : h->spent) {
+    if (idle) pool_give(h->device, b.first, b.second);
+    else (void)hipFree(b.first);
+  }
+  h->spent.clear();
+}
+
 #define REQUIRE(cond, code, msg)        \
   do {                                  \
     if (!(cond)) {                      \
@@ -95,41 +202,51 @@ struct Fail {
     }                                   \
   } while (0)
 
+enum Fill { kZero, kRaw };                   // kRaw: written before it is read
+
 template <typename T>
 struct DevBuf {
   T *p = nullptr;
   size_t n = 0;
+  size_t bytes = 0;                          // of the pool's block
   ptn_handle h = nullptr;
   DevBuf() = default;
-  DevBuf(ptn_handle hh, size_t count) { alloc(hh, count); }
-  void alloc(ptn_handle hh, size_t count) {
+  DevBuf(ptn_handle hh, size_t count, Fill fill = kZero) { alloc(hh, count, fill); }
+  void alloc(ptn_handle hh, size_t count, Fill fill = kZero) {
     h = hh;
     n = count ? count : 1;
-    HIPCHK(hipMalloc((void **)&p, n * sizeof(T)));
-    HIPCHK(hipMemsetAsync(p, 0, n * sizeof(T), h->stream));
+    h->spent.reserve(h->spent.size() + 64);  // the destructor's push does not allocate
+    HIPCHK(pool_take(h->device, pool_size(n * sizeof(T)), (void **)&p, &bytes));
+    if (fill == kZero) HIPCHK(hipMemsetAsync(p, 0, n * sizeof(T), h->stream));
   }
   ~DevBuf() {
-    if (p) (void)hipFree(p);
+    if (!p) return;
+    try {
+      h->spent.emplace_back((void *)p, bytes);
+    } catch (const std::bad_alloc &) {
+      (void)hipFree(p);                      // (waits for the device)
+    }
   }
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
   operator T *() const { return p; }
+  void swap(DevBuf &o) {
+    std::swap(p, o.p); std::swap(n, o.n); std::swap(bytes, o.bytes); std::swap(h, o.h);
+  }
 };
 
+// page-locked, coherent host memory that kernels write directly, cleared for a call (dev = its
+// device address); the handle keeps it
 template <typename T>
-struct PinnedBuf {      // page-locked, coherent host memory that kernels write directly (dev = its device address)
+struct PinnedBuf {
   T *p = nullptr;
   T *dev = nullptr;
-  explicit PinnedBuf(ptn_handle h) {
-    HIPCHK(hipHostMalloc((void **)&p, sizeof(T), hipHostMallocMapped | hipHostMallocCoherent));
+  PinnedBuf(ptn_handle h, void *&kept) {
+    if (!kept) HIPCHK(hipHostMalloc(&kept, sizeof(T), hipHostMallocMapped | hipHostMallocCoherent));
+    p = (T *)kept;
     std::memset((void *)p, 0, sizeof(T));
     HIPCHK(hipHostGetDevicePointer((void **)&dev, p, 0));
   }
-  ~PinnedBuf() {
-    if (p) (void)hipHostFree(p);
-  }
-  PinnedBuf(const PinnedBuf &) = delete;
-  PinnedBuf &operator=(const PinnedBuf &) = delete;
 };
 
 struct EventPair {                           // two timing-free events, destroyed with the scope
@@ -178,6 +295,7 @@ struct MlpState {
     w.alloc(h, kMlpParams); g.alloc(h, kMlpParams); m1.alloc(h, kMlpParams); m2.alloc(h, kMlpParams);
     wb.alloc(h, kMlpWb); w2t.alloc(h, (size_t)kMlpH * kMlpH); w3t.alloc(h, (size_t)kMlpH * kMlpR);
     part.alloc(h, 64);
+    HIPCHK(hipStreamSynchronize(h->stream));  // the fills have run: hipMemcpy follows on another stream
   }
   template <typename T_>
   static void grow(ptn_handle h, DevBuf<T_> &b, size_t count) {
@@ -195,6 +313,7 @@ struct MlpState {
     grow(h, dYb, ro); grow(h, dYT, ro); grow(h, dH1, rh); grow(h, dH1T, rh); grow(h, dH2, rh); grow(h, dH2T, rh);
     grow(h, Y, ro); grow(h, T, ro); grow(h, dYf, ro); grow(h, scale, (size_t)r); grow(h, rank, (size_t)r);
     grow(h, start, ro);
+    HIPCHK(hipStreamSynchronize(h->stream));
     rows = r;
   }
   void ensure_data(int64_t need) {
@@ -204,14 +323,13 @@ struct MlpState {
     DevBuf<uint16_t> nx(h, (size_t)nc * kMlpIn);
     DevBuf<float> nt(h, (size_t)nc * kMlpR);
     DevBuf<unsigned char> nr(h, (size_t)nc);
+    HIPCHK(hipStreamSynchronize(h->stream));
     if (n > 0) {
       HIPCHK(hipMemcpy(nx.p, dx.p, (size_t)n * kMlpIn * 2, hipMemcpyDeviceToDevice));
       HIPCHK(hipMemcpy(nt.p, dt.p, (size_t)n * kMlpR * 4, hipMemcpyDeviceToDevice));
       HIPCHK(hipMemcpy(nr.p, drank.p, (size_t)n, hipMemcpyDeviceToDevice));
     }
-    std::swap(dx.p, nx.p); std::swap(dx.n, nx.n); dx.h = h;
-    std::swap(dt.p, nt.p); std::swap(dt.n, nt.n); dt.h = h;
-    std::swap(drank.p, nr.p); std::swap(drank.n, nr.n); drank.h = h;
+    dx.swap(nx); dt.swap(nt); drank.swap(nr);
     cap = nc;
   }
   // Y = network(X) for B rows (activations kept for the backward pass)
@@ -321,40 +439,42 @@ struct Work {
       if (dims[k] > maxI) maxI = dims[k];
     }
     fsz = o;
-    fac.alloc(h, fsz); old.alloc(h, fsz); acc.alloc(h, fsz);
-    grams.alloc(h, (size_t)N * R * R); agr.alloc(h, (size_t)N * R * R);
-    Vm.alloc(h, (size_t)(N + 1) * R * R); Vacc.alloc(h, (size_t)R * R);
-    M.alloc(h, maxI * ldr); Aold.alloc(h, maxI * ldr); colsum.alloc(h, kMaxRank);
-    prm.alloc(h, kMaxOrder + 1); mask.alloc(h, nnls_mask_words(maxI)); flags.alloc(h, 4);
-    nscr.alloc(h, 2 * kMaxOrder * kMaxRank); scal.alloc(h, 8); betas.alloc(h, (size_t)(N + 1) * (kMaxInner + 1));
-    gpart.alloc(h, (size_t)((maxI + 31) / 32) * R * R); gpart_side.alloc(h, (size_t)((maxI + 31) / 32) * R * R);
-    cscr.alloc(h, (size_t)3 * R * R + R);    // R x R work of the unconstrained / orthogonality updates
+    fac.alloc(h, fsz, kRaw); old.alloc(h, fsz, kRaw); acc.alloc(h, fsz, kRaw);
+    grams.alloc(h, (size_t)N * R * R, kRaw); agr.alloc(h, (size_t)N * R * R, kRaw);
+    Vm.alloc(h, (size_t)(N + 1) * R * R, kRaw); Vacc.alloc(h, (size_t)R * R, kRaw);
+    M.alloc(h, maxI * ldr, kRaw); Aold.alloc(h, maxI * ldr, kRaw); colsum.alloc(h, kMaxRank, kRaw);
+    prm.alloc(h, kMaxOrder + 1); mask.alloc(h, nnls_mask_words(maxI), kRaw); flags.alloc(h, 4, kRaw);
+    nscr.alloc(h, 2 * kMaxOrder * kMaxRank, kRaw); scal.alloc(h, 8, kRaw);
+    betas.alloc(h, (size_t)(N + 1) * (kMaxInner + 1), kRaw);
+    gpart.alloc(h, (size_t)((maxI + 31) / 32) * R * R, kRaw);
+    gpart_side.alloc(h, (size_t)((maxI + 31) / 32) * R * R, kRaw);
+    cscr.alloc(h, (size_t)3 * R * R + R, kRaw);    // R x R work of the unconstrained / orthogonality updates
     const int64_t C = total / dims[0];
     const int64_t yl = left_rows();
     // reduction partials: mode-0 split-K (<= 256 splits of I_0 rows) and row contractions (<= 64 splits)
     part_cap = std::max<int64_t>(256 * dims[0] * ldr, 64 * maxI * ldr);
     if (!mfma32) {
       if (need_tree && N >= 4) part_cap = std::max<int64_t>(part_cap, 64 * yl * ldr);
-      T.alloc(h, C * ldr);
-      if (need_tree) YL.alloc(h, yl * ldr);
+      T.alloc(h, C * ldr, kRaw);
+      if (need_tree) YL.alloc(h, yl * ldr, kRaw);
     } else {
       part32_cap = 256 * dims[0] * rpf;
       if (need_tree && N >= 4) part32_cap = std::max<int64_t>(part32_cap, 64 * yl * rpf);
-      part32.alloc(h, part32_cap);
-      T32.alloc(h, std::max(C, dims[0]) * rpf);
-      if (need_tree) YL32.alloc(h, yl * rpf);
+      part32.alloc(h, part32_cap, kRaw);
+      T32.alloc(h, std::max(C, dims[0]) * rpf, kRaw);
+      if (need_tree) YL32.alloc(h, yl * rpf, kRaw);
     }
-    part.alloc(h, part_cap);
+    part.alloc(h, part_cap, kRaw);
   }
   // buffers of the paired left-node pass (dimension tree, FP32-output contractions)
   void enable_pair() {
     const int64_t yl = left_rows();
-    YL2.alloc(h, yl * 2 * rpf);
-    M2.alloc(h, 2 * dims[0] * ldr);          // [Mhat | M] of mode 0 from the paired pass
+    YL2.alloc(h, yl * 2 * rpf, kRaw);
+    M2.alloc(h, 2 * dims[0] * ldr, kRaw);          // [Mhat | M] of mode 0 from the paired pass
     if (N >= 4 && 64 * yl * 2 * rpf > part32_cap) {
       part32.~DevBuf(); new (&part32) DevBuf<float>();
       part32_cap = 64 * yl * 2 * rpf;
-      part32.alloc(h, part32_cap);
+      part32.alloc(h, part32_cap, kRaw);
     }
   }
   // the tree's root splits at half = ceil(N / 2) (DIM_HALF_SIZE, DimTrees.hpp:274): the left
@@ -377,16 +497,18 @@ struct Work {
   void pack(const KrSpec &k, int64_t K, int kperm, const KrSpec *k2 = nullptr, hipStream_t ps = nullptr) {
     const int width = k2 ? 2 * rpf : rpf;
     const int64_t frag = wpack_elems(K, width);
+    const bool x3 = arith == PTN_ARITH_BF16X3;
     if (frag > wcap) {
-      HIPCHK(hipStreamSynchronize(h->stream));
-      whi.~DevBuf(); new (&whi) DevBuf<uint16_t>();
-      wlo.~DevBuf(); new (&wlo) DevBuf<uint16_t>();
-      wf.~DevBuf(); new (&wf) DevBuf<float>();
-      whi.alloc(h, frag * 8); wlo.alloc(h, frag * 8);
-      wf.alloc(h, frag * 8);
+      if (x3) {
+        whi.~DevBuf(); new (&whi) DevBuf<uint16_t>();
+        wlo.~DevBuf(); new (&wlo) DevBuf<uint16_t>();
+        whi.alloc(h, frag * 8, kRaw); wlo.alloc(h, frag * 8, kRaw);
+      } else {
+        wf.~DevBuf(); new (&wf) DevBuf<float>();
+        wf.alloc(h, frag * 8, kRaw);
+      }
       wcap = frag;
     }
-    const bool x3 = arith == PTN_ARITH_BF16X3;
     pack_w(ps ? ps : h->stream, k, k2, K, width, ldr, kperm, x3 ? (void *)whi.p : nullptr,
            x3 ? (void *)wlo.p : nullptr, x3 ? nullptr : wf.p);
   }
@@ -753,7 +875,7 @@ void upload_factors(Work &w, const double *packed_host, double *dst_rows) {
   ptn_handle h = w.h;
   int64_t n = 0;
   for (int k = 0; k < w.N; ++k) n += w.dims[k] * w.R;
-  DevBuf<double> tmp(h, n);
+  DevBuf<double> tmp(h, n, kRaw);
   HIPCHK(hipMemcpyAsync(tmp.p, packed_host, n * sizeof(double), hipMemcpyHostToDevice, h->stream));
   int64_t o = 0;
   for (int k = 0; k < w.N; ++k) {
@@ -767,7 +889,7 @@ void download_factors(Work &w, const double *src_rows, double *packed_host) {
   ptn_handle h = w.h;
   int64_t n = 0;
   for (int k = 0; k < w.N; ++k) n += w.dims[k] * w.R;
-  DevBuf<double> tmp(h, n);
+  DevBuf<double> tmp(h, n, kRaw);
   int64_t o = 0;
   for (int k = 0; k < w.N; ++k) {
     rows_to_colmajor(h->stream, w.dims[k], w.R, w.ldr, src_rows + w.off[k], tmp.p + o);
@@ -797,10 +919,9 @@ void update_nonneg(Work &w, int mode, const ptn_options &o, const ModeIn &in) {
   NnlsParams *p = in.p;
   const int64_t need = (int64_t)(o.max_inner + 1) * w.maxI * w.ldr;
   if (need > w.hist_cap) {
-    HIPCHK(hipStreamSynchronize(s));
     w.hist.~DevBuf();
     new (&w.hist) DevBuf<double>();
-    w.hist.alloc(h, need);
+    w.hist.alloc(h, need, kRaw);
     w.hist_cap = need;
   }
   const bool warm = o.warm_start != 0, harvest = o.mlp_harvest != 0;
@@ -924,6 +1045,9 @@ ptn_status ptn_create(ptn_handle *out, int device) {
       REQUIRE(ptr != nullptr, PTN_ERR_HIP, "no device address for the no-allocation scratch");
       noalloc_ptr[device] = ptr;
     }
+    std::lock_guard<std::mutex> plock(pools[device].mu);
+    ++pools[device].handles;
+    h->pooled = true;
   });
   if (st != PTN_OK) {
     ptn_destroy(h);
@@ -943,6 +1067,14 @@ void ptn_destroy(ptn_handle h) {
   if (h->x32) (void)hipFree(h->x32);
   delete h->batch;
   delete h->mlp;
+  give_back_spent(h);
+  for (void *r : h->readback)
+    if (r) (void)hipHostFree(r);
+  if (h->pooled) {
+    DevicePool &P = pools[h->device];
+    std::lock_guard<std::mutex> lock(P.mu);
+    if (--P.handles == 0) pool_trim(P, 0);
+  }
   if (h->scal) (void)hipFree(h->scal);
   if (h->part) (void)hipFree(h->part);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -961,6 +1093,10 @@ namespace {
 
 ptn_status run(ptn_handle h, const std::function<void()> &fn) {
   if (!h) return PTN_ERR_INVALID;
+  struct AtEnd {                             // also on the way out of an error
+    ptn_handle h;
+    ~AtEnd() { give_back_spent(h); }
+  } at_end{h};
   try {
     if (h->stream) {
       hipError_t e = hipSetDevice(h->device);
@@ -994,11 +1130,11 @@ void alloc_tensor(ptn_handle h, int N, const int64_t *dims, int storage) {
   // kTensorPad zero elements after the tensor: the contiguous-K contractions read whole
   // 32-element steps, which may run past the end of the last fiber
   if (storage & PTN_TENSOR_F64) {
-    HIPCHK(hipMalloc((void **)&h->x64, (h->total + kTensorPad) * sizeof(double)));
+    HIPCHK(device_malloc(h->device, (void **)&h->x64, (h->total + kTensorPad) * sizeof(double)));
     HIPCHK(hipMemsetAsync(h->x64 + h->total, 0, kTensorPad * sizeof(double), h->stream));
   }
   if (storage & PTN_TENSOR_F32) {
-    HIPCHK(hipMalloc((void **)&h->x32, (h->total + kTensorPad) * sizeof(float)));
+    HIPCHK(device_malloc(h->device, (void **)&h->x32, (h->total + kTensorPad) * sizeof(float)));
     HIPCHK(hipMemsetAsync(h->x32 + h->total, 0, kTensorPad * sizeof(float), h->stream));
   }
 }
@@ -1022,7 +1158,7 @@ ptn_status ptn_set_tensor(ptn_handle h, int N, const int64_t *dims, const double
       HIPCHK(hipMemcpyAsync(h->x64, X, h->total * sizeof(double), hipMemcpyHostToDevice, h->stream));
       if (h->x32) cast_f64_to_f32(h->stream, h->total, h->x64, h->x32);
     } else {
-      DevBuf<double> tmp(h, h->total);
+      DevBuf<double> tmp(h, h->total, kRaw);
       HIPCHK(hipMemcpyAsync(tmp.p, X, h->total * sizeof(double), hipMemcpyHostToDevice, h->stream));
       cast_f64_to_f32(h->stream, h->total, tmp.p, h->x32);
       HIPCHK(hipStreamSynchronize(h->stream));
@@ -1039,7 +1175,7 @@ ptn_status ptn_generate_tensor(ptn_handle h, int N, const int64_t *dims, int R_t
     alloc_tensor(h, N, dims, storage);
     int64_t nf = 0;
     for (int k = 0; k < N; ++k) nf += dims[k] * R_true;
-    DevBuf<double> fac(h, nf);
+    DevBuf<double> fac(h, nf, kRaw);
     gen_factors(h->stream, N, dims, R_true, seed, dist, fac.p);
     cp_full(h->stream, N, dims, R_true, fac.p, h->x64, h->x32);
     if (!std::isnan(snr_db)) {
@@ -1062,7 +1198,7 @@ ptn_status ptn_generate_factors(ptn_handle h, int N, const int64_t *dims, int R,
     REQUIRE(packed_out, PTN_ERR_INVALID, "output is null");
     int64_t nf = 0;
     for (int k = 0; k < N; ++k) nf += dims[k] * R;
-    DevBuf<double> fac(h, nf);
+    DevBuf<double> fac(h, nf, kRaw);
     gen_factors(h->stream, N, dims, R, seed, dist, fac.p);
     HIPCHK(hipMemcpyAsync(packed_out, fac.p, nf * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -1161,7 +1297,7 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
       int flags[4];
       unsigned seq;                           // the sweep index, published last by the device
     };
-    PinnedBuf<Readback> rbuf0(h), rbuf1(h);
+    PinnedBuf<Readback> rbuf0(h, h->readback[0]), rbuf1(h, h->readback[1]);
     struct PassEvents {                       // time_passes: 2 sweep slots x (start, end) x 2 passes
       hipEvent_t e[2][4] = {};
       ~PassEvents() {
@@ -1177,9 +1313,9 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
     }
     Readback *rbs[2] = {rbuf0.p, rbuf1.p};
     Readback *rbd[2] = {rbuf0.dev, rbuf1.dev};     // the same buffers as the device addresses them
-    DevBuf<double> snap0(h, w.fsz), snap1(h, w.fsz);
+    DevBuf<double> snap0(h, w.fsz, kRaw), snap1(h, w.fsz, kRaw);
     double *snaps[2] = {snap0.p, snap1.p};
-    EventPair evs(h);
+    std::unique_ptr<EventPair> evs(o.time_passes ? new EventPair(h) : nullptr);
     {
       const int fl[4] = {0, 0, o.accel_fail, o.accel_coeff};
       HIPCHK(hipMemcpy(w.flags.p, fl, sizeof(fl), hipMemcpyHostToDevice));
@@ -1321,13 +1457,13 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
         }
       }
       if (!snapped) HIPCHK(hipMemcpyAsync(snaps[it & 1], w.fac, w.fsz * sizeof(double), hipMemcpyDeviceToDevice, ms));
-      if (w.kev) HIPCHK(hipEventRecord(evs.e[it & 1], ms));   // timed runs read their pass events after it
+      if (w.kev) HIPCHK(hipEventRecord(evs->e[it & 1], ms));   // timed runs read their pass events after it
       tried_at[it & 1] = tried;
     };
 
     auto process = [&](int it) {
       if (w.kev) {
-        HIPCHK(hipEventSynchronize(evs.e[it & 1]));
+        HIPCHK(hipEventSynchronize(evs->e[it & 1]));
       } else {
         // the sweep's last readback kernel publishes `it` after a system-scope fence; the
         // stream is queried now and then so that a failed launch ends the wait
@@ -1412,7 +1548,7 @@ ptn_status ptn_mttkrp(ptn_handle h, int R, const double *factors_packed, int mod
     Work w(h, R, arith, false);
     upload_factors(w, factors_packed, w.fac);
     mttkrp_standard(w, w.fac, mode, w.M);
-    DevBuf<double> cm(h, w.dims[mode] * R);
+    DevBuf<double> cm(h, w.dims[mode] * R, kRaw);
     rows_to_colmajor(h->stream, w.dims[mode], R, w.ldr, w.M, cm.p);
     HIPCHK(hipMemcpyAsync(M_out, cm.p, w.dims[mode] * R * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -1431,7 +1567,7 @@ ptn_status ptn_mttkrp_dimtree(ptn_handle h, int R, const double *factors_packed,
     int64_t o = 0;
     for (int n = 0; n < w.N; ++n) {
       mttkrp_tree(w, w.fac, n, w.M);
-      DevBuf<double> cm(h, w.dims[n] * R);
+      DevBuf<double> cm(h, w.dims[n] * R, kRaw);
       rows_to_colmajor(h->stream, w.dims[n], R, w.ldr, w.M, cm.p);
       HIPCHK(hipMemcpyAsync(M_packed_out + o, cm.p, w.dims[n] * R * sizeof(double), hipMemcpyDeviceToHost,
                             h->stream));
@@ -1446,7 +1582,7 @@ ptn_status ptn_sym_extremes(ptn_handle h, int R, const double *V, double *L, dou
   return run(h, [&] {
     REQUIRE(R >= 1 && R <= PTN_MAX_RANK, PTN_ERR_UNSUPPORTED, "rank must be in [1, 64]");
     REQUIRE(V && L && mu, PTN_ERR_INVALID, "null argument");
-    DevBuf<double> dV(h, (size_t)R * R);
+    DevBuf<double> dV(h, (size_t)R * R, kRaw);
     DevBuf<NnlsParams> p(h, 1);
     HIPCHK(hipMemcpyAsync(dV.p, V, (size_t)R * R * sizeof(double), hipMemcpyHostToDevice, h->stream));
     eig_extremes(h->stream, R, dV.p, p.p);
@@ -1466,11 +1602,12 @@ ptn_status ptn_nesterov_mnls(ptn_handle h, int64_t I, int R, const double *Z, co
     REQUIRE(max_inner >= 0 && max_inner <= kMaxInner, PTN_ERR_UNSUPPORTED, "max_inner must be in [0, 255]");
     REQUIRE(Z && W && A, PTN_ERR_INVALID, "null argument");
     const int ldr = round_up16(R);
-    DevBuf<double> dZ(h, (size_t)R * R), tmp(h, I * R), dW(h, I * ldr), dA(h, I * ldr), dB(h, I * ldr);
-    DevBuf<double> hist(h, (size_t)(max_inner + 1) * I * ldr), betas(h, kMaxInner + 1);
-    DevBuf<double> colsum(h, kMaxRank);
+    DevBuf<double> dZ(h, (size_t)R * R, kRaw), tmp(h, I * R, kRaw), dW(h, I * ldr, kRaw), dA(h, I * ldr, kRaw),
+        dB(h, I * ldr, kRaw);
+    DevBuf<double> hist(h, (size_t)(max_inner + 1) * I * ldr, kRaw), betas(h, kMaxInner + 1, kRaw);
+    DevBuf<double> colsum(h, kMaxRank, kRaw);
     DevBuf<NnlsParams> p(h, 1);
-    DevBuf<uint64_t> mask(h, nnls_mask_words(I));
+    DevBuf<uint64_t> mask(h, nnls_mask_words(I), kRaw);
     std::vector<double> zr((size_t)R * R);
     for (int a = 0; a < R; ++a)
       for (int b = 0; b < R; ++b) zr[a * R + b] = Z[a + (int64_t)R * b];
@@ -1753,7 +1890,7 @@ void batch_layout(ptn_handle h, int nprob, const int *dims, const int *ranks) {
   b->nx = xo;
   b->nrows = fo;
   // three copies: mode 0 fastest (the tensors as given), mode 1 fastest, mode 2 fastest
-  HIPCHK(hipMalloc((void **)&b->x32, 3 * xo * sizeof(float)));
+  HIPCHK(device_malloc(h->device, (void **)&b->x32, 3 * xo * sizeof(float)));
   HIPCHK(hipMemsetAsync(b->x32, 0, 3 * xo * sizeof(float), h->stream));
   delete h->batch;
   h->batch = b.release();

@@ -530,6 +530,47 @@ def test_als_other_constraints(h, cons):
                 assert np.allclose(ratio, ratio[0:1, :], rtol=1e-12)
 
 
+def test_work_buffers_shared_between_handles_and_threads():
+    """Calls take their work buffers from a pool that the handles of a GPU share: calls of
+    different sizes on four handles in four threads at once, with failing calls between them,
+    give the bits that each handle gives alone."""
+    import threading
+    rng = np.random.default_rng(8)
+    shapes = [((37, 23, 41), 5), ((120, 90, 70), 20), ((40, 31, 22, 9), 12), ((300, 64, 50), 40)]
+    handles, calls = [], []
+    for dims, R in shapes:
+        hd = P.Handle(0)
+        hd.set_tensor(rng.standard_normal(dims), storage=P.TENSOR_BOTH)
+        A = [rng.random((I, R)) for I in dims]
+        handles.append(hd)
+        calls.append([lambda hd=hd, A=A: hd.mttkrp(A, 1), lambda hd=hd, A=A: hd.mttkrp_dimtree(A, arith=P.ARITH_F32),
+                      lambda hd=hd, A=A, R=R: hd.cpd(R, A, max_iter=4, threshold_error=0.0)[0]])
+    alone = [[c() for c in cs] for cs in calls]
+    bad = []
+
+    def work(k):
+        for _ in range(5):
+            try:
+                handles[k].mttkrp([np.zeros((3, 65))], 0)     # rank above the limit
+                bad.append(k)
+            except P.PtnError:
+                pass
+            for c, want in zip(calls[k], alone[k]):
+                got = c()
+                same = all(np.array_equal(g, w) for g, w in zip(got, want)) if isinstance(want, list) else \
+                    np.array_equal(got, want)
+                if not same:
+                    bad.append(k)
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(shapes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for hd in handles:
+        hd.close()
+    assert not bad
+
+
 @pytest.mark.parametrize("dims", [(100, 100, 100), (60, 127, 128), (40, 50, 61, 85)])
 def test_fp32_products_with_splits_past_the_last_column(h, dims):
     """k chunks are rounded up to 16 columns, so the last of many splits can start past the end
