@@ -161,27 +161,111 @@ struct FacPtrs {
   const double *p[kMaxOrder];
 };
 
-// Sum over slabs of (X - A_last KR^T)^2 (Cpd.hpp:131-135): reconstruct each element from
-// the factor rows, FP64.
-__global__ void k_cost_explicit(Dims D, int R, int ldr, FacPtrs F, int64_t total, const double *x64,
-                                const float *x32, double *partials) {
-  double s = 0.0;
-  const int last = D.N - 1;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    int64_t ik[kMaxOrder];
-    int64_t rem = idx;
-    for (int k = 0; k < D.N; ++k) { ik[k] = rem % D.d[k]; rem /= D.d[k]; }
-    double rec = 0.0;
-    for (int r = 0; r < R; ++r) {
-      double p = F.p[0][ik[0] * ldr + r];
-      for (int k = 1; k < last; ++k) p *= F.p[k][ik[k] * ldr + r];
-      rec = fma(F.p[last][ik[last] * ldr + r], p, rec);
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+// Sum over slabs of (X - A_last KR^T)^2 (Cpd.hpp:131-135): the reconstruction is the product
+// of mode 0's rows and the Khatri-Rao rows of the other modes, 2 R flops per element, formed
+// tile by tile on v_mfma_f64_16x16x4f64 and compared with X in registers.
+//
+// Bounds: 2 ldr flops per element on the FP64 matrix cores (800^3, R = 32: 0.42 ms) and one
+// reading of X (FP32: 0.32 ms).  Each element by a thread of its own, R products of N factor
+// entries fetched for each, took 58.3 ms there; this takes 0.69 ms.
+//
+// A wave holds the Khatri-Rao rows of 16 CT columns (fibres) as its A operand, formed once,
+// and walks mode 0 in tiles of 16 rows: lane (g, f) of a tile supplies r = KQ g + s at step s
+// for both operands (KQ = ldr / 4), so its share of a factor row is KQ consecutive doubles,
+// and receives X(i0 = f, column g + 4 v).  Tile j + 1's loads are issued before tile j's MFMAs.
+// CT: 4 while the registers hold it (KQ <= 8), else 2.  The blocks of y split mode 0 where
+// there are few columns.  Rows past I0 and columns past C read the last one and are not added.
+template <typename TX, int KQ, int CT>
+__global__ __launch_bounds__(256, 2) void k_cost_explicit(Dims D, int64_t C, FacPtrs F, const TX *__restrict__ X,
+                                                          int tiles_per_y, double *__restrict__ partials) {
+  constexpr int LDR = 4 * KQ;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, f = lane & 15;
+  const int64_t I0 = D.d[0];
+  const int64_t tiles = (I0 + 15) / 16;
+  const int64_t j0 = (int64_t)blockIdx.y * tiles_per_y;
+  const int64_t j1 = j0 + tiles_per_y < tiles ? j0 + tiles_per_y : tiles;
+  double sum = 0.0;
+  for (int64_t cb = ((int64_t)blockIdx.x * 4 + wave) * (16 * CT); cb < C; cb += (int64_t)gridDim.x * (64 * CT)) {
+    double kr[CT][KQ];
+#pragma unroll
+    for (int t = 0; t < CT; ++t) {
+      const int64_t c = cb + 16 * t + f;
+      uint32_t rem = (uint32_t)(c < C ? c : C - 1);
+#pragma unroll
+      for (int s = 0; s < KQ; ++s) kr[t][s] = 1.0;
+      for (int k = 1; k < D.N; ++k) {
+        const uint32_t dk = (uint32_t)D.d[k], i = rem % dk;
+        rem /= dk;
+        const f64x2 *row = (const f64x2 *)(F.p[k] + (int64_t)i * LDR + KQ * g);
+#pragma unroll
+        for (int s = 0; s < KQ / 2; ++s) {
+          const f64x2 v = row[s];
+          kr[t][2 * s] *= v[0];
+          kr[t][2 * s + 1] *= v[1];
+        }
+      }
     }
-    double d = (x64 ? x64[idx] : (double)x32[idx]) - rec;
-    s = fma(d, d, s);
+    const TX *col[CT];                           // columns cb + 16 t + g, then every 4th
+#pragma unroll
+    for (int t = 0; t < CT; ++t) col[t] = X + I0 * (cb + 16 * t + g);
+    struct Buf {
+      TX x[CT][4];
+      f64x2 a[KQ / 2];
+    };
+    auto load = [&](int64_t j, Buf &B) {
+      const int64_t i = 16 * j + f < I0 ? 16 * j + f : I0 - 1;
+      const f64x2 *row = (const f64x2 *)(F.p[0] + i * LDR + KQ * g);
+#pragma unroll
+      for (int s = 0; s < KQ / 2; ++s) B.a[s] = row[s];
+#pragma unroll
+      for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const bool in = cb + 16 * t + g + 4 * v < C;
+          B.x[t][v] = *(in ? col[t] + I0 * (4 * v) + i : X);
+        }
+    };
+    auto add = [&](int64_t j, const Buf &B) {
+      f64x4 rec[CT];
+#pragma unroll
+      for (int t = 0; t < CT; ++t) rec[t] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < KQ; ++s)
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+          rec[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(kr[t][s], B.a[s / 2][s % 2], rec[t], 0, 0, 0);
+      const bool row_in = 16 * j + f < I0;
+#pragma unroll
+      for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const double d = (double)B.x[t][v] - rec[t][v];
+          if (row_in && cb + 16 * t + g + 4 * v < C) sum = fma(d, d, sum);
+        }
+    };
+    if (j0 >= j1) continue;
+    Buf b0, b1;
+    load(j0, b0);
+    int64_t j = j0;
+    for (; j + 2 < j1; j += 2) {
+      load(j + 1, b1);
+      add(j, b0);
+      load(j + 2, b0);
+      add(j + 1, b1);
+    }
+    if (j + 1 < j1) {
+      load(j + 1, b1);
+      add(j, b0);
+      add(j + 1, b1);
+    } else {
+      add(j, b0);
+    }
   }
-  block_sum_store<void>(s, partials);
+  block_sum_store<void>(sum, partials + (int64_t)blockIdx.y * gridDim.x);
 }
 
 // Zero fill by vector stores (used where a buffer must start at zero in code a caller may
@@ -255,14 +339,29 @@ void cast_f64_to_f32(hipStream_t s, int64_t n, const double *src, float *dst) {
   k_cast<<<grid_for(n, 256), 256, 0, s>>>(n, src, dst);
 }
 
-void cost_explicit_partials(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *const *fac,
-                            const double *x64, const float *x32, double *partials, int nparts) {
+int cost_explicit_partials(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *const *fac,
+                           const double *x64, const float *x32, double *partials) {
   Dims D = make_dims(N, dims, R);
   FacPtrs F{};
   for (int k = 0; k < N; ++k) F.p[k] = fac[k];
-  int64_t total = 1;
-  for (int k = 0; k < N; ++k) total *= dims[k];
-  k_cost_explicit<<<nparts, 256, 0, s>>>(D, R, ldr, F, total, x64, x32, partials);
+  int64_t C = 1;
+  for (int k = 1; k < N; ++k) C *= dims[k];
+  const int KQ = ldr / 4, CT = KQ <= 8 ? 4 : 2;
+  const int64_t tiles = (dims[0] + 15) / 16;
+  int64_t gx = (C + 64 * CT - 1) / (64 * CT);
+  if (gx > kCostParts) gx = kCostParts;
+  int64_t gy = kCostParts / gx < tiles ? kCostParts / gx : tiles;   // mode 0 split where columns are few
+  const int per = (int)((tiles + gy - 1) / gy);
+  gy = (tiles + per - 1) / per;
+  const dim3 grid((unsigned)gx, (unsigned)gy);
+#define PTN_CE(KQV, CTV)                                                                       \
+  if (KQ == KQV) {                                                                             \
+    if (x64) k_cost_explicit<double, KQV, CTV><<<grid, 256, 0, s>>>(D, C, F, x64, per, partials); \
+    else     k_cost_explicit<float, KQV, CTV><<<grid, 256, 0, s>>>(D, C, F, x32, per, partials);  \
+  }
+  PTN_CE(4, 4) PTN_CE(8, 4) PTN_CE(12, 2) PTN_CE(16, 2)
+#undef PTN_CE
+  return (int)(gx * gy);
 }
 
 void fill_zero(hipStream_t s, void *p, int64_t words) {

@@ -903,9 +903,9 @@ double cost_explicit(Work &w, const double *base) {
   ptn_handle h = w.h;
   const double *fp[kMaxOrder];
   for (int k = 0; k < w.N; ++k) fp[k] = base + w.off[k];
-  cost_explicit_partials(h->stream, w.N, w.dims, w.R, w.ldr, fp, h->x64, h->x64 ? nullptr : h->x32, w.part,
-                         kNormParts);
-  sum_partials(h->stream, w.part, kNormParts, w.scal.p + 3);
+  const int parts = cost_explicit_partials(h->stream, w.N, w.dims, w.R, w.ldr, fp, h->x64,
+                                           h->x64 ? nullptr : h->x32, w.part);   // part_cap >= 256 x 16
+  sum_partials(h->stream, w.part, parts, w.scal.p + 3);
   return std::sqrt(read_scalar(h, w.scal.p + 3));
 }
 

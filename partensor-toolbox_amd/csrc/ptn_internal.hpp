@@ -161,8 +161,10 @@ void square_norm_partials(hipStream_t s, int64_t n, const double *x64, const flo
 void sum_partials(hipStream_t s, const double *partials, int nparts, double *out);
 void noise_scale(hipStream_t s, const double *nx2, const double *ne2, double snr_db, double *scale);
 void cast_f64_to_f32(hipStream_t s, int64_t n, const double *src, float *dst);
-void cost_explicit_partials(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *const *fac,
-                            const double *x64, const float *x32, double *partials, int nparts);
+// partial sums of (X - [[A]])^2 (at most kCostParts of them, returned): factor rows of ldr doubles
+constexpr int kCostParts = 2048;
+int cost_explicit_partials(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *const *fac,
+                           const double *x64, const float *x32, double *partials);
 
 // ---- layout conversion ----
 // zeroes `words` 8-byte words at p with a kernel (no memset node)

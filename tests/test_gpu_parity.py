@@ -157,6 +157,24 @@ def test_cost_explicit_matches_oracle(h):
     assert h.cost_explicit(init) == pytest.approx(o.cost_explicit(X, init), rel=1e-13)
 
 
+@pytest.mark.parametrize("storage", [P.TENSOR_F64, P.TENSOR_F32])
+@pytest.mark.parametrize("dims,R", [((1, 3, 5), 1), ((16, 8, 8), 16), ((17, 13, 5), 17), ((200, 7, 3), 33),
+                                    ((33, 300, 31), 48), ((15, 129, 130), 49), ((31, 9, 10, 7), 64),
+                                    ((3, 4, 3, 5, 6), 20), ((700, 64, 33), 5)])
+def test_cost_explicit_at_the_tiles_edges(h, dims, R, storage):
+    """Rows of mode 0 in tiles of 16, columns in groups of 128 or 256, mode 0 split where columns
+    are few, every padded rank, FP64 and FP32 tensors (FP32 values in both), against numpy in
+    FP64.  A sum of positive terms of few roundings each: 1e-13 relative."""
+    rng = np.random.default_rng(R)
+    X = rng.standard_normal(dims).astype(np.float32).astype(np.float64)
+    A = [rng.random((I, R)) for I in dims]
+    rec = A[0]
+    for a in A[1:]:
+        rec = rec[..., None, :] * a
+    h.set_tensor(X, storage=storage)
+    assert h.cost_explicit(A) == pytest.approx(np.linalg.norm(X - rec.sum(-1)), rel=1e-13)
+
+
 # ------------------------------------------------------------ R x R pieces --
 
 def test_sym_extremes_match_oracle(h, golden_dir):
