@@ -26,6 +26,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // 16-byte loads at element alignment
 
 namespace {
 
@@ -307,154 +308,24 @@ __global__ __launch_bounds__(256, NT >= 4 || MODE == kGemmFp32 ? 2 : 1) void k_g
 }
 
 // ---------------------------------------------------------------------------
-// gemm_ck_f32: each wave owns 64 fibers (2 MFMA row tiles of 32) and walks the
-// contraction in 32-element steps: lane (i, kg) reads 16 consecutive elements (64
-// bytes) of its fiber, so each step consumes whole 128-byte lines.  Operands use the
-// kperm = 1 k order of k_pack_w.  FUSE: the fibers of a wave share one index of the
-// last mode (c = i1 + I1 * i2, 64 consecutive i1 per wave) and the epilogue multiplies
-// each fiber row by the FP64 factor row A1[i1] and sums them: the right node of the
-// order-3 dimension tree (X x_0 A_0, then the TTV with A_1, DimTrees.hpp:668-800) in
-// one pass, written as one partial row per (i2, i1-chunk).
+// gemm_ck_lds: the contraction over the contiguous index, staged through LDS.  A block owns
+// 256 consecutive fibers; per 32-element step each group of 8 consecutive threads reads 128
+// bytes of one fiber at whatever element it starts, the 256 x 32 tile is written to LDS (rows
+// padded to 36 floats, which keeps the 16-byte reads and writes free of bank conflicts), and
+// each wave reads its 64 fibers back in the MFMA layout (the kperm = 1 k order of k_pack_w).
+// The next step's lines are prefetched into registers while the current step is multiplied.
+// A step that reaches past the fiber reads on (the next fiber, or the allocation's zero pad of
+// at least 32 elements after the last) and zeroes those elements in LDS.
+// NTL: non-temporal loads where every 128 bytes are a line of their own (L a multiple of 32);
+// elsewhere a line is read by two steps, and cached loads keep it (701 x 555 x 333, R = 20: 383 us
+// when a length that is no multiple of 4 was read element by element from memory, 138 now;
+// 700 x 555 x 333 184 us with non-temporal loads, 143 with cached ones).
+// FUSE: the block's fibers share one index of the last mode (c = i1 + I1 * i2, 64 consecutive
+// i1 per wave) and the epilogue multiplies each fiber row by the FP64 factor row A1[i1] and
+// sums them: the right node of the order-3 dimension tree (X x_0 A_0, then the TTV with A_1,
+// DimTrees.hpp:668-800) in one pass, written as one partial row per (i2, i1-chunk).
 // ---------------------------------------------------------------------------
-template <int MODE, int NT, bool VEC, bool FUSE>
-__global__ __launch_bounds__(256) void k_gemm_ck_f32(const float *__restrict__ X, int64_t L, int64_t C, int64_t I1,
-                                                     const bf16x8 *__restrict__ whi, const bf16x8 *__restrict__ wlo,
-                                                     const float *__restrict__ wf, float *__restrict__ T,
-                                                     const double *__restrict__ A1, int ldr,
-                                                     double *__restrict__ part) {
-  constexpr int RPF = 32 * NT;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane & 31, kg = lane >> 5;
-  const int64_t wid = (int64_t)blockIdx.x * 4 + wave;
-  int64_t cb, nfib, i1b = 0, i2 = 0;
-  if (FUSE) {
-    const int64_t wpf = (I1 + 63) / 64;
-    i2 = wid / wpf;
-    i1b = (wid % wpf) * 64;
-    cb = i1b + I1 * i2;
-    nfib = I1 - i1b < 64 ? I1 - i1b : 64;
-    if (i2 * I1 >= C) return;
-  } else {
-    cb = wid * 64;
-    if (cb >= C) return;
-    nfib = C - cb < 64 ? C - cb : 64;
-  }
-
-  f32x16 acc[2][NT];
-#pragma unroll
-  for (int s = 0; s < 2; ++s)
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[s][t][v] = 0.f;
-
-  // Unconditional loads and nothing zeroed: a missing fiber reads fiber cb and only
-  // fills its own (discarded) row of D; elements a >= L meet the zero rows of the
-  // packed operand.  VEC (L % 4 == 0) reads whole 32-element steps: past the end of a
-  // fiber that is the next fiber, and past the last fiber the allocation's zero pad
-  // (at least 32 elements).  The next step's loads are clamped to the last step, so
-  // every iteration takes the same path.
-  const float *f0 = X + L * (cb + (i < nfib ? i : 0));
-  const float *f1 = X + L * (cb + (32 + i < nfib ? 32 + i : 0));
-  const int64_t alast = ((L - 1) / 32) * 32;
-  float xn[2][16];
-  auto load = [&](int64_t a0, float (&dst)[2][16]) {
-    const int64_t a = (a0 < alast ? a0 : alast) + 16 * kg;
-    if (VEC) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4 u = __builtin_nontemporal_load((const f32x4 *)(f0 + a + 4 * q));
-        const f32x4 w = __builtin_nontemporal_load((const f32x4 *)(f1 + a + 4 * q));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { dst[0][4 * q + j] = u[j]; dst[1][4 * q + j] = w[j]; }
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int64_t ac = a + j < L ? a + j : L - 1;
-        dst[0][j] = f0[ac];
-        dst[1][j] = f1[ac];
-      }
-    }
-  };
-  load(0, xn);
-  for (int64_t a0 = 0; a0 < L; a0 += 32) {
-    float xc[2][16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) { xc[0][j] = xn[0][j]; xc[1][j] = xn[1][j]; }
-    const int64_t s32 = a0 >> 5;
-    // this step's packed operand first: memory counters retire in order, so loads
-    // issued after the next step's tensor loads would make the MFMAs wait for them
-    bf16x8 bh[2][NT], bl[2][NT];
-    f32x8 bf[2][NT];
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        if constexpr (MODE == kGemmBf16x3) {
-          bh[s2][t] = whi[((s32 * 2 + s2) * NT + t) * 64 + lane];
-          bl[s2][t] = wlo[((s32 * 2 + s2) * NT + t) * 64 + lane];
-        } else {
-          bf[s2][t] = ((const f32x8 *)wf)[((s32 * 2 + s2) * NT + t) * 64 + lane];
-        }
-      }
-    load(a0 + 32, xn);
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      float x0[8], x1[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) { x0[j] = xc[0][8 * s2 + j]; x1[j] = xc[1][8 * s2 + j]; }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        // FP32 path: lane (c, kg) supplies W[a0 + 16 kg + 8 s2 + q][c] at MFMA step q
-        mma_step<MODE>(x0, bh[s2][t], bl[s2][t], bf[s2][t], acc[0][t]);
-        mma_step<MODE>(x1, bh[s2][t], bl[s2][t], bf[s2][t], acc[1][t]);
-      }
-    }
-  }
-  if (!FUSE) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t f = 32 * s + 8 * (v / 4) + 4 * kg + (v % 4);
-        if (f < nfib) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t) T[(cb + f) * RPF + 32 * t + i] = acc[s][t][v];
-        }
-      }
-    return;
-  }
-  // fused TTV with A1 over the wave's fibers (FP64 accumulation)
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int col = 32 * t + i;
-    double sum = 0.0;
-    if (col < ldr) {
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int64_t f = 32 * s + 8 * (v / 4) + 4 * kg + (v % 4);
-          if (f < nfib) sum = fma((double)acc[s][t][v], A1[(i1b + f) * ldr + col], sum);
-        }
-    }
-    sum += __shfl_xor(sum, 32, 64);
-    if (kg == 0 && col < ldr) part[wid * ldr + col] = sum;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// gemm_ck_lds: the same contraction as gemm_ck_f32 (L % 4 == 0) with the tensor staged
-// through LDS.  A block owns 256 consecutive fibers; per 32-element step each group of
-// 8 consecutive threads reads one whole 128-byte line of one fiber (global requests are
-// full lines), the 256 x 32 tile is written to LDS (rows padded to 36 floats, which
-// keeps the 16-byte reads and writes free of bank conflicts), and each wave reads its
-// 64 fibers back in the MFMA layout.  The next step's lines are prefetched into
-// registers while the current step is multiplied.  FUSE as in gemm_ck_f32, with the
-// block's fibers inside one index of the last mode.
-// ---------------------------------------------------------------------------
-template <int MODE, int NT, bool FUSE>
+template <int MODE, int NT, bool FUSE, bool NTL>
 __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X, int64_t L, int64_t C, int64_t I1,
                                                      const bf16x8 *__restrict__ whi, const bf16x8 *__restrict__ wlo,
                                                      const float *__restrict__ wf, float *__restrict__ T,
@@ -492,7 +363,10 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
   auto fetch = [&](int64_t a0) {
     const int64_t a = a0 < alast ? a0 : alast;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) pre[q] = __builtin_nontemporal_load((const f32x4 *)(src[q] + a));
+    for (int q = 0; q < 8; ++q) {
+      if constexpr (NTL) pre[q] = __builtin_nontemporal_load((const f32x4 *)(src[q] + a));
+      else pre[q] = *(const f32x4u *)(src[q] + a);
+    }
   };
 
   f32x16 acc[2][NT];
@@ -506,6 +380,14 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
   fetch(0);
   for (int64_t a0 = 0; a0 < L; a0 += 32) {
     __syncthreads();
+    if constexpr (!NTL) {
+      if (a0 + 32 > L) {                        // the last step of a length that is no multiple of 32
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) pre[q][j] = a0 + k4 + j < L ? pre[q][j] : 0.f;
+      }
+    }
 #pragma unroll
     for (int q = 0; q < 8; ++q) *(f32x4 *)(tile + (32 * q + (tid >> 3)) * LDP + k4) = pre[q];
     __syncthreads();
@@ -681,38 +563,23 @@ void gemm_ck_f32(hipStream_t s, GemmMode mode, const float *x32, int64_t L, int6
                  double *part) {
   const bool fuse = fuse_I1 > 0;
   const bf16x8 *h = (const bf16x8 *)whi, *l = (const bf16x8 *)wlo;
-  const bool vec = (L % 4) == 0;
-  if (vec) {
-    const int64_t blocks = fuse ? (C / fuse_I1) * ((fuse_I1 + 255) / 256) : (C + 255) / 256;
-    dim3 g2((unsigned)blocks);
-#define PTN_CKL(MODEV, NTV, FUSEV) \
-  k_gemm_ck_lds<MODEV, NTV, FUSEV><<<g2, 256, 0, s>>>(x32, L, C, fuse_I1, h, l, wf, T, A1, ldr, part)
-    if (mode == kGemmBf16x3) {
-      if (RPF == 32) { if (fuse) PTN_CKL(kGemmBf16x3, 1, true); else PTN_CKL(kGemmBf16x3, 1, false); }
-      else           { if (fuse) PTN_CKL(kGemmBf16x3, 2, true); else PTN_CKL(kGemmBf16x3, 2, false); }
-    } else {
-      if (RPF == 32) { if (fuse) PTN_CKL(kGemmFp32, 1, true); else PTN_CKL(kGemmFp32, 1, false); }
-      else           { if (fuse) PTN_CKL(kGemmFp32, 2, true); else PTN_CKL(kGemmFp32, 2, false); }
-    }
-#undef PTN_CKL
-    return;
-  }
-  const int64_t waves = fuse ? (C / fuse_I1) * ((fuse_I1 + 63) / 64) : (C + 63) / 64;
-  dim3 grid((unsigned)((waves + 3) / 4));
-#define PTN_CK32(MODEV, NTV, VECV, FUSEV)                                                                  \
-  k_gemm_ck_f32<MODEV, NTV, VECV, FUSEV><<<grid, 256, 0, s>>>(x32, L, C, fuse_I1, h, l, wf, T, A1, ldr, part)
-#define PTN_CK32_F(MODEV, NTV, VECV) \
-  { if (fuse) PTN_CK32(MODEV, NTV, VECV, true); else PTN_CK32(MODEV, NTV, VECV, false); }
-#define PTN_CK32_V(MODEV, NTV) \
-  { if (vec) PTN_CK32_F(MODEV, NTV, true) else PTN_CK32_F(MODEV, NTV, false) }
+  const int64_t blocks = fuse ? (C / fuse_I1) * ((fuse_I1 + 255) / 256) : (C + 255) / 256;
+  const dim3 g2((unsigned)blocks);
+#define PTN_CKL(MODEV, NTV, FUSEV)                                                                        \
+  do {                                                                                                    \
+    if (L % 32 == 0)                                                                                      \
+      k_gemm_ck_lds<MODEV, NTV, FUSEV, true><<<g2, 256, 0, s>>>(x32, L, C, fuse_I1, h, l, wf, T, A1, ldr, part);  \
+    else                                                                                                  \
+      k_gemm_ck_lds<MODEV, NTV, FUSEV, false><<<g2, 256, 0, s>>>(x32, L, C, fuse_I1, h, l, wf, T, A1, ldr, part); \
+  } while (0)
   if (mode == kGemmBf16x3) {
-    if (RPF == 32) PTN_CK32_V(kGemmBf16x3, 1) else PTN_CK32_V(kGemmBf16x3, 2)
+    if (RPF == 32) { if (fuse) PTN_CKL(kGemmBf16x3, 1, true); else PTN_CKL(kGemmBf16x3, 1, false); }
+    else           { if (fuse) PTN_CKL(kGemmBf16x3, 2, true); else PTN_CKL(kGemmBf16x3, 2, false); }
   } else {
-    if (RPF == 32) PTN_CK32_V(kGemmFp32, 1) else PTN_CK32_V(kGemmFp32, 2)
+    if (RPF == 32) { if (fuse) PTN_CKL(kGemmFp32, 1, true); else PTN_CKL(kGemmFp32, 1, false); }
+    else           { if (fuse) PTN_CKL(kGemmFp32, 2, true); else PTN_CKL(kGemmFp32, 2, false); }
   }
-#undef PTN_CK32_V
-#undef PTN_CK32_F
-#undef PTN_CK32
+#undef PTN_CKL
 }
 
 void reduce_chunks(hipStream_t s, const double *part, int64_t I2, int64_t wpf, int ldr, double *M) {

@@ -589,6 +589,35 @@ def test_work_buffers_shared_between_handles_and_threads():
     assert not bad
 
 
+@pytest.mark.parametrize("R", [3, 32, 33, 64])
+@pytest.mark.parametrize("dims", [(1, 7, 9), (3, 300, 5), (31, 17, 33), (32, 64, 5), (33, 20, 30), (50, 257, 3),
+                                  (97, 10, 11), (130, 9, 8)])
+def test_fp32_fibre_contraction_at_unaligned_lengths(h, dims, R):
+    """The FP32 and bf16x3 contractions over mode 0 read fibres in 32-element steps wherever they
+    start.  Small integers make every product and sum exact in both (below 2^24, 16 bits of
+    split products), so the MTTKRPs of modes 1 and 2 must equal numpy's; an infinity at the start
+    of a fibre stays in the rows that contain it, though the fibre before is read past its end."""
+    rng = np.random.default_rng(R)
+    X = rng.integers(-8, 9, dims).astype(np.float64)
+    A = [rng.integers(-4, 5, (I, R)).astype(np.float64) for I in dims]
+    for fill in (None, np.inf):
+        if fill is not None:
+            X[0, 3, 2] = fill
+            A[0][0], A[1][3], A[2][2] = 1.0, 1.0, 1.0
+        h.set_tensor(X, storage=P.TENSOR_F32)
+        T = np.tensordot(A[0], X, axes=(0, 0))                       # R x I1 x I2
+        clean = {1: np.arange(dims[1]) != 3, 2: np.arange(dims[2]) != 2}
+        for arith in (P.ARITH_F32, P.ARITH_BF16X3):
+            for mode in (1, 2):
+                keep = clean[mode] if fill is not None else slice(None)
+                with np.errstate(invalid="ignore"):
+                    want = np.einsum("rjk,kr->jr", T, A[2]) if mode == 1 else np.einsum("rjk,jr->kr", T, A[1])
+                got = h.mttkrp(A, mode, arith=arith)
+                assert np.array_equal(got[keep], want[keep])
+                if fill is not None:
+                    assert not np.isfinite(got[~keep]).any()
+
+
 @pytest.mark.parametrize("dims", [(100, 100, 100), (60, 127, 128), (40, 50, 61, 85)])
 def test_fp32_products_with_splits_past_the_last_column(h, dims):
     """k chunks are rounded up to 16 columns, so the last of many splits can start past the end
