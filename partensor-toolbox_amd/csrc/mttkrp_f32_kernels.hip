@@ -468,6 +468,142 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
   }
 }
 
+// ---------------------------------------------------------------------------
+// gemm_ck_few: gemm_ck_lds (unfused) for so few fibers that blocks of 256 leave CUs idle.  A
+// block is m x NT waves on 32 m fibers, each wave one 32 x 32 tile of the result, with m chosen
+// so that the blocks come out even on the 256 CUs (few_tiles).  The staged tile is 64 elements
+// of each fiber, in two of gemm_ck_lds's 32-element steps: the same products in the same order.
+// Tiles alternate between two LDS buffers, one barrier each; the next tile's operand fragments
+// and the tensor elements of the tile after it are on their way while a tile is multiplied.
+// The order-4 right node at 200^4 has 40 000 fibers of 40 000 elements, 157 blocks of 256: FP32
+// products at R = 64 3.16 -> 2.29 ms (MFMA-bound: 1.34 ms at the peak, 1.65 with its 2500 tiles
+// on 1024 SIMDs), bf16x3 1.98 -> 1.28 ms (5.0 TB/s), at R = 20 1.80 -> 1.11 ms.
+// ---------------------------------------------------------------------------
+template <int MODE, int NT, bool NTL>
+__global__ __launch_bounds__(384 * NT) void k_gemm_ck_few(const float *__restrict__ X, int64_t L, int64_t C,
+                                                     const bf16x8 *__restrict__ whi, const bf16x8 *__restrict__ wlo,
+                                                     const float *__restrict__ wf, float *__restrict__ T) {
+  constexpr int RPF = 32 * NT, KS = 64, LDP = KS + 4, NQ = 8 / NT;
+  extern __shared__ __align__(16) float tiles[];                  // 2 x (32 m x LDP)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t = wave % NT, ft = wave / NT, m = blockDim.x / (64 * NT);
+  const int i = lane & 31, kg = lane >> 5;
+  const int64_t cb = (int64_t)blockIdx.x * (32 * m);
+  const int nfb = C - cb < 32 * m ? (int)(C - cb) : 32 * m;
+  // global side: instruction q reads fiber 4 m NT q + tid / 16, elements 4 (tid % 16) .. + 3 (where
+  // the last 32-element step is the first half of a tile, the second half reads it again)
+  const int k4 = 4 * (tid & 15), fstep = 4 * m * NT, f0 = tid >> 4;
+  const float *src[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int fl = fstep * q + f0;
+    src[q] = X + L * (cb + (fl < nfb ? fl : 0));
+  }
+  const int64_t nstep = (L + 31) / 32, alast = 32 * (nstep - 1), nfull = nstep / 2;
+  f32x4 pre[NQ];
+  auto fetch = [&](int64_t n, int q0, int q1) {
+    int64_t a = KS * n + (k4 & 32);
+    a = (a < alast ? a : alast) + (k4 & 31);
+#pragma unroll
+    for (int q = q0; q < q1; ++q) {
+      if constexpr (NTL) pre[q] = __builtin_nontemporal_load((const f32x4 *)(src[q] + a));
+      else pre[q] = *(const f32x4u *)(src[q] + a);
+    }
+  };
+  auto store = [&](int64_t n) {
+    if constexpr (!NTL) {
+      if (KS * (n + 1) > L) {                   // elements past the fiber
+        const int64_t a = KS * n + k4;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) pre[q][j] = a + j < L ? pre[q][j] : 0.f;
+      }
+    }
+    float *buf = tiles + (n & 1) * (32 * m * LDP) + k4;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) *(f32x4 *)(buf + (fstep * q + f0) * LDP) = pre[q];
+  };
+  struct Frag {                                 // the operand of a tile: four 16-wide k steps
+    bf16x8 h[4], l[4];
+    f32x8 f[4];
+  };
+  auto operand = [&](int64_t n, Frag &B, int u0, int u1) {
+#pragma unroll
+    for (int u = u0; u < u1; ++u) {
+      const int64_t s16 = 4 * n + u < 2 * nstep ? 4 * n + u : 2 * nstep - 1;
+      if constexpr (MODE == kGemmBf16x3) {
+        B.h[u] = whi[(s16 * NT + t) * 64 + lane];
+        B.l[u] = wlo[(s16 * NT + t) * 64 + lane];
+      } else {
+        B.f[u] = ((const f32x8 *)wf)[(s16 * NT + t) * 64 + lane];
+      }
+    }
+  };
+  f32x16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  auto values = [&](int64_t n, int hf, float (&xc)[16]) {
+    const float *row = tiles + (n & 1) * (32 * m * LDP) + (32 * ft + i) * LDP + 32 * hf + 16 * kg;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 u = *(const f32x4 *)(row + 4 * q);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) xc[4 * q + j] = u[j];
+    }
+  };
+  auto multiply = [&](const float (&xc)[16], int s2, const Frag &B, int u) {
+    float x0[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x0[j] = xc[8 * s2 + j];
+    mma_step<MODE>(x0, B.h[u], B.l[u], B.f[u], acc);
+  };
+  // tile n, with tile n + 1's elements stored and operand and tile n + 2's elements requested
+  // before it (past the last tile: the last step again, not used)
+  auto turn = [&](int64_t n, const Frag &cur, Frag &nxt) {
+    store(n + 1);
+    operand(n + 1, nxt, 0, 4);
+    fetch(n + 2, 0, NQ);
+    __builtin_amdgcn_sched_barrier(0);          // the requests stay ahead of the products
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      float xc[16];
+      values(n, hf, xc);
+      multiply(xc, 0, cur, 2 * hf);
+      multiply(xc, 1, cur, 2 * hf + 1);
+    }
+    __syncthreads();
+  };
+  auto half_tile = [&](int64_t n, const Frag &cur) {
+    float xc[16];
+    values(n, 0, xc);
+    multiply(xc, 0, cur, 0);
+    multiply(xc, 1, cur, 1);
+  };
+  Frag b0, b1;
+  fetch(0, 0, NQ);
+  operand(0, b0, 0, 4);
+  store(0);
+  fetch(1, 0, NQ);
+  __syncthreads();
+  int64_t n = 0;
+  for (; n + 2 <= nfull; n += 2) {
+    turn(n, b0, b1);
+    turn(n + 1, b1, b0);
+  }
+  if (n < nfull) {
+    turn(n, b0, b1);
+    if (nstep & 1) half_tile(n + 1, b1);
+  } else if (nstep & 1) {
+    half_tile(n, b0);
+  }
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int f = 32 * ft + 8 * (v / 4) + 4 * kg + (v % 4);
+    if (f < nfb) T[(cb + f) * RPF + 32 * t + i] = acc[v];
+  }
+}
+
 // M[i2][r] = sum over the i1-chunks of the fused right node, in chunk order.
 __global__ void k_reduce_chunks(const double *__restrict__ part, int64_t I2, int64_t wpf, int ldr,
                                 double *__restrict__ M) {
@@ -558,11 +694,46 @@ void gemm_cm_f32(hipStream_t s, GemmMode mode, const float *x32, int64_t M, int6
 #undef PTN_CM32K
 }
 
+// Tiles of 32 fibers per block of k_gemm_ck_few, or 0 for k_gemm_ck_lds, by the fiber count.
+// Above 200 000 fibers blocks of 256 fill the chip (250 000: bf16x3 157 us against 166 at R = 64,
+// 160 000: 309 against 274).  Below 16 384 a block's own latency decides, and for FP32 products,
+// bound by the matrix cores, so do the SIMDs that it leaves idle (90 000, R = 64: 610 us at m = 1,
+// 645 at 4, 927 at 5): one tile.  Otherwise the m of 2 .. 5 whose blocks leave the fewest tiles
+// to the busiest CU (40 000: m = 5, 250 blocks, 1.28 ms, against 1.77 at m = 4, 313 blocks).
+static int few_tiles(GemmMode mode, int NT, int64_t C) {
+  if (C > 200000) return 0;
+  if (C < 16384 || (mode == kGemmFp32 && (NT == 2 || C < 65536))) return 1;
+  int best = 1;
+  int64_t most = INT64_MAX;
+  for (int m = 2; m <= 5; ++m) {
+    const int64_t blocks = (C + 32 * m - 1) / (32 * m), tiles = (blocks + 255) / 256 * m;
+    if (tiles <= most) {
+      most = tiles;
+      best = m;
+    }
+  }
+  return best;
+}
+
 void gemm_ck_f32(hipStream_t s, GemmMode mode, const float *x32, int64_t L, int64_t C, int RPF, const void *whi,
                  const void *wlo, const float *wf, float *T, int64_t fuse_I1, const double *A1, int ldr,
                  double *part) {
   const bool fuse = fuse_I1 > 0;
   const bf16x8 *h = (const bf16x8 *)whi, *l = (const bf16x8 *)wlo;
+  if (const int m = fuse ? 0 : few_tiles(mode, RPF / 32, C)) {
+    const int NT = RPF / 32;
+    const dim3 g((unsigned)((C + 32 * m - 1) / (32 * m)));
+    const size_t lds = (size_t)2 * 32 * m * 68 * sizeof(float);
+#define PTN_CKF(MODEV, NTV)                                                                                  \
+  do {                                                                                                       \
+    if (L % 32 == 0) k_gemm_ck_few<MODEV, NTV, true><<<g, 64 * NTV * m, lds, s>>>(x32, L, C, h, l, wf, T);     \
+    else k_gemm_ck_few<MODEV, NTV, false><<<g, 64 * NTV * m, lds, s>>>(x32, L, C, h, l, wf, T);                \
+  } while (0)
+    if (mode == kGemmBf16x3) { if (NT == 1) PTN_CKF(kGemmBf16x3, 1); else PTN_CKF(kGemmBf16x3, 2); }
+    else                     { if (NT == 1) PTN_CKF(kGemmFp32, 1); else PTN_CKF(kGemmFp32, 2); }
+#undef PTN_CKF
+    return;
+  }
   const int64_t blocks = fuse ? (C / fuse_I1) * ((fuse_I1 + 255) / 256) : (C + 255) / 256;
   const dim3 g2((unsigned)blocks);
 #define PTN_CKL(MODEV, NTV, FUSEV)                                                                        \

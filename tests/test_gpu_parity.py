@@ -618,6 +618,23 @@ def test_fp32_fibre_contraction_at_unaligned_lengths(h, dims, R):
                     assert not np.isfinite(got[~keep]).any()
 
 
+@pytest.mark.parametrize("R", [7, 40])
+@pytest.mark.parametrize("dims", [(31, 127, 129), (32, 127, 129), (33, 128, 129), (64, 160, 250), (65, 200, 331),
+                                  (97, 256, 257), (96, 300, 301), (63, 400, 501), (40, 447, 450)])
+def test_fp32_fibre_contraction_at_the_block_shapes_edges(h, dims, R):
+    """Fibre counts below and above 16384, 65536 and 200000, where the block goes from one tile of
+    32 fibres to 2 .. 5 to the blocks of 256, fibres of one half, one and several 64-element
+    tiles.  Small integers: exact, as above."""
+    rng = np.random.default_rng(R)
+    X = rng.integers(-8, 9, dims).astype(np.float64)
+    A = [rng.integers(-4, 5, (I, R)).astype(np.float64) for I in dims]
+    h.set_tensor(X, storage=P.TENSOR_F32)
+    T = np.tensordot(A[0], X, axes=(0, 0))
+    want = np.einsum("rjk,kr->jr", T, A[2])
+    for arith in (P.ARITH_F32, P.ARITH_BF16X3):
+        assert np.array_equal(h.mttkrp(A, 1, arith=arith), want)
+
+
 @pytest.mark.parametrize("dims", [(100, 100, 100), (60, 127, 128), (40, 50, 61, 85)])
 def test_fp32_products_with_splits_past_the_last_column(h, dims):
     """k chunks are rounded up to 16 columns, so the last of many splits can start past the end
