@@ -20,7 +20,8 @@ constexpr int kBMax = 128;    // largest mode size
 
 struct BatchLds {
   double F[2][kBMax * kBR];   // the two factors a contraction multiplies by; during a solve
-                              // the two Nesterov extrapolation points; F[0] then the result
+                              // (256-thread blocks) the two Nesterov extrapolation points;
+                              // F[0] then the result
   double M[kBMax * kBR];      // MTTKRP of the mode being updated
   double G[3][kBR * kBR];     // Grams of the current factors
   double V[kBR * kBR];        // Hadamard product for the mode being updated
@@ -427,12 +428,21 @@ __device__ __forceinline__ void mttkrp_block(const float *X, int Iout, int Ia, i
 // result, after the zero-column fallback (Cpd.hpp:206-207, an exact-zero test of each
 // column), to Ag (global rows, which hold the start point on entry) and to S.F[0]; returns
 // the step count.
+//
+// The A fragments read one column of 16 consecutive rows: rows of 16 doubles put them on two
+// bank pairs (8-way conflicts, on the path of every step of every wave), rows of 18 on all.
+// 512-thread blocks keep Y in the LDS of the MTTKRP's partial bands (P, idle during a solve)
+// with rows of 18 (512-problem batch, 20 sweeps: FP32 matrix cores 1.24 -> 1.19 ms per sweep,
+// FP64 ones 1.36 -> 1.29, with one copy of the rest of the sweep for all ranks); 256-thread
+// blocks, whose LDS just lets two share a CU, in F with rows of 16.
 template <int BS, int RP>
-__device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *Ag, double d1, double d2, int max_inner) {
+__device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *P, double *Ag, double d1, double d2,
+                                          int max_inner) {
+  constexpr int kYS = BS == 512 ? 18 : kBR;
   constexpr int NW = BS / 64, TPW = (kBMax / 16 + NW - 1) / NW, NQ = RP / 4;
   const int t = tid(), lane = t & 63, wave = t >> 6, m = lane & 15, kk = lane >> 4;
   const int T = (I + 15) / 16;
-  double *Yb0 = S.F[0], *Yb1 = S.F[1];
+  double *Yb0 = BS == 512 ? P : S.F[0], *Yb1 = BS == 512 ? P + kBMax * kYS : S.F[1];
   const double lambda = S.prm.lambda, L = S.prm.L, invL = 1.0 / L;
   double zb[NQ];
 #pragma unroll
@@ -453,8 +463,8 @@ __device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *Ag,
         const double a0 = on ? Ag[row * kBR + m] : 0.0;
         ac[tt][j] = a0;
         wt[tt][j] = on ? S.M[row * kBR + m] + lambda * a0 : 0.0;
-        Yb0[row * kBR + m] = a0;                       // columns >= R: exact zeros in both
-        if (!on) Yb1[row * kBR + m] = 0.0;
+        Yb0[row * kYS + m] = a0;                       // columns >= R: exact zeros in both
+        if (!on) Yb1[row * kYS + m] = 0.0;
       }
     }
   }
@@ -482,9 +492,9 @@ __device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *Ag,
         const int ra = tile * 16 + m;                  // A fragment row (rows past I: not used)
         double af[NQ], yv[4];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) af[q] = Y[(ra < kBMax ? ra : 0) * kBR + 4 * q + kk];
+        for (int q = 0; q < NQ; ++q) af[q] = Y[(ra < kBMax ? ra : 0) * kYS + 4 * q + kk];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) yv[j] = Y[(tile * 16 + kk + 4 * j) * kBR + m];
+        for (int j = 0; j < 4; ++j) yv[j] = Y[(tile * 16 + kk + 4 * j) * kYS + m];
         f64x4 g = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int q = 0; q < NQ; ++q) g = __builtin_amdgcn_mfma_f64_16x16x4f64(af[q], zb[q], g, 0, 0, 0);
@@ -500,7 +510,7 @@ __device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *Ag,
           const double av = tq > 0.0 ? tq : 0.0;
           if (valid) an[tt][j] = av;
           const double yn = (1.0 + beta) * av - beta * ac[tt][j];
-          if (valid) Yn[row * kBR + m] = yn;
+          if (valid) Yn[row * kYS + m] = yn;
         }
       }
     }
@@ -547,7 +557,7 @@ __device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *Ag,
         double v = ac[tt][j];
         if (fb) v = 0.9 * v + 0.1 * Ag[row * kBR + m];
         Ag[row * kBR + m] = v;
-        Yb0[row * kBR + m] = v;
+        S.F[0][row * kBR + m] = v;
       }
     }
   __syncthreads();
@@ -558,7 +568,7 @@ __device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *Ag,
 // Member g of the problem's group: member 0 works on the problem's state and writes its
 // status and log; members g > 0 on private copies of the state (identical values: every
 // member takes the same steps on the same data).
-template <int BS, int RP, bool F32>
+template <int BS, bool F32>
 __device__ __forceinline__ void sweep_problem(const BatchArgs &a, int p, int g, int sweep, BatchLds &S, double *P) {
   constexpr int NW = BS / 64;                  // the last wave solves the eigenproblem first
   const BatchDesc &d = a.desc[p];
@@ -599,7 +609,14 @@ __device__ __forceinline__ void sweep_problem(const BatchArgs &a, int p, int g, 
     // the MTTKRP (the same share made that sweep 1.49 -> 1.53 ms)
     if constexpr (F32) mttkrp_block<BS, F32, 4>(X + (int64_t)n * a.xcopy, In, Ia, Ib, S, P, NW - 1, grp, eig);
     else mttkrp_block<BS, F32, 3>(X + (int64_t)n * a.xcopy, In, Ia, Ib, S, P, NW, grp, eig);
-    const int it = nnls_block<BS, RP>(In, R, S, n == 0 ? A0 : n == 1 ? A1 : A2, a.d1, a.d2, a.max_inner);
+    double *An = n == 0 ? A0 : n == 1 ? A1 : A2;
+    int it;
+    switch ((R + 3) >> 2) {                    // R rounded up to the MFMA's k: the solve alone
+      case 1: it = nnls_block<BS, 4>(In, R, S, P, An, a.d1, a.d2, a.max_inner); break;
+      case 2: it = nnls_block<BS, 8>(In, R, S, P, An, a.d1, a.d2, a.max_inner); break;
+      case 3: it = nnls_block<BS, 12>(In, R, S, P, An, a.d1, a.d2, a.max_inner); break;
+      default: it = nnls_block<BS, 16>(In, R, S, P, An, a.d1, a.d2, a.max_inner); break;
+    }
     if (t == 0) S.iters[n] = it;
     gram_block<BS>(S.F[0], In, R, S.G[n]);
     if (n == 2) {
@@ -729,12 +746,7 @@ __global__ __launch_bounds__(BS, 2) void k_batch_sweep(BatchArgs a) {
     __syncthreads();
     if (q >= a.nitems) break;
     const int item = a.order[q], p = item >> 3, g = item & 7;   // (problem, member)
-    switch ((a.desc[p].R + 3) >> 2) {
-      case 1: sweep_problem<BS, 4, F32>(a, p, g, sweep, S, P); break;
-      case 2: sweep_problem<BS, 8, F32>(a, p, g, sweep, S, P); break;
-      case 3: sweep_problem<BS, 12, F32>(a, p, g, sweep, S, P); break;
-      default: sweep_problem<BS, 16, F32>(a, p, g, sweep, S, P); break;
-    }
+    sweep_problem<BS, F32>(a, p, g, sweep, S, P);
   }
 }
 
