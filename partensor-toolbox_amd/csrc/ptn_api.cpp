@@ -7,6 +7,7 @@
 #include "ptn_internal.hpp"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <functional>
@@ -2187,8 +2188,9 @@ ptn_status ptn_cpd_batch(ptn_handle h, const double *init_packed, const ptn_opti
     double tune_s = 0.0;
     const bool tune = block == 0;
     if (tune) {
-      // autotuner: a few launch shapes, each timed over the first two sweeps from the
-      // same state (saved here and restored after every candidate)
+      // autotuner: two launch shapes, each timed over the first two sweeps from the same
+      // state (saved here and restored after every candidate).  Timing four shapes took 13 of
+      // the 50 ms of 20 sweeps of 512 problems, two take 4.8.
       const auto t0 = std::chrono::steady_clock::now();
       HIPCHK(hipMemcpyAsync(st_snap.p, st.p, P * sizeof(BatchProb), hipMemcpyDeviceToDevice, s));
       HIPCHK(hipMemcpyAsync(fac_snap.p, fac.p, nr * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -2201,21 +2203,38 @@ ptn_status ptn_cpd_batch(ptn_handle h, const double *init_packed, const ptn_opti
         HIPCHK(hipMemcpyAsync(grams.p, grams_snap.p, grams.n * sizeof(double), hipMemcpyDeviceToDevice, s));
         restart();
       };
-      const int cand[][2] = {{256, 2 * cu}, {256, cu}, {512, cu}, {512, cu / 2 > 0 ? cu / 2 : 1}};
+      // The candidates, the one more often best first.  Every problem on a block of its own
+      // at once: 512 threads, on one block per CU or per two (8 .. 200 problems of modes
+      // 16 .. 128 were within 5% of each other).  More problems than CUs: 512 threads, or 256
+      // with two blocks per CU, which suits many small problems (2000 of modes 16 .. 32: 1.84
+      // against 1.21 ms per sweep; 512 of modes 16 .. 128: 1.18 against 1.78).  256 threads on
+      // one block per CU were never best (1.02 .. 1.7 times the best of these), nor half the
+      // CUs with more problems (1.2 .. 2 times).
+      const std::vector<std::array<int, 2>> cand =
+          P <= cu ? std::vector<std::array<int, 2>>{{512, cu}, {512, std::max(cu / 2, 1)}}
+                  : std::vector<std::array<int, 2>>{{512, cu}, {256, 2 * cu}};
       const int tsweeps = std::min(2, o.max_iter);
-      double best = 1e300;
+      double best = 1e300, best_first = 1e300;
       TimingEvents ev(h);
       for (const auto &c : cand) {
         set_shape(c[1]);
         restore();
-        HIPCHK(hipEventRecord(ev.e[0], s));
+        // two sweeps, the second only if the first came within a fifth of the best first one
+        double ms = 0.0;
         for (int k = 0; k < tsweeps; ++k) {
+          HIPCHK(hipEventRecord(ev.e[0], s));
           batch_sweep(s, a, c[0], c[1]);
           batch_next_sweep(s, ctr.p);
+          HIPCHK(hipEventRecord(ev.e[1], s));
+          const double t = ev.ms(h);
+          HIPCHK(hipGetLastError());
+          ms += t;
+          if (k == 0 && t > 1.2 * best_first) {
+            ms = 1e300;
+            break;
+          }
+          if (k == 0) best_first = std::min(best_first, t);
         }
-        HIPCHK(hipEventRecord(ev.e[1], s));
-        const double ms = ev.ms(h);
-        HIPCHK(hipGetLastError());
         if (ms < best) {
           best = ms;
           block = c[0];
