@@ -532,7 +532,18 @@ __global__ void k_reduce_splits_x2(const f64x2 *__restrict__ partials, int split
                                    f64x2 *__restrict__ out) {
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n2; e += (int64_t)gridDim.x * blockDim.x) {
     f64x2 s = {0.0, 0.0};
-    for (int q = 0; q < splits; ++q) {
+    int q = 0;
+    for (; q + 8 <= splits; q += 8) {           // eight loads in flight (39 splits of 100 rows 11 -> 6 us)
+      f64x2 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = partials[(q + j) * n2 + e];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        s[0] += v[j][0];
+        s[1] += v[j][1];
+      }
+    }
+    for (; q < splits; ++q) {
       const f64x2 v = partials[q * n2 + e];
       s[0] += v[0];
       s[1] += v[1];

@@ -12,6 +12,8 @@ namespace ptn {
 
 namespace {
 
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
 struct GramPtrs {
   const double *p[kMaxOrder];
 };
@@ -61,32 +63,59 @@ __device__ __forceinline__ void gram_rows32(const double (*As)[kMaxRank + 4], in
       if (a0 + x < R && b0 + y < R) o[(a0 + x) * R + b0 + y] = acc[x][y];
 }
 
-__global__ __launch_bounds__(256) void k_gram_chunks(int64_t I, int R, int ldr, const double *__restrict__ A,
-                                                     double *__restrict__ partials) {
-  __shared__ double As[32][kMaxRank + 4];
-  const int tid = threadIdx.x;
-  const int64_t i0 = (int64_t)blockIdx.x * 32;
-  for (int x = tid; x < 32 * (kMaxRank + 4); x += 256) {
-    const int i = x / (kMaxRank + 4), c = x % (kMaxRank + 4);
-    As[i][c] = (i0 + i < I && c < R) ? A[(i0 + i) * ldr + c] : 0.0;
+// Rows [i0, i0 + 32) of a factor (ldr = 16 NT doubles a row, consecutive) into As, zeros past I
+// and past R: each thread's NT 16-byte loads are in flight together.  The kernels that use it
+// (a few blocks, a few rows each) are bound by such latencies: one element at a time through
+// an index division they waited for each load (800 rows, R = 32 beside the tensor passes:
+// k_gram_chunks 22 -> 12 us, k_nnls_finish 22 -> 14; 100 rows, R = 10: 6.3 -> 4.3, 8.3 -> 5.2).
+template <int NT>
+__device__ __forceinline__ void load_rows32(const double *__restrict__ A, int64_t i0, int64_t I, int R,
+                                            double (*As)[kMaxRank + 4], double *__restrict__ copy) {
+  constexpr int LDR = 16 * NT, H = LDR / 2;
+  f64x2 v[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) {
+    const int e = threadIdx.x + 256 * u, i = e / H, c = 2 * (e % H);
+    v[u] = f64x2{0.0, 0.0};
+    if (i0 + i < I) v[u] = *(const f64x2 *)(A + (i0 + i) * LDR + c);
   }
+#pragma unroll
+  for (int u = 0; u < NT; ++u) {
+    const int e = threadIdx.x + 256 * u, i = e / H, c = 2 * (e % H);
+    if (copy && i0 + i < I) *(f64x2 *)(copy + (i0 + i) * LDR + c) = v[u];
+    As[i][c] = c < R ? v[u][0] : 0.0;
+    As[i][c + 1] = c + 1 < R ? v[u][1] : 0.0;
+  }
+}
+
+template <int NT>
+__global__ __launch_bounds__(256) void k_gram_chunks(int64_t I, int R, const double *__restrict__ A,
+                                                     double *__restrict__ partials) {
+  __shared__ __align__(16) double As[32][kMaxRank + 4];
+  load_rows32<NT>(A, (int64_t)blockIdx.x * 32, I, R, As, nullptr);
   __syncthreads();
-  gram_rows32(As, R, tid, partials + (int64_t)blockIdx.x * R * R);
+  gram_rows32(As, R, threadIdx.x, partials + (int64_t)blockIdx.x * R * R);
+}
+
+// the sum of entry e over the chunk partials, in order, eight loads in flight
+__device__ __forceinline__ double combine_chunks(const double *__restrict__ partials, int e, int RR, int nchunks) {
+  double g = partials[e];
+  int c = 1;
+  for (; c + 8 <= nchunks; c += 8) {
+    double p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = partials[(int64_t)(c + j) * RR + e];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) g = g + p[j];
+  }
+  for (; c < nchunks; ++c) g = g + partials[(int64_t)c * RR + e];
+  return g;
 }
 
 __global__ __launch_bounds__(256) void k_gram_combine(int R, int nchunks, const double *__restrict__ partials,
                                                       double *__restrict__ G) {
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < R * R; e += gridDim.x * blockDim.x) {
-    double g = partials[e];
-    int c = 1;
-    for (; c + 4 <= nchunks; c += 4) {
-      const double p0 = partials[(int64_t)c * R * R + e], p1 = partials[(int64_t)(c + 1) * R * R + e];
-      const double p2 = partials[(int64_t)(c + 2) * R * R + e], p3 = partials[(int64_t)(c + 3) * R * R + e];
-      g = (((g + p0) + p1) + p2) + p3;
-    }
-    for (; c < nchunks; ++c) g = g + partials[(int64_t)c * R * R + e];
-    G[e] = g;
-  }
+  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < R * R; e += gridDim.x * blockDim.x)
+    G[e] = combine_chunks(partials, e, R * R, nchunks);
 }
 
 // With ng > 0 the matrix is first formed as the Hadamard product of the ng Grams in
@@ -221,7 +250,7 @@ __global__ void k_nnls_prep(const NnlsParams *prm, int max_inner, double *betas)
   }
 }
 
-__device__ __forceinline__ int first_common_check(const volatile unsigned long long *mask, int max_inner) {
+__device__ __forceinline__ int first_common_check(const unsigned long long *mask, int max_inner) {
   for (int w = 0; w < 4; ++w) {
     unsigned long long m = mask[w];
     if (m) {
@@ -278,43 +307,36 @@ __device__ __forceinline__ double zero_col_mix(double a, double aold) { return 0
 // k_nnls_select over the rows [32 b, 32 b + 32) of block b, which also leaves the
 // block's partial Gram of the selected rows (k_gram_chunks' association) in
 // partials[b]; k_gram_finish applies the zero-column test and combines.
-__global__ __launch_bounds__(256) void k_nnls_finish(int64_t I, int R, int ldr, const double *__restrict__ hist,
+template <int NT>
+__global__ __launch_bounds__(256) void k_nnls_finish(int64_t I, int R, const double *__restrict__ hist,
                                                      const unsigned long long *__restrict__ mask, int max_inner,
                                                      double *__restrict__ Anew, double *colsum,
                                                      double *__restrict__ partials, NnlsParams *prm) {
-  __shared__ double As[32][kMaxRank + 4];
-  __shared__ unsigned long long mred[256];
-  __shared__ int sk;
+  constexpr int LDR = 16 * NT;
+  __shared__ __align__(16) double As[32][kMaxRank + 4];
+  __shared__ unsigned long long wmask[4][4];
   const int tid = threadIdx.x;
   {
+    // the AND of the blocks' masks, four words each: lane l takes word l % 4 of every 64th
+    // block, the lanes of a wave meet in shuffles, the waves in LDS (one barrier)
     const int64_t nblk = (I + 3) / 4;
     unsigned long long m = ~0ull;
     for (int64_t b = tid >> 2; b < nblk; b += 64) m &= mask[b * 4 + (tid & 3)];
-    mred[tid] = m;
-    __syncthreads();
-    for (int o = 128; o >= 4; o >>= 1) {
-      if (tid < o) mred[tid] &= mred[tid + o];
-      __syncthreads();
-    }
-    if (tid == 0) sk = first_common_check(mred, max_inner);
+#pragma unroll
+    for (int o = 4; o < 64; o <<= 1) m &= __shfl_xor(m, o, 64);
+    if ((tid & 63) < 4) wmask[tid >> 6][tid & 3] = m;
     __syncthreads();
   }
-  const int kstar = sk;
+  unsigned long long all[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) all[w] = ((wmask[0][w] & wmask[1][w]) & wmask[2][w]) & wmask[3][w];
+  const int kstar = first_common_check(all, max_inner);
   if (blockIdx.x == 0 && tid == 0) prm->iters = kstar;
-  const double *src = hist + (int64_t)kstar * I * ldr;
-  const int64_t i0 = (int64_t)blockIdx.x * 32;
-  for (int x = tid; x < 32 * (kMaxRank + 4); x += 256) {
-    const int i = x / (kMaxRank + 4), c = x % (kMaxRank + 4);
-    double v = 0.0;
-    if (i0 + i < I && c < ldr) {
-      v = src[(i0 + i) * ldr + c];
-      Anew[(i0 + i) * ldr + c] = v;
-    }
-    As[i][c] = c < R ? v : 0.0;
-  }
+  load_rows32<NT>(hist + (int64_t)kstar * I * LDR, (int64_t)blockIdx.x * 32, I, R, As, Anew);
   __syncthreads();
   if (tid < R) {
     double cs = 0.0;
+#pragma unroll 8
     for (int i = 0; i < 32; ++i) cs += fabs(As[i][tid]);
     atomicAdd(&colsum[tid], cs);
   }
@@ -329,22 +351,12 @@ __global__ __launch_bounds__(256) void k_gram_finish(int64_t I, int R, int ldr, 
                                                      const double *__restrict__ partials, double *__restrict__ G,
                                                      const double *colsum, const double *Aold, double *A,
                                                      NnlsParams *prm) {
-  double mn = INFINITY;
-  for (int r = 0; r < R; ++r) mn = colsum[r] < mn ? colsum[r] : mn;
-  const bool hit = mn == 0.0;
+  const int lane = threadIdx.x & 63;           // (R <= 64; the column sums are sums of magnitudes)
+  const bool hit = __ballot(lane < R && colsum[lane] == 0.0) != 0ull;
   if (blockIdx.x == 0 && threadIdx.x == 0) prm->fallback = hit;
   if (!hit) {
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < R * R; e += gridDim.x * blockDim.x) {
-      double g = partials[e];
-      int c = 1;
-      for (; c + 4 <= nchunks; c += 4) {
-        const double p0 = partials[(int64_t)c * R * R + e], p1 = partials[(int64_t)(c + 1) * R * R + e];
-        const double p2 = partials[(int64_t)(c + 2) * R * R + e], p3 = partials[(int64_t)(c + 3) * R * R + e];
-        g = (((g + p0) + p1) + p2) + p3;
-      }
-      for (; c < nchunks; ++c) g = g + partials[(int64_t)c * R * R + e];
-      G[e] = g;
-    }
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < R * R; e += gridDim.x * blockDim.x)
+      G[e] = combine_chunks(partials, e, R * R, nchunks);
     return;
   }
   if (blockIdx.x != 0) return;
@@ -581,7 +593,13 @@ void hadamard(hipStream_t s, int R, int ng, const double *const *grams, double *
 
 void gram(hipStream_t s, int64_t I, int R, int ldr, const double *A, double *G, double *partials) {
   const int nchunks = (int)((I + 31) / 32);
-  k_gram_chunks<<<nchunks, 256, 0, s>>>(I, R, ldr, A, partials);
+#define PTN_GC(NTV) \
+  if (ldr == 16 * NTV) k_gram_chunks<NTV><<<nchunks, 256, 0, s>>>(I, R, A, partials)
+  PTN_GC(1);
+  PTN_GC(2);
+  PTN_GC(3);
+  PTN_GC(4);
+#undef PTN_GC
   k_gram_combine<<<(unsigned)((R * R + 63) / 64), 64, 0, s>>>(R, nchunks, partials, G);
 }
 
@@ -621,8 +639,15 @@ void nnls_iterate(hipStream_t s, int64_t I, int R, int ldr, const double *V, con
 void nnls_finish(hipStream_t s, int64_t I, int R, int ldr, const double *hist, const uint64_t *mask, int max_inner,
                  double *A, double *colsum, const double *Aold, double *G, double *partials, NnlsParams *p) {
   const int nchunks = (int)((I + 31) / 32);
-  k_nnls_finish<<<(unsigned)nchunks, 256, 0, s>>>(I, R, ldr, hist, (const unsigned long long *)mask, max_inner, A,
-                                                  colsum, partials, p);
+#define PTN_NF(NTV)                                                                                         \
+  if (ldr == 16 * NTV)                                                                                      \
+  k_nnls_finish<NTV><<<(unsigned)nchunks, 256, 0, s>>>(I, R, hist, (const unsigned long long *)mask, max_inner, A, \
+                                                       colsum, partials, p)
+  PTN_NF(1);
+  PTN_NF(2);
+  PTN_NF(3);
+  PTN_NF(4);
+#undef PTN_NF
   k_gram_finish<<<(unsigned)((R * R + 255) / 256), 256, 0, s>>>(I, R, ldr, nchunks, partials, G, colsum, Aold, A, p);
 }
 
