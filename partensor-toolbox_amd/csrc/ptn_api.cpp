@@ -53,6 +53,7 @@ struct ptn_handle_s {
   int64_t total = 0;
   double *x64 = nullptr;
   float *x32 = nullptr;
+  size_t x64_bytes = 0, x32_bytes = 0;       // of the pool's blocks that hold the tensor
   double *scal = nullptr;    // device scalars: [0] ||X||^2, [1..] scratch
   double *part = nullptr;    // reduction partials for norms
   bool frob_valid = false;
@@ -264,6 +265,7 @@ struct EventPair {                           // two timing-free events, destroye
 };
 
 ptn_status run(ptn_handle h, const std::function<void()> &fn);
+void drop_tensor(ptn_handle h);
 
 // ------------------------------------------------------------------------------------
 // the warm-start network: parameters, Adam state, training set, activations
@@ -1064,8 +1066,7 @@ void ptn_destroy(ptn_handle h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   if (h->side) (void)hipStreamSynchronize(h->side);
   if (h->aux) (void)hipStreamSynchronize(h->aux);
-  if (h->x64) (void)hipFree(h->x64);
-  if (h->x32) (void)hipFree(h->x32);
+  drop_tensor(h);
   delete h->batch;
   delete h->mlp;
   give_back_spent(h);
@@ -1119,11 +1120,17 @@ ptn_status run(ptn_handle h, const std::function<void()> &fn) {
   }
 }
 
+void drop_tensor(ptn_handle h) {
+  if (h->x64) pool_give(h->device, h->x64, h->x64_bytes);
+  if (h->x32) pool_give(h->device, h->x32, h->x32_bytes);
+  h->x64 = nullptr;
+  h->x32 = nullptr;
+}
+
 void alloc_tensor(ptn_handle h, int N, const int64_t *dims, int storage) {
   REQUIRE(storage >= 1 && storage <= 3, PTN_ERR_INVALID, "storage must be F64, F32 or BOTH");
   check_dims(h, N, dims);
-  if (h->x64) { HIPCHK(hipFree(h->x64)); h->x64 = nullptr; }
-  if (h->x32) { HIPCHK(hipFree(h->x32)); h->x32 = nullptr; }
+  drop_tensor(h);                             // (the calls that read it have waited for their streams)
   h->N = N;
   for (int k = 0; k < N; ++k) h->dims[k] = dims[k];
   h->total = prod(dims, N);
@@ -1131,11 +1138,11 @@ void alloc_tensor(ptn_handle h, int N, const int64_t *dims, int storage) {
   // kTensorPad zero elements after the tensor: the contiguous-K contractions read whole
   // 32-element steps, which may run past the end of the last fiber
   if (storage & PTN_TENSOR_F64) {
-    HIPCHK(device_malloc(h->device, (void **)&h->x64, (h->total + kTensorPad) * sizeof(double)));
+    HIPCHK(pool_take(h->device, pool_size((h->total + kTensorPad) * sizeof(double)), (void **)&h->x64, &h->x64_bytes));
     HIPCHK(hipMemsetAsync(h->x64 + h->total, 0, kTensorPad * sizeof(double), h->stream));
   }
   if (storage & PTN_TENSOR_F32) {
-    HIPCHK(device_malloc(h->device, (void **)&h->x32, (h->total + kTensorPad) * sizeof(float)));
+    HIPCHK(pool_take(h->device, pool_size((h->total + kTensorPad) * sizeof(float)), (void **)&h->x32, &h->x32_bytes));
     HIPCHK(hipMemsetAsync(h->x32 + h->total, 0, kTensorPad * sizeof(float), h->stream));
   }
 }
