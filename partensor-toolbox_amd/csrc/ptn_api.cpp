@@ -450,7 +450,9 @@ struct Work {
     nscr.alloc(h, 2 * kMaxOrder * kMaxRank, kRaw); scal.alloc(h, 8, kRaw);
     betas.alloc(h, (size_t)(N + 1) * (kMaxInner + 1), kRaw);
     gpart.alloc(h, (size_t)((maxI + 31) / 32) * R * R, kRaw);
-    gpart_side.alloc(h, (size_t)((maxI + 31) / 32) * R * R, kRaw);
+    int64_t chunks = 0;
+    for (int k = 0; k < N; ++k) chunks += (dims[k] + 31) / 32;
+    gpart_side.alloc(h, (size_t)chunks * R * R, kRaw);
     cscr.alloc(h, (size_t)3 * R * R + R, kRaw);    // R x R work of the unconstrained / orthogonality updates
     const int64_t C = total / dims[0];
     const int64_t yl = left_rows();
@@ -1419,16 +1421,19 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
           if (side_cost)
             cost_gram(ss, w.dims[last] * w.ldr, w.M, w.F(last), R, sel[last].V, w.G(last), w.scal.p, w.scal.p + 1, 0);
           if (pair) prep_mode(w, w.grams, 0, tree, slot(w, 0), o, ss);
-          for (int k = 0; k < N; ++k)
-            gram(ss, w.dims[k], R, w.ldr, w.Fb(w.acc, k), w.agr.p + (int64_t)k * R * R, w.gpart_side);
-          if (pair) prep_mode(w, w.agr, 0, tree, slot(w, N), o, ss);
-          // accel_cost_function (CpdDimTree.hpp:174-181): its fit term from the last mode's
-          // MTTKRP, or from mode 0 of the paired left-node pass
+          // the accelerated factors' Grams and V_hat of accel_cost_function
+          // (CpdDimTree.hpp:174-181): its fit term from the last mode's MTTKRP, or from mode 0
+          // of the paired left-node pass
           int list[kMaxOrder];
-          int nl = v_order(N, cm, false, list);
-          const double *gp[kMaxOrder];
-          for (int j = 0; j < nl; ++j) gp[j] = w.agr.p + (int64_t)list[j] * R * R;
-          hadamard(ss, R, nl, gp, w.Vacc);
+          const int nl = v_order(N, cm, false, list);
+          const double *ap[kMaxOrder];
+          double *gp[kMaxOrder];
+          for (int k = 0; k < N; ++k) {
+            ap[k] = w.Fb(w.acc, k);
+            gp[k] = w.agr.p + (int64_t)k * R * R;
+          }
+          grams_all(ss, N, w.dims, R, w.ldr, ap, gp, nl, list, w.Vacc, w.gpart_side);
+          if (pair) prep_mode(w, w.agr, 0, tree, slot(w, N), o, ss);
           join();                    // the side stream has finished with the Grams, V_hat and slots
           cost_gram(ms, w.dims[cm] * w.ldr, mfit, w.Fb(w.acc, cm), R, w.Vacc, w.agr.p + (int64_t)cm * R * R,
                     w.scal.p, w.scal.p + 2, 1);

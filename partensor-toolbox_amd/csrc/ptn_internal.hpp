@@ -222,6 +222,10 @@ void reduce_splits_f32(hipStream_t s, const float *partials, int splits, int64_t
 void hadamard(hipStream_t s, int R, int ng, const double *const *grams, double *V);
 // partials: ceil(I/32) x R x R doubles
 void gram(hipStream_t s, int64_t I, int R, int ldr, const double *A, double *G, double *partials);
+// the Grams G[k] of all N factors A[k] (dims[k] rows) and V = the Hadamard product of the ng listed
+// ones in list order; partials: R x R for every 32 rows of every factor
+void grams_all(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *const *A, double *const *G,
+               int ng, const int *list, double *V, double *partials);
 void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p);
 // V = Hadamard of the ng Grams (list order), its extreme eigenvalues with GLambda, and
 // the max_inner momentum coefficients: everything an NNLS update needs besides M.

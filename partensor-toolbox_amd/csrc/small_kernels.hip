@@ -118,6 +118,47 @@ __global__ __launch_bounds__(256) void k_gram_combine(int R, int nchunks, const 
     G[e] = combine_chunks(partials, e, R * R, nchunks);
 }
 
+// The Grams of all factors and the Hadamard product of some of them (the line search's: A_hat's
+// Grams and V_hat) in two launches: block b sums one 32-row chunk of one factor, then wave k
+// of a block combines 64 entries of factor k's Gram in k_gram_combine's order and the first
+// wave multiplies the ng listed ones in list order (k_hadamard's).  Two launches per factor
+// and one for the product kept the line search of small tensors waiting for the side stream
+// (100^3, R = 10, 50 sweeps 14.7 -> 13.8 ms).
+struct GramBatch {
+  int N, ng;
+  int64_t I[kMaxOrder];
+  int chunk0[kMaxOrder + 1];                   // first chunk of each factor, then their number
+  const double *A[kMaxOrder];
+  double *G[kMaxOrder];
+  int list[kMaxOrder];
+};
+template <int NT>
+__global__ __launch_bounds__(256) void k_gram_chunks_all(GramBatch b, int R, double *__restrict__ partials) {
+  __shared__ __align__(16) double As[32][kMaxRank + 4];
+  int k = 0;
+  while (k + 1 < b.N && (int)blockIdx.x >= b.chunk0[k + 1]) ++k;
+  load_rows32<NT>(b.A[k], (int64_t)((int)blockIdx.x - b.chunk0[k]) * 32, b.I[k], R, As, nullptr);
+  __syncthreads();
+  gram_rows32(As, R, threadIdx.x, partials + (int64_t)blockIdx.x * R * R);
+}
+__global__ __launch_bounds__(64 * kMaxOrder) void k_gram_combine_all(GramBatch b, int R,
+                                                                     const double *__restrict__ partials,
+                                                                     double *__restrict__ V) {
+  __shared__ double g[kMaxOrder][64];
+  const int lane = threadIdx.x & 63, k = threadIdx.x >> 6, e = blockIdx.x * 64 + lane;
+  if (e < R * R) {
+    const double v = combine_chunks(partials + (int64_t)b.chunk0[k] * R * R, e, R * R, b.chunk0[k + 1] - b.chunk0[k]);
+    b.G[k][e] = v;
+    g[k][lane] = v;
+  }
+  __syncthreads();
+  if (k == 0 && e < R * R) {
+    double v = g[b.list[0]][lane];
+    for (int j = 1; j < b.ng; ++j) v = g[b.list[j]][lane] * v;
+    V[e] = v;
+  }
+}
+
 // With ng > 0 the matrix is first formed as the Hadamard product of the ng Grams in
 // list order (V = G_l0, V = G_lj * V; PartialCwiseProd) and stored to Vout; with
 // betas != nullptr the momentum coefficients of the Nesterov solve follow the
@@ -601,6 +642,28 @@ void gram(hipStream_t s, int64_t I, int R, int ldr, const double *A, double *G, 
   PTN_GC(4);
 #undef PTN_GC
   k_gram_combine<<<(unsigned)((R * R + 63) / 64), 64, 0, s>>>(R, nchunks, partials, G);
+}
+
+void grams_all(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *const *A, double *const *G,
+               int ng, const int *list, double *V, double *partials) {
+  GramBatch b{};
+  b.N = N;
+  b.ng = ng;
+  for (int k = 0; k < N; ++k) {
+    b.I[k] = dims[k];
+    b.A[k] = A[k];
+    b.G[k] = G[k];
+    b.chunk0[k + 1] = b.chunk0[k] + (int)((dims[k] + 31) / 32);
+  }
+  for (int j = 0; j < ng; ++j) b.list[j] = list[j];
+#define PTN_GA(NTV) \
+  if (ldr == 16 * NTV) k_gram_chunks_all<NTV><<<(unsigned)b.chunk0[N], 256, 0, s>>>(b, R, partials)
+  PTN_GA(1);
+  PTN_GA(2);
+  PTN_GA(3);
+  PTN_GA(4);
+#undef PTN_GA
+  k_gram_combine_all<<<(unsigned)((R * R + 63) / 64), 64 * N, 0, s>>>(b, R, partials, V);
 }
 
 void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p) {
