@@ -813,6 +813,14 @@ void left_node_pair(Work &w, double *cur, double *acc) {
   w.m0_ready = true;
 }
 
+// The main and side streams exchanged while the scope lasts: what is enqueued on the main stream
+// goes to the side stream.
+struct StreamsSwapped {
+  ptn_handle h;
+  explicit StreamsSwapped(ptn_handle hh) : h(hh) { std::swap(h->stream, h->side); }
+  ~StreamsSwapped() { std::swap(h->stream, h->side); }
+};
+
 // Hadamard order of V_n: ascending (PartialCwiseProd, right-nested) for the standard
 // form; the tree path order (TreeMode_N_Product / TTVs_util) for the dimension tree.
 int v_order(int N, int mode, bool tree, int *list) {
@@ -1280,7 +1288,8 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
     HIPCHK(hipStreamSynchronize(h->stream));
 
     // The side stream forms V_n, its eigenvalues and the momentum coefficients of mode n
-    // while the main stream contracts the tensor for mode n; during the line-search pass
+    // while the main stream contracts the tensor for mode n (small tensors: the other way
+    // round, eig_first below); during the line-search pass
     // it also forms the accelerated factors' Grams, V_hat, the sweep's cost and both
     // mode-0 set-ups of the next sweep.  The aux stream forms the order-3 tree's right node
     // (right_node_early).  All three run at the default priority.
@@ -1346,24 +1355,41 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
       // the last factor and its Gram as they are unless it is the weight factor)
       const bool side_cost = step_now && pair && !(o.normalization && !all_orth && wf == last);
       const bool early_right = tree && w.mfma32 && N == 3;
+      // A tensor that is read in less time than the eigen routine takes (28, 65 and 150 us at
+      // the three padded ranks; a contraction reads about 4.5 TB/s): the set-up, then the longer
+      // of the two, follows the Gram on the main stream, and the contraction crosses to the side
+      // stream and back beside it, so neither hop is waited for.  Sweeps per this and the other
+      // order: 100^3 R = 10 229 / 269 us, 200^3 R = 20 342 / 375, 400^3 R = 64 (512 MB) 1232 /
+      // 1452; 300^3 R = 16 (216 MB) 394 / 387, 400^3 R = 16 635 / 598.
+      const int64_t eig_bytes = (int64_t)(R <= 16 ? 128 : R <= 32 ? 288 : 640) << 20;
+      const bool short_read = !early_right && w.total * (w.f32 ? 4 : 8) <= eig_bytes;
       for (int n = 0; n < N; ++n) {
-        if (!(n == 0 && prepped0)) {
+        const bool set_up = !(n == 0 && prepped0);
+        const bool eig_first = short_read && o.constraints[n] == PTN_NONNEGATIVITY;
+        auto contract = [&] {
+          if (tree) mttkrp_tree(w, w.fac, n, w.M);
+          else mttkrp_standard(w, w.fac, n, w.M);
+        };
+        if (set_up) {
           sel[n] = slot(w, n);
           fork();
-          prep_mode(w, w.grams, n, tree, sel[n], o, ss);
+          prep_mode(w, w.grams, n, tree, sel[n], o, eig_first ? ms : ss);
         }
-        // mode 1's set-up is queued on the side stream before the right node on the third,
-        // so that its eigen wave starts before the right node's blocks fill the CUs; the
-        // third stream waits on the fork's event (only the side stream was fed since)
-        if (n == 1 && early_right) right_node_early(w, w.fac, h->ev[0]);
-        // mode 2's set-up ends on the side stream before the right node on the third, so
-        // the main stream joins the side stream before it waits for the right node: both
-        // waits then pass before the leaf contraction instead of one on each side of it
-        const bool join_early = n == 2 && early_right;
-        if (join_early) join();
-        if (tree) mttkrp_tree(w, w.fac, n, w.M);
-        else mttkrp_standard(w, w.fac, n, w.M);
-        if (!(n == 0 && prepped0) && !join_early) join();   // mode 0: joined after the line-search pass
+        if (set_up && eig_first) {
+          StreamsSwapped swapped(h);
+          contract();
+        } else {
+          // mode 1's set-up is queued on the side stream before the right node on the third,
+          // so that its eigen wave starts before the right node's blocks fill the CUs; the
+          // third stream waits on the fork's event (only the side stream was fed since)
+          if (n == 1 && early_right) right_node_early(w, w.fac, h->ev[0]);
+          // mode 2's set-up ends on the side stream before the right node on the third, so
+          // the main stream joins the side stream before it waits for the right node: both
+          // waits then pass before the leaf contraction instead of one on each side of it
+          if (n == 2 && early_right) join();
+          contract();
+        }
+        if (set_up && !(n == 2 && early_right)) join();   // mode 0: joined after the line-search pass
         update_factor(w, n, o, sel[n]);
         if (n == last && !side_cost)
           cost_gram(ms, w.dims[last] * w.ldr, w.M, w.F(last), R, sel[last].V, w.G(last), w.scal.p, w.scal.p + 1, 0);
