@@ -601,7 +601,7 @@ __device__ __forceinline__ void sweep_problem(const BatchArgs &a, int p, int g, 
       PTN_WAVE_SYNC();
       double amax, amin;
       eig_extremes_wave<kBR>(R, S.eig, amax, amin);
-      if (l == 0) glambda_betas(amax, amin, &S.prm, a.max_inner, S.betas);
+      glambda_betas(amax, amin, &S.prm, a.max_inner, S.betas);
     };
     const int In = n == 0 ? I0 : n == 1 ? I1 : I2;
     // FP64 matrix cores: the eigen wave (R <= 16: microseconds) then takes 3/4 of an MTTKRP

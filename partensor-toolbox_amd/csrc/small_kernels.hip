@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void k_eig_extremes(int R, const double *__res
   __syncthreads();
   double amax, amin;
   eig_extremes_block<RB>(n, S, part, amax, amin);
-  if (threadIdx.x == 0) glambda_betas(amax, amin, prm, max_inner, betas);
+  if (threadIdx.x < 64) glambda_betas(amax, amin, prm, max_inner, betas);
 }
 
 
@@ -280,15 +280,7 @@ __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr,
 
 // Momentum coefficients beta_k of NesterovMNLS.hpp:222-223 (shared by every row).
 __global__ void k_nnls_prep(const NnlsParams *prm, int max_inner, double *betas) {
-  if (threadIdx.x == 0) {
-    const double q = prm->q;
-    double alpha = 1.0;
-    for (int k = 0; k < max_inner; ++k) {
-      const double na = update_alpha(alpha, q);
-      betas[k] = alpha * (1.0 - alpha) / (alpha * alpha + na);
-      alpha = na;
-    }
-  }
+  momentum_wave(prm->q, max_inner, betas);
 }
 
 __device__ __forceinline__ int first_common_check(const unsigned long long *mask, int max_inner) {
