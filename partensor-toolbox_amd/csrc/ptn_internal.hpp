@@ -226,13 +226,13 @@ void gram(hipStream_t s, int64_t I, int R, int ldr, const double *A, double *G, 
 // ones in list order; partials: R x R for every 32 rows of every factor
 void grams_all(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *const *A, double *const *G,
                int ng, const int *list, double *V, double *partials);
-void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p);
+// extreme singular values of V, GLambda and (betas != nullptr) the momentum coefficients
+void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p, int max_inner, double *betas);
 // V = Hadamard of the ng Grams (list order), its extreme eigenvalues with GLambda, and
 // the max_inner momentum coefficients: everything an NNLS update needs besides M.
 void nnls_setup(hipStream_t s, int R, int ng, const double *const *grams, double *V, NnlsParams *p, int max_inner,
                 double *betas);
 // betas: max_inner doubles
-void nnls_prep(hipStream_t s, const NnlsParams *p, int max_inner, double *betas);
 // satisfaction masks of nnls_iterate: 4 words per block of 4 rows
 inline int64_t nnls_mask_words(int64_t I) { return (I + 3) / 4 * 4; }
 // hist: (max_inner + 1) x I x ldr doubles; mask: nnls_mask_words(I) words

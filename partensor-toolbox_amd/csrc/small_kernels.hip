@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void k_eig_extremes(int R, const double *__res
 // (NesterovMNLS.hpp:217) at every check; the row's mask is the AND over its lanes
 // (max |G.Y| <= d1 and min G >= -d2 hold iff they hold entry-wise).  Iterate A_k goes
 // to hist[k]; the common stopping point is selected afterwards.  The momentum
-// coefficients depend only on q and come precomputed (k_nnls_prep).
+// coefficients depend only on q and come precomputed (momentum_wave).
 template <int RB>
 __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr, const double *__restrict__ V,
                                                       const NnlsParams *__restrict__ prm,
@@ -276,11 +276,6 @@ __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr,
     if (max_inner < lo + 64) m |= (max_inner <= lo) ? ~0ull : (~0ull << (max_inner - lo));
     mask[(int64_t)blockIdx.x * 4 + w] = m;
   }
-}
-
-// Momentum coefficients beta_k of NesterovMNLS.hpp:222-223 (shared by every row).
-__global__ void k_nnls_prep(const NnlsParams *prm, int max_inner, double *betas) {
-  momentum_wave(prm->q, max_inner, betas);
 }
 
 __device__ __forceinline__ int first_common_check(const unsigned long long *mask, int max_inner) {
@@ -658,11 +653,11 @@ void grams_all(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const 
   k_gram_combine_all<<<(unsigned)((R * R + 63) / 64), 64 * N, 0, s>>>(b, R, partials, V);
 }
 
-void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p) {
+void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p, int max_inner, double *betas) {
   const GramPtrs G{};
-  if (R <= 16) k_eig_extremes<16><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, 0, nullptr);
-  else if (R <= 32) k_eig_extremes<32><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, 0, nullptr);
-  else k_eig_extremes<64><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, 0, nullptr);
+  if (R <= 16) k_eig_extremes<16><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
+  else if (R <= 32) k_eig_extremes<32><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
+  else k_eig_extremes<64><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
 }
 
 void nnls_setup(hipStream_t s, int R, int ng, const double *const *grams, double *V, NnlsParams *p, int max_inner,
@@ -672,10 +667,6 @@ void nnls_setup(hipStream_t s, int R, int ng, const double *const *grams, double
   if (R <= 16) k_eig_extremes<16><<<1, 256, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
   else if (R <= 32) k_eig_extremes<32><<<1, 256, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
   else k_eig_extremes<64><<<1, 256, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
-}
-
-void nnls_prep(hipStream_t s, const NnlsParams *p, int max_inner, double *betas) {
-  k_nnls_prep<<<1, 64, 0, s>>>(p, max_inner, betas);
 }
 
 void nnls_iterate(hipStream_t s, int64_t I, int R, int ldr, const double *V, const NnlsParams *p,
