@@ -755,6 +755,30 @@ def test_zero_column_fallback_on_gpu(h, dims):
     assert stg["f_value"] == pytest.approx(sto["f_value"], rel=1e-12)
 
 
+@pytest.mark.parametrize("R", [3, 17, 33, 49])
+@pytest.mark.parametrize("dims", [[1, 31, 32], [33, 128, 129], [255, 256, 257], [300, 5, 4]])
+def test_update_finish_at_the_row_chunks_edges(h, dims, R):
+    """The end of an update (the stopping iterate, the zero-column test, the Gram) for row counts
+    about the 32-row chunks and the eight partial sums added at a time, at every padded rank; a
+    tensor with its sign turned takes the zero-column mix, upright it does where the oracle does.
+    Against the oracle: the MTTKRPs
+    agree to rounding, the rest operation by operation, so the factors within 1e-10."""
+    rng = np.random.default_rng(R)
+    A = [rng.random((I, 2)) for I in dims]
+    init = [rng.random((I, R)) for I in dims]
+    kw = dict(max_iter=2, threshold_error=0.0, normalization=0, acceleration=0)
+    for sign in (1.0, -1.0):
+        X = sign * o.cp_full(A)
+        h.set_tensor(X)
+        Fg, _, logg = h.cpd(R, init, **kw)
+        Fo, _, logo = o.cpd(X, R, init, cost_form=o.COST_GRAM, **kw)
+        assert [l["zero_col_fallback"] for l in logg] == [l["zero_col_fallback"] for l in logo]
+        assert [l["nnls_iters"] for l in logg] == [l["nnls_iters"] for l in logo]
+        assert sign > 0 or logg[0]["zero_col_fallback"][0] == 1
+        for a, b in zip(Fg, Fo):
+            assert P.rel_err(a, b) <= 1e-10
+
+
 def test_invalid_arguments_raise(h):
     say("error paths")
     h.set_tensor(np.ones((4, 5, 6), order="F"))
