@@ -12,65 +12,133 @@ namespace ptn {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------------------
 // C[m][n] = sum_k A[m][k] B[n][k] (+ bias[n]) (* (gate[m][n] > 0)) (ReLU), both operands
-// bf16 with k contiguous (K a multiple of 16, leading dimensions multiples of 8).  Each
-// wave owns a 32 x 32 tile; lane (i, kg) loads the 16-byte k-slices A[m0+i][k+8kg..] and
-// B[n0+i][k+8kg..] straight into its MFMA fragments.  Rows / columns past M / N read a
-// clamped row and are not stored.
+// bf16 with k contiguous (K a multiple of 16, leading dimensions multiples of 8).  A block
+// is one wave with a 32 x 32 tile.  Rows / columns past M / N read a clamped row and are
+// not stored.  Cbt: a transposed copy of the bf16 result (ldcbt a multiple of 4), so that
+// the weight gradients find their operands k-contiguous.
+//
+// The layers are small, so neither the matrix cores nor the memory bound them but a wave's
+// loads: fetching the fragments where they lie takes 64 cache lines for each load, and four
+// waves to a block left three CUs in four idle at 1024 rows.  So a wave fetches 128 k of its
+// 64 rows with sixteen lanes to a row, two such groups in flight, and takes the fragments from
+// LDS (rows 272 bytes apart: sixteen rows lie in different banks).  Average over the eight
+// products of a step of 1024 rows: 15.0 us, with the two groups but fragments fetched where they
+// lie 14.1 us, so 8.9 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_gemm_nt(int M, int N, int K, const __bf16 *__restrict__ A, int lda,
-                                                 const __bf16 *__restrict__ B, int ldb, const float *__restrict__ bias,
-                                                 const __bf16 *__restrict__ gate, int ldg, int relu,
-                                                 float *__restrict__ C, int ldc, __bf16 *__restrict__ Cb, int ldcb) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane & 31, kg = lane >> 5;
-  const int m0 = blockIdx.y * 64 + 32 * (wave >> 1), n0 = blockIdx.x * 64 + 32 * (wave & 1);
-  if (m0 >= M || n0 >= N) return;                       // no block-wide barrier below
-  const int ma = m0 + i < M ? m0 + i : M - 1, nb = n0 + i < N ? n0 + i : N - 1;
-  const bf16x8 *pa = (const bf16x8 *)(A + (int64_t)ma * lda + 8 * kg);
-  const bf16x8 *pb = (const bf16x8 *)(B + (int64_t)nb * ldb + 8 * kg);
+__global__ __launch_bounds__(64) void k_gemm_nt(int M, int N, int K, const __bf16 *__restrict__ A, int lda,
+                                                const __bf16 *__restrict__ B, int ldb, const float *__restrict__ bias,
+                                                const __bf16 *__restrict__ gate, int ldg, int relu,
+                                                float *__restrict__ C, int ldc, __bf16 *__restrict__ Cb, int ldcb,
+                                                __bf16 *__restrict__ Cbt, int ldcbt) {
+  constexpr int KG = 128, LD = KG + 8;
+  __shared__ __align__(16) __bf16 tile[64 * LD];         // 32 rows of A, 32 of B
+  const int lane = threadIdx.x, i = lane & 31, kg = lane >> 5;
+  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+  const int fr = lane >> 4, fc = 8 * (lane & 15);        // fetching: row within four, first column
+  const __bf16 *pa[8], *pb[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int m = m0 + 4 * q + fr, n = n0 + 4 * q + fr;
+    pa[q] = A + (int64_t)(m < M ? m : M - 1) * lda;
+    pb[q] = B + (int64_t)(n < N ? n : N - 1) * ldb;
+  }
+  struct Rows {
+    bf16x8 a[8], b[8];
+  };
+  auto load = [&](int k, Rows &f) {
+    const int c = k + fc < K ? k + fc : 0;               // a column past K: read, never used
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      f.a[q] = *(const bf16x8 *)(pa[q] + c);
+      f.b[q] = *(const bf16x8 *)(pb[q] + c);
+    }
+  };
   f32x16 acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-  int k = 0;
-  for (; k + 32 <= K; k += 32) {
-    const bf16x8 a0 = pa[k / 8], b0 = pb[k / 8], a1 = pa[k / 8 + 2], b1 = pb[k / 8 + 2];
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, acc, 0, 0, 0);
+  auto mul = [&](int k, const Rows &f, Rows &next) {     // then group k + 2 KG into next
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      *(bf16x8 *)(tile + (4 * q + fr) * LD + fc) = f.a[q];
+      *(bf16x8 *)(tile + (32 + 4 * q + fr) * LD + fc) = f.b[q];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (k + 2 * KG < K) load(k + 2 * KG, next);
+    const __bf16 *ta = tile + i * LD + 8 * kg, *tb = ta + 32 * LD;
+    const int nu = K - k < KG ? (K - k) / 16 : KG / 16;
+#pragma unroll
+    for (int u = 0; u < KG / 16; ++u)
+      if (u < nu)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(ta + 16 * u), *(const bf16x8 *)(tb + 16 * u),
+                                                      acc, 0, 0, 0);
+  };
+  Rows f0, f1;
+  load(0, f0);
+  if (KG < K) load(KG, f1);
+  for (int k = 0; k < K; k += 2 * KG) {
+    mul(k, f0, f0);
+    if (k + KG < K) mul(k + KG, f1, f1);
   }
-  for (; k < K; k += 16) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[k / 8], pb[k / 8], acc, 0, 0, 0);
   const int n = n0 + i;
   if (n >= N) return;
   const float bn = bias ? bias[n] : 0.f;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int m = m0 + 8 * (v / 4) + 4 * kg + (v % 4);
-    if (m < M) {
-      float x = acc[v] + bn;
-      if (gate && !((float)gate[(int64_t)m * ldg + n] > 0.f)) x = 0.f;
-      if (relu) x = x > 0.f ? x : 0.f;
-      if (C) C[(int64_t)m * ldc + n] = x;
-      if (Cb) Cb[(int64_t)m * ldcb + n] = (__bf16)x;
+  for (int q = 0; q < 4; ++q) {
+    bf16x4 t4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + 8 * q + 4 * kg + r;
+      float x = acc[4 * q + r] + bn;
+      if (m < M) {
+        if (gate && !((float)gate[(int64_t)m * ldg + n] > 0.f)) x = 0.f;
+        if (relu) x = x > 0.f ? x : 0.f;
+        if (C) C[(int64_t)m * ldc + n] = x;
+        if (Cb) Cb[(int64_t)m * ldcb + n] = (__bf16)x;
+      }
+      t4[r] = (__bf16)x;
     }
+    // (M is a multiple of 4 wherever a transposed copy is asked for)
+    if (Cbt && m0 + 8 * q + 4 * kg < M) *(bf16x4 *)(Cbt + (int64_t)n * ldcbt + m0 + 8 * q + 4 * kg) = t4;
   }
 }
 
-// out[c][r] = in[r][c] (bf16), 32 x 32 tiles through LDS
-__global__ __launch_bounds__(256) void k_transpose_bf16(int rows, int cols, const __bf16 *__restrict__ in, int ldi,
-                                                        __bf16 *__restrict__ out, int ldo) {
+// Several transposes in one launch (an epoch of 8192 rows in batches of 1024: eight launches of
+// 4.7 us a step; the layers' own results are written transposed by their products): out[c][r] = in[r][c] (bf16), 32 x 32 tiles through LDS;
+// block b belongs to the matrix whose tiles start at or before b.
+struct Transposes {
+  int n;
+  int first[5];                                         // first tile of each matrix, then their number
+  int rows[4], cols[4], ldi[4], ldo[4];
+  const __bf16 *in[4];
+  __bf16 *out[4];
+};
+__global__ __launch_bounds__(256) void k_transposes(Transposes T) {
   __shared__ __bf16 t[32][33];
-  const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  int w = 0;
+  while (w + 1 < T.n && (int)blockIdx.x >= T.first[w + 1]) ++w;
+  const int tile = blockIdx.x - T.first[w], tc = (T.cols[w] + 31) / 32;
+  const int r0 = tile / tc * 32, c0 = tile % tc * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int rows = T.rows[w], cols = T.cols[w];
+  const __bf16 *in = T.in[w];
+  __bf16 *out = T.out[w];
+#pragma unroll
   for (int y = ty; y < 32; y += 8) {
     const int r = r0 + y, c = c0 + tx;
-    t[y][tx] = (r < rows && c < cols) ? in[(int64_t)r * ldi + c] : (__bf16)0.f;
+    t[y][tx] = (r < rows && c < cols) ? in[(int64_t)r * T.ldi[w] + c] : (__bf16)0.f;
   }
   __syncthreads();
+#pragma unroll
   for (int y = ty; y < 32; y += 8) {
     const int c = c0 + y, r = r0 + tx;
-    if (c < cols && r < rows) out[(int64_t)c * ldo + r] = t[tx][y];
+    if (c < cols && r < rows) out[(int64_t)c * T.ldo[w] + r] = t[tx][y];
   }
 }
 
@@ -212,7 +280,8 @@ __global__ __launch_bounds__(256) void k_mse_grad(int B, const float *__restrict
 // loads, one row each, and leave them column by column in LDS, where 16 lanes walk their columns
 // four rows per read while the next 256 rows are on their way.  One thread per column reading
 // its rows from memory one by one waited for every load: 1024 rows of 256 columns 224 us, here
-// 6.4 us (an epoch of 8192 rows in batches of 1024: 7.2 -> 1.9 ms).  Rows past M enter as +0, which leaves a sum that starts at +0 as it is.
+// 6.4 us (an epoch of 8192 rows in batches of 1024: 7.2 -> 1.9 ms).  Rows past M enter as +0,
+// which leaves a sum that starts at +0 as it is.
 template <typename TG>
 __global__ __launch_bounds__(256) void k_colsum(int M, const TG *__restrict__ G, int ldg, float *__restrict__ out) {
   constexpr int LD = 256 + 4;                   // 16 lanes x 16-byte reads touch every bank once
@@ -299,15 +368,25 @@ __global__ __launch_bounds__(256) void k_gather(int B, const int *__restrict__ i
 }  // namespace
 
 void gemm_nt(hipStream_t s, int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *bias,
-             const void *gate, int ldg, int relu, float *C, int ldc, void *Cb, int ldcb) {
-  dim3 grid((N + 63) / 64, (M + 63) / 64);
-  k_gemm_nt<<<grid, 256, 0, s>>>(M, N, K, (const __bf16 *)A, lda, (const __bf16 *)B, ldb, bias, (const __bf16 *)gate,
-                                 ldg, relu, C, ldc, (__bf16 *)Cb, ldcb);
+             const void *gate, int ldg, int relu, float *C, int ldc, void *Cb, int ldcb, void *Cbt, int ldcbt) {
+  dim3 grid((N + 31) / 32, (M + 31) / 32);
+  k_gemm_nt<<<grid, 64, 0, s>>>(M, N, K, (const __bf16 *)A, lda, (const __bf16 *)B, ldb, bias, (const __bf16 *)gate,
+                                 ldg, relu, C, ldc, (__bf16 *)Cb, ldcb, (__bf16 *)Cbt, ldcbt);
 }
 
-void transpose_bf16(hipStream_t s, int rows, int cols, const void *in, int ldi, void *out, int ldo) {
-  dim3 grid((cols + 31) / 32, (rows + 31) / 32);
-  k_transpose_bf16<<<grid, 256, 0, s>>>(rows, cols, (const __bf16 *)in, ldi, (__bf16 *)out, ldo);
+void transposes_bf16(hipStream_t s, int n, const TransposeBf16 *m) {
+  Transposes T{};
+  T.n = n;
+  for (int w = 0; w < n; ++w) {
+    T.rows[w] = m[w].rows;
+    T.cols[w] = m[w].cols;
+    T.ldi[w] = m[w].cols;
+    T.ldo[w] = m[w].rows;
+    T.in[w] = (const __bf16 *)m[w].in;
+    T.out[w] = (__bf16 *)m[w].out;
+    T.first[w + 1] = T.first[w] + (m[w].rows + 31) / 32 * ((m[w].cols + 31) / 32);
+  }
+  k_transposes<<<T.first[n], 256, 0, s>>>(T);
 }
 
 void mlp_features(hipStream_t s, int64_t I, int R, int ldr, const double *V, const double *M, const double *A,

@@ -335,35 +335,37 @@ struct MlpState {
     dx.swap(nx); dt.swap(nt); drank.swap(nr);
     cap = nc;
   }
-  // Y = network(X) for B rows (activations kept for the backward pass)
-  void forward(hipStream_t s, int B) {
+  // Y = network(X) for B rows; back (B a multiple of 32): the activations are kept for the
+  // backward pass, upright and transposed
+  void forward(hipStream_t s, int B, bool back) {
     gemm_nt(s, B, kMlpH, kMlpIn, X.p, kMlpIn, wb.p + kMlpW1b, kMlpIn, w.p + kMlpB1, nullptr, 0, 1, nullptr, 0, H1.p,
-            kMlpH);
+            kMlpH, back ? H1T.p : nullptr, B);
     gemm_nt(s, B, kMlpH, kMlpH, H1.p, kMlpH, wb.p + kMlpW2b, kMlpH, w.p + kMlpB2, nullptr, 0, 1, nullptr, 0, H2.p,
-            kMlpH);
+            kMlpH, back ? H2T.p : nullptr, B);
     gemm_nt(s, B, kMlpR, kMlpH, H2.p, kMlpH, wb.p + kMlpW3b, kMlpH, w.p + kMlpB3, nullptr, 0, 0, Y.p, kMlpR, nullptr,
-            0);
+            0, nullptr, 0);
   }
-  // gradient of the masked mean squared error into g (B a multiple of 32); per-block
+  // gradient of the masked mean squared error into g (after forward(s, B, true)); per-block
   // partial losses in part[0..64)
   void backward(hipStream_t s, int B, float inv_count) {
     mse_grad(s, B, Y.p, T.p, rank.p, inv_count, dYb.p, dYf.p, part.p, 64);
+    const TransposeBf16 tr[4] = {{B, kMlpIn, X.p, XT.p},
+                                 {B, kMlpR, dYb.p, dYT.p},
+                                 {kMlpH, kMlpH, wb.p + kMlpW2b, w2t.p},
+                                 {kMlpR, kMlpH, wb.p + kMlpW3b, w3t.p}};
+    transposes_bf16(s, 4, tr);
     colsum_f32(s, B, kMlpR, dYf.p, kMlpR, g.p + kMlpB3);
-    transpose_bf16(s, B, kMlpR, dYb.p, kMlpR, dYT.p, B);
-    transpose_bf16(s, B, kMlpH, H2.p, kMlpH, H2T.p, B);
-    gemm_nt(s, kMlpR, kMlpH, B, dYT.p, B, H2T.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW3, kMlpH, nullptr, 0);
-    transpose_bf16(s, kMlpR, kMlpH, wb.p + kMlpW3b, kMlpH, w3t.p, kMlpR);
-    gemm_nt(s, B, kMlpH, kMlpR, dYb.p, kMlpR, w3t.p, kMlpR, nullptr, H2.p, kMlpH, 0, nullptr, 0, dH2.p, kMlpH);
+    gemm_nt(s, kMlpR, kMlpH, B, dYT.p, B, H2T.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW3, kMlpH, nullptr, 0, nullptr, 0);
+    gemm_nt(s, B, kMlpH, kMlpR, dYb.p, kMlpR, w3t.p, kMlpR, nullptr, H2.p, kMlpH, 0, nullptr, 0, dH2.p, kMlpH, dH2T.p,
+            B);
     colsum_bf16(s, B, kMlpH, dH2.p, kMlpH, g.p + kMlpB2);
-    transpose_bf16(s, B, kMlpH, dH2.p, kMlpH, dH2T.p, B);
-    transpose_bf16(s, B, kMlpH, H1.p, kMlpH, H1T.p, B);
-    gemm_nt(s, kMlpH, kMlpH, B, dH2T.p, B, H1T.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW2, kMlpH, nullptr, 0);
-    transpose_bf16(s, kMlpH, kMlpH, wb.p + kMlpW2b, kMlpH, w2t.p, kMlpH);
-    gemm_nt(s, B, kMlpH, kMlpH, dH2.p, kMlpH, w2t.p, kMlpH, nullptr, H1.p, kMlpH, 0, nullptr, 0, dH1.p, kMlpH);
+    gemm_nt(s, kMlpH, kMlpH, B, dH2T.p, B, H1T.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW2, kMlpH, nullptr, 0, nullptr,
+            0);
+    gemm_nt(s, B, kMlpH, kMlpH, dH2.p, kMlpH, w2t.p, kMlpH, nullptr, H1.p, kMlpH, 0, nullptr, 0, dH1.p, kMlpH, dH1T.p,
+            B);
     colsum_bf16(s, B, kMlpH, dH1.p, kMlpH, g.p + kMlpB1);
-    transpose_bf16(s, B, kMlpH, dH1.p, kMlpH, dH1T.p, B);
-    transpose_bf16(s, B, kMlpIn, X.p, kMlpIn, XT.p, B);
-    gemm_nt(s, kMlpH, kMlpIn, B, dH1T.p, B, XT.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW1, kMlpIn, nullptr, 0);
+    gemm_nt(s, kMlpH, kMlpIn, B, dH1T.p, B, XT.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW1, kMlpIn, nullptr, 0, nullptr,
+            0);
   }
 };
 
@@ -944,7 +946,7 @@ void update_nonneg(Work &w, int mode, const ptn_options &o, const ModeIn &in) {
   if (warm) {
     // the network proposes each row's start; rows failing the KKT test keep A (k_warm_select)
     mlp_features(s, I, w.R, w.ldr, in.V, w.M, A, nullptr, ms->X.p, nullptr, nullptr, ms->scale.p);
-    ms->forward(s, (int)I);
+    ms->forward(s, (int)I, false);
     if (o.warm_refine > 0) {
       // every finite proposal first takes warm_refine Nesterov steps of the same subproblem
       // (anchor A, the global stop test included); the test then judges the refined rows
@@ -2436,7 +2438,7 @@ ptn_status ptn_mlp_forward(ptn_handle h, int n, const float *X, float *Y) {
     MlpState &ms = *h->mlp;
     ms.ensure_rows(n);
     upload_rows(ms, n, n, X, nullptr, nullptr);
-    ms.forward(h->stream, n);
+    ms.forward(h->stream, n, false);
     HIPCHK(hipMemcpyAsync(Y, ms.Y.p, (size_t)n * kMlpR * sizeof(float), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());
@@ -2459,7 +2461,7 @@ ptn_status ptn_mlp_loss_grad(ptn_handle h, int n, const float *X, const float *T
     const int np = (n + 31) / 32 * 32;
     ms.ensure_rows(np);
     upload_rows(ms, n, np, X, T, rank);
-    ms.forward(h->stream, np);
+    ms.forward(h->stream, np, true);
     ms.backward(h->stream, np, (float)(1.0 / (double)count));
     std::vector<double> part(64);
     HIPCHK(hipMemcpyAsync(part.data(), ms.part.p, 64 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
@@ -2544,7 +2546,7 @@ ptn_status ptn_mlp_train(ptn_handle h, int epochs, int batch, double lr, uint64_
         int64_t count = 0;
         for (int64_t r = st * batch; r < (st + 1) * batch; ++r) count += ms.hrank[perm[r]];
         gather_rows(s, batch, idx.p + st * batch, ms.dx.p, ms.dt.p, ms.drank.p, ms.X.p, ms.T.p, ms.rank.p);
-        ms.forward(s, batch);
+        ms.forward(s, batch, true);
         ms.backward(s, batch, count > 0 ? (float)(1.0 / (double)count) : 0.f);
         adam_step(s, kMlpParams, ms.w.p, ms.g.p, ms.m1.p, ms.m2.p, (float)lr, 0.9f, 0.999f, 1e-8f, ++ms.step, ms.wb.p);
         sum_partials(s, ms.part.p, 64, losses.p + ep * spe + st);

@@ -133,8 +133,13 @@ __host__ __device__ inline int64_t mlp_bf16_index(int64_t e) {
   return -1;
 }
 void gemm_nt(hipStream_t s, int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *bias,
-             const void *gate, int ldg, int relu, float *C, int ldc, void *Cb, int ldcb);
-void transpose_bf16(hipStream_t s, int rows, int cols, const void *in, int ldi, void *out, int ldo);
+             const void *gate, int ldg, int relu, float *C, int ldc, void *Cb, int ldcb, void *Cbt, int ldcbt);
+struct TransposeBf16 {                       // out (cols x rows) = in^T (rows x cols), both contiguous
+  int rows, cols;
+  const void *in;
+  void *out;
+};
+void transposes_bf16(hipStream_t s, int n, const TransposeBf16 *m);   // n <= 4, one launch
 void mlp_features(hipStream_t s, int64_t I, int R, int ldr, const double *V, const double *M, const double *A,
                   const double *Anew, void *X, float *T, unsigned char *rank, float *scale);
 // C: the proposals after warm_refine Nesterov steps (null: the network's outputs Y, scale)

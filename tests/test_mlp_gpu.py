@@ -76,6 +76,23 @@ def test_bias_gradients_at_the_edges_of_the_row_tiles(h, n):
         assert P.rel_err(g[a:b].astype(np.float64), go[a:b]) < 5e-4
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 128, 160, 257])
+def test_products_at_the_edges_of_the_tiles(h, n):
+    # the layers' products are taken in 32 x 32 tiles and 128 of the inner index at a time; the
+    # batch is the layers' rows and the weight gradients' inner index.  Bounds: a hidden
+    # activation that rounds to the neighbouring BF16 value (~1e-4), as above
+    h.mlp_init(7)
+    w = h.mlp_params().astype(np.float64)
+    X, T, rank = _data(n, 3)
+    Yo, _ = m.forward(w, X, bf16=True)
+    assert P.rel_err(h.mlp_forward(X), Yo) < 5e-4
+    loss, g = h.mlp_loss_grad(X, T, rank)
+    lo, go = m.loss_grad(w, X, T, rank, bf16=True)
+    assert loss == pytest.approx(lo, rel=1e-4)
+    for a, b in zip(BLOCKS, BLOCKS[1:]):
+        assert P.rel_err(g[a:b].astype(np.float64), go[a:b]) < 5e-4
+
+
 def test_harvested_features_match_oracle(h):
     dims, R = [12, 10, 8], 3
     X, _ = o.make_tensor(dims, R, seed=3, snr_db=30.0)
