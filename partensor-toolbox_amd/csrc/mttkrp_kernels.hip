@@ -43,7 +43,7 @@ KrArgs to_args(const KrSpec &w) {
 }
 
 template <typename TX>
-__device__ __forceinline__ double ld(const TX *p) { return (double)__builtin_nontemporal_load(p); }
+__device__ __forceinline__ double ld(const TX *p) { return (double)*p; }
 
 // ---------------------------------------------------------------------------
 // gemm_cm: a block owns 64 consecutive rows and one k-chunk; its 4 waves take
