@@ -553,10 +553,13 @@ __device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *P, 
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int row = (wave + NW * tt) * 16 + kk + 4 * j;
-      if (on && wave + NW * tt < T && row < I) {
-        double v = ac[tt][j];
-        if (fb) v = 0.9 * v + 0.1 * Ag[row * kBR + m];
-        Ag[row * kBR + m] = v;
+      if (wave + NW * tt < T && row < I) {
+        double v = 0.0;                      // columns >= R of F: zeros, the cost sums over all 16
+        if (on) {
+          v = ac[tt][j];
+          if (fb) v = 0.9 * v + 0.1 * Ag[row * kBR + m];
+          Ag[row * kBR + m] = v;
+        }
         S.F[0][row * kBR + m] = v;
       }
     }

@@ -201,6 +201,35 @@ def test_batch_launch_shapes_agree_bitwise(h):
     assert a256[2] == pytest.approx(a512[2], rel=1e-11)
 
 
+@pytest.mark.parametrize("arith", [P.ARITH_F64, P.ARITH_F32])
+def test_batch_does_not_read_what_lds_held_before(h, arith):
+    """A launch finds in LDS what the kernels before it left there.  An MTTKRP of a tensor of
+    NaNs (infinities) leaves those; the batch's results after it are the bits of those after an
+    MTTKRP of ones, for modes shorter and longer than the modes solved before them."""
+    probs = [((2, 3, 4), 2), ((16, 17, 18), 4), ((48, 80, 112), 12), ((112, 80, 48), 11), ((20, 20, 20), 1),
+             ((10, 104, 121), 5), ((33, 16, 128), 16), ((90, 16, 128), 11)]
+    h.batch_set(_tensors(probs, seed0=20), [R for _, R in probs])
+    init = [o.gen_factors(list(d), R, seed=500 + p) for p, (d, R) in enumerate(probs)]
+    dims, runs = [512, 64, 64], []
+    ones = [np.ones((d, 64)) for d in dims]
+    with P.Handle(0) as h2:
+        for v in (1.0, np.nan, np.inf):
+            h2.set_tensor(np.full(dims, v), storage=P.TENSOR_BOTH)
+            for block in (512, 256):
+                for mode in range(3):
+                    h2.mttkrp(ones, mode)
+                    h2.mttkrp(ones, mode, arith=P.ARITH_F32)
+                F, st, _, _ = h.cpd_batch(init, block=block, grid=256, with_log=False, arith=arith, max_iter=6,
+                                          threshold_error=0.0)
+                runs.append((v, block, F, [s["f_value"] for s in st]))
+    for v, block, F, f in runs[2:]:
+        _, _, F0, f0 = runs[0] if block == 512 else runs[1]
+        assert f == f0, (v, block)
+        for p, Fp in enumerate(F):
+            for a, b in zip(Fp, F0[p]):
+                assert np.array_equal(a, b), (v, block, p)
+
+
 def test_batch_threshold_stop(h):
     """Problems stop on their own threshold test at the oracle's sweep and are left alone
     afterwards; the stopping sweep takes no line search."""
