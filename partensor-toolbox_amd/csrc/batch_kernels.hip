@@ -567,6 +567,21 @@ __device__ __forceinline__ int nnls_block(int I, int R, BatchLds &S, double *P, 
   return it;
 }
 
+// The constants and momentum coefficients of a solve, from S.V (one wave).  A function of its
+// own, so that its registers are not the MTTKRP's beside it (per sweep of the 512-problem batch
+// on FP32 / FP64 matrix cores 1.31 / 1.25 ms inlined, 1.16 / 1.21 so; 2000 problems of modes
+// 16 .. 32, 256-thread blocks, with the routine as it was 1.01 / 1.12, now 0.90 / 1.03); it takes
+// the LDS address, since a generic one would make its accesses flat.
+typedef __attribute__((address_space(3))) BatchLds *lds_ptr;
+__device__ __noinline__ void nnls_constants(lds_ptr Sp, int R, int max_inner) {
+  BatchLds &S = *(BatchLds *)Sp;
+  for (int x = threadIdx.x & 63; x < kBR * kBR; x += 64) S.eig.t[x] = S.V[x];
+  PTN_WAVE_SYNC();
+  double amax, amin;
+  eig_extremes_wave(R, S.eig, amax, amin);
+  glambda_betas(amax, amin, &S.prm, max_inner, S.betas);
+}
+
 // one sweep of one problem
 // Member g of the problem's group: member 0 works on the problem's state and writes its
 // status and log; members g > 0 on private copies of the state (identical values: every
@@ -598,14 +613,7 @@ __device__ __forceinline__ void sweep_problem(const BatchArgs &a, int p, int g, 
     load_rows<BS>(n == 0 ? A1 : A0, Ia, S.F[0]);
     load_rows<BS>(n == 2 ? A1 : A2, Ib, S.F[1]);
     __syncthreads();
-    auto eig = [&] {
-      const int l = t & 63;
-      for (int x = l; x < kBR * kBR; x += 64) S.eig.t[x] = S.V[x];
-      PTN_WAVE_SYNC();
-      double amax, amin;
-      eig_extremes_wave<kBR>(R, S.eig, amax, amin);
-      glambda_betas(amax, amin, &S.prm, a.max_inner, S.betas);
-    };
+    auto eig = [&] { nnls_constants((lds_ptr)&S, R, a.max_inner); };
     const int In = n == 0 ? I0 : n == 1 ? I1 : I2;
     // FP64 matrix cores: the eigen wave (R <= 16: microseconds) then takes 3/4 of an MTTKRP
     // share (1.76 -> 1.69 ms per 512-problem sweep); FP32 ones: the other seven waves split

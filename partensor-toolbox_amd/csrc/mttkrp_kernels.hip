@@ -42,6 +42,9 @@ KrArgs to_args(const KrSpec &w) {
   return a;
 }
 
+// A cached load: where rows are no whole cache lines, neighbouring columns share them, and a
+// non-temporal line is fetched again for each (501 x 403 x 307 at rank 17: 140 us, cached 120;
+// 800^3 at rank 32, whole lines: 877 either way).
 template <typename TX>
 __device__ __forceinline__ double ld(const TX *p) { return (double)*p; }
 

@@ -162,15 +162,14 @@ __global__ __launch_bounds__(64 * kMaxOrder) void k_gram_combine_all(GramBatch b
 // With ng > 0 the matrix is first formed as the Hadamard product of the ng Grams in
 // list order (V = G_l0, V = G_lj * V; PartialCwiseProd) and stored to Vout; with
 // betas != nullptr the momentum coefficients of the Nesterov solve follow the
-// eigenvalues (one kernel prepares an NNLS update).  One block of four waves.
+// eigenvalues (one kernel prepares an NNLS update).  One block.
 template <int RB>
-__global__ __launch_bounds__(256) void k_eig_extremes(int R, const double *__restrict__ V, GramPtrs G, int ng,
+__global__ __launch_bounds__(kEigThreads<RB>) void k_eig_extremes(int R, const double *__restrict__ V, GramPtrs G, int ng,
                                                       double *__restrict__ Vout, NnlsParams *prm, int max_inner,
                                                       double *__restrict__ betas) {
   __shared__ EigLds<RB> S;
-  __shared__ double part[4][RB];
   const int n = R;
-  for (int x = threadIdx.x; x < RB * RB; x += 256) {
+  for (int x = threadIdx.x; x < RB * RB; x += kEigThreads<RB>) {
     const int r = x / RB, c = x % RB;
     double v = 0.0;
     if (r < n && c < n) {
@@ -187,7 +186,7 @@ __global__ __launch_bounds__(256) void k_eig_extremes(int R, const double *__res
   }
   __syncthreads();
   double amax, amin;
-  eig_extremes_block<RB>(n, S, part, amax, amin);
+  eig_extremes_block<RB>(n, S, amax, amin);
   if (threadIdx.x < 64) glambda_betas(amax, amin, prm, max_inner, betas);
 }
 
@@ -655,18 +654,18 @@ void grams_all(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const 
 
 void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p, int max_inner, double *betas) {
   const GramPtrs G{};
-  if (R <= 16) k_eig_extremes<16><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
-  else if (R <= 32) k_eig_extremes<32><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
-  else k_eig_extremes<64><<<1, 256, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
+  if (R <= 16) k_eig_extremes<16><<<1, kEigThreads<16>, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
+  else if (R <= 32) k_eig_extremes<32><<<1, kEigThreads<32>, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
+  else k_eig_extremes<64><<<1, kEigThreads<64>, 0, s>>>(R, V, G, 0, nullptr, p, max_inner, betas);
 }
 
 void nnls_setup(hipStream_t s, int R, int ng, const double *const *grams, double *V, NnlsParams *p, int max_inner,
                 double *betas) {
   GramPtrs G{};
   for (int j = 0; j < ng; ++j) G.p[j] = grams[j];
-  if (R <= 16) k_eig_extremes<16><<<1, 256, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
-  else if (R <= 32) k_eig_extremes<32><<<1, 256, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
-  else k_eig_extremes<64><<<1, 256, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
+  if (R <= 16) k_eig_extremes<16><<<1, kEigThreads<16>, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
+  else if (R <= 32) k_eig_extremes<32><<<1, kEigThreads<32>, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
+  else k_eig_extremes<64><<<1, kEigThreads<64>, 0, s>>>(R, nullptr, G, ng, V, p, max_inner, betas);
 }
 
 void nnls_iterate(hipStream_t s, int64_t I, int R, int ldr, const double *V, const NnlsParams *p,

@@ -217,6 +217,26 @@ def test_sym_extremes_edge_cases_match_oracle(h, n, kind):
     assert L == Lo and mu == muo
 
 
+@pytest.mark.parametrize("R", [1, 2, 3, 4, 5, 15, 16, 17, 18, 31, 32, 33, 61, 63, 64])
+def test_extremes_at_the_edges_of_the_padded_ranks(h, R):
+    # bitwise the oracle's on both sides of the routine's forms (one wave, two, four; pivot
+    # steps in fours): plain, indefinite, and what its branches look for, uncoupled columns
+    # (a column to eliminate that is zero already), repeated and zero eigenvalues, and entries
+    # whose squares leave the range in which the short division is taken
+    rng = np.random.default_rng(R)
+    B = rng.standard_normal((2 * R + 1, R))
+    S = rng.standard_normal((R, R))
+    D = np.diag(rng.standard_normal(R))
+    K = np.kron(np.eye((R + 2) // 3), np.ones((3, 3)))[:R, :R]
+    for name, V in (("gram", B.T @ B), ("indefinite", S + S.T), ("diagonal", D), ("blocks", K), ("ones", np.ones((R, R))),
+                    ("zero", np.zeros((R, R))), ("identity", np.eye(R)), ("large", (B.T @ B) * 2.0**300),
+                    ("small", (S + S.T) * 2.0**-300), ("graded", (B.T @ B) * np.outer(*[10.0 ** -np.arange(R)] * 2))):
+        V = (V + V.T) / 2
+        L, mu = h.sym_extremes(V)
+        Lo, muo, _ = o.sym_extremes(V)
+        assert L == Lo and mu == muo, name
+
+
 @pytest.mark.parametrize("I,R,d", [(7, 4, 1e-2), (300, 32, 1e-2), (129, 64, 1e-2), (50, 10, 0.0), (20, 5, 1e30)])
 def test_nesterov_matches_oracle(h, I, R, d):
     say("nnls", I, R, d)
