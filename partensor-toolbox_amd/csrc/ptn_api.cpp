@@ -590,7 +590,7 @@ Node node_cm(Work &w, const KrSpec &k, int64_t Mrows, int64_t K, int S, double *
       gemm_cm_f64(s, w.x64(), w.x32(), Mrows, K, k, w.ldr, S, w.part);
     }
     w.pass_mark(timed, true, s);
-    if (S > 1) reduce_splits(s, w.part, S, Mrows * w.ldr, dst64);
+    if (S > 1) reduce_splits(s, w.part, S, Mrows * w.ldr, dst64, true);
     return Node{dst64, nullptr, w.ldr};
   }
   w.pack(k, K, 0);
@@ -654,13 +654,13 @@ void contract_node(Work &w, const Node &nd, const KrSpec &sp, int outmode, doubl
     REQUIRE(S * In * w.ldr <= w.part_cap, PTN_ERR_INVALID, "partial buffer too small");
     contract2(s, nd.p64, nd.p32, nd.ld, D0, D1, outmode, sp.fac[1 - outmode], w.ldr, w.R, S, S == 1 ? M : w.part,
               nd.sel, nd.sel_off);
-    if (S > 1) reduce_splits(s, w.part, S, In * w.ldr, M);
+    if (S > 1) reduce_splits(s, w.part, S, In * w.ldr, M, !w.mfma32);
     return;
   }
   const int S = pick_splits(In, Cother / 64, 64);
   REQUIRE(S * In * w.ldr <= w.part_cap, PTN_ERR_INVALID, "partial buffer too small");
   contract_rows(s, nd.p64, nd.p32, nd.ld, sp, outmode, w.ldr, S, w.part, nd.sel, nd.sel_off);
-  reduce_splits(s, w.part, S, In * w.ldr, M);
+  reduce_splits(s, w.part, S, In * w.ldr, M, !w.mfma32);
 }
 
 
@@ -672,12 +672,19 @@ void mttkrp_standard(Work &w, double *base, int mode, double *M) {
     KrSpec k{};
     for (int j = 1; j < N; ++j) { k.dim[k.nm] = w.dims[j]; k.fac[k.nm] = w.Fb(base, j); k.nm++; }
     const int64_t Ktot = w.total / I0;
-    const int S = pick_splits((I0 + 63) / 64, Ktot / 256, 256);
     if (!w.mfma32) {
+      // Two blocks to a CU run at once, so the splits of a tensor of up to 1 GB make one wave of
+      // 512 blocks; larger ones are better off with a few waves, whose ends overlap.  A split takes
+      // at least 32 columns, eight for each wave (with 256 at least, and 2048 blocks for all: 100^3
+      // at rank 10 14.4 us, here 11.5; 37 x 23 x 41 at 5 17.1 and 8.1; 200^3 at 32 34.6 and 31.1;
+      // 501 x 403 x 307 at 33 183 and 174; 640^3 at 48 641 us, with 512 blocks 665).
+      const int64_t blocks = (I0 + 63) / 64, target = w.total < ((int64_t)1 << 27) ? 512 : 2048;
+      const int S = (int)std::max<int64_t>(1, std::min(std::min<int64_t>(target / blocks, 256), Ktot / 32));
       gemm_cm_f64(w.h->stream, w.x64(), w.x32(), I0, Ktot, k, w.ldr, S, w.part);
-      reduce_splits(w.h->stream, w.part, S, I0 * w.ldr, M);
+      reduce_splits(w.h->stream, w.part, S, I0 * w.ldr, M, true);
     } else {
       // FP32 partials summed in FP64 by the row contraction of a 1-digit node per split
+      const int S = pick_splits((I0 + 63) / 64, Ktot / 256, 256);
       Node nd = node_cm(w, k, I0, Ktot, S, nullptr, w.T32);
       KrSpec sp{};
       sp.nm = 1; sp.dim[0] = I0;
@@ -807,7 +814,7 @@ void left_node_pair(Work &w, double *cur, double *acc) {
     const int S2 = pick_splits((D0 + 7) / 8, D1 / 16, 64);   // contract_node's split of outmode 0
     REQUIRE(2 * S2 * D0 * w.ldr <= w.part_cap, PTN_ERR_INVALID, "partial buffer too small");
     contract2_pair(s, w.YL2.p + w.rpf, w.YL2.p, width, D0, D1, 0, la.fac[1], lc.fac[1], w.ldr, w.R, S2, w.part);
-    reduce_splits(s, w.part, S2, 2 * D0 * w.ldr, w.M2);
+    reduce_splits(s, w.part, S2, 2 * D0 * w.ldr, w.M2, false);
   } else {                                   // three or more digits (orders 5 .. 8): one contraction per half
     contract_node(w, Node{nullptr, w.YL2.p + w.rpf, width}, la, 0, w.M2);
     contract_node(w, Node{nullptr, w.YL2.p, width}, lc, 0, w.M2 + D0 * w.ldr);

@@ -192,7 +192,9 @@ void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, 
 void contract_rows(hipStream_t s, const double *T64, const float *T32, int64_t ldt, const KrSpec &spec,
                    int outmode, int ldr, int splits, double *partials, const int *sel = nullptr,
                    int64_t sel_off = 0);
-void reduce_splits(hipStream_t s, const double *partials, int splits, int64_t n, double *out);
+// runs: many splits may be summed in eight runs (FP64 contractions; the sums of FP32 partials keep
+// their one order, since a rounding of theirs can turn a BF16 rounding of the next sweep)
+void reduce_splits(hipStream_t s, const double *partials, int splits, int64_t n, double *out, bool runs);
 // Two-digit node Y (rows i0 + D0 i1, ld values per row) contracted against the other
 // digit's factor F: part[split][i][ldr] for the kept digit i (outmode 0: i0, 1: i1).
 // sel (optional, device): the node starts at Y + (*sel) * sel_off.
