@@ -1298,16 +1298,28 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
 
     // The side stream forms V_n, its eigenvalues and the momentum coefficients of mode n
     // while the main stream contracts the tensor for mode n (small tensors: the other way
-    // round, eig_first below); during the line-search pass
-    // it also forms the accelerated factors' Grams, V_hat, the sweep's cost and both
+    // round, eig_first below, or one after the other); during the line-search pass it also forms the accelerated factors' Grams, V_hat, the sweep's cost and both
     // mode-0 set-ups of the next sweep.  The aux stream forms the order-3 tree's right node
     // (right_node_early).  All three run at the default priority.
-    hipStream_t ms = h->stream, ss = h->side;
+    // A hop between the streams costs the host two calls and the device 5 to 10 us of waiting, so
+    // where a mode's contraction is shorter than that and little of the eigen routine everything
+    // stays on one stream.  Sweeps on one / on two, R <= 16: 20^3 160 / 210 us, 64^3 180 / 216,
+    // 100^3 205 / 215, 301 x 205 x 150 (74 MB) 258 / 278, 300^3 (216 MB) 365 / 339; R <= 32, where
+    // the eigen routine takes 50 us, order 3 on the FP64 matrix cores: 64^3 296 / 321, 100^3 (8 MB)
+    // 320 / 326, 150^3 (27 MB) the same, 200^3 (64 MB) 318 / 304, but with the more and longer
+    // kernels of other contractions beside it 64^3 BF16x3 299 / 282, 30^4 437 / 422, FP32 438 / 392;
+    // R > 32 (116 us): 100^3 560 / 549.
+    const bool early_right = tree && w.mfma32 && N == 3;
+    const int64_t one_bytes = (int64_t)(R <= 16 ? 96 : R <= 32 && N == 3 && !w.mfma32 ? 8 : 0) << 20;
+    const bool one_stream = !early_right && w.total * (w.f32 ? 4 : 8) <= one_bytes;
+    hipStream_t ms = h->stream, ss = one_stream ? ms : h->side;
     auto fork = [&] {      // side waits for the main stream's work so far
+      if (one_stream) return;
       HIPCHK(hipEventRecord(h->ev[0], ms));
       HIPCHK(hipStreamWaitEvent(ss, h->ev[0], 0));
     };
     auto join = [&] {      // main waits for the side stream's work so far
+      if (one_stream) return;
       HIPCHK(hipEventRecord(h->ev[1], ss));
       HIPCHK(hipStreamWaitEvent(ms, h->ev[1], 0));
     };
@@ -1363,7 +1375,6 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
       // decision, so it runs on the side stream beside the next pass (Normalize leaves
       // the last factor and its Gram as they are unless it is the weight factor)
       const bool side_cost = step_now && pair && !(o.normalization && !all_orth && wf == last);
-      const bool early_right = tree && w.mfma32 && N == 3;
       // A tensor that is read in less time than the eigen routine takes (28, 65 and 150 us at
       // the three padded ranks; a contraction reads about 4.5 TB/s): the set-up, then the longer
       // of the two, follows the Gram on the main stream, and the contraction crosses to the side
@@ -1371,7 +1382,7 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
       // order: 100^3 R = 10 229 / 269 us, 200^3 R = 20 342 / 375, 400^3 R = 64 (512 MB) 1232 /
       // 1452; 300^3 R = 16 (216 MB) 394 / 387, 400^3 R = 16 635 / 598.
       const int64_t eig_bytes = (int64_t)(R <= 16 ? 128 : R <= 32 ? 288 : 640) << 20;
-      const bool short_read = !early_right && w.total * (w.f32 ? 4 : 8) <= eig_bytes;
+      const bool short_read = !early_right && !one_stream && w.total * (w.f32 ? 4 : 8) <= eig_bytes;
       for (int n = 0; n < N; ++n) {
         const bool set_up = !(n == 0 && prepped0);
         const bool eig_first = short_read && o.constraints[n] == PTN_NONNEGATIVITY;
