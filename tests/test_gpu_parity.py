@@ -402,6 +402,36 @@ def test_als_small_parity(h, dims, R):
         _als_parity(h, X, R, init, mttkrp_form=form, oform=_oform(form), max_iter=15, threshold_error=0.0)
 
 
+@pytest.mark.parametrize("dims,R", [([40, 30, 20], 16), ([40, 30, 20], 17), ([13, 9, 10, 8], 17),
+                                    ([128, 128, 64], 32), ([128, 128, 65], 32)])
+def test_als_on_one_stream_and_on_two(h, dims, R):
+    """Both sides of the rule that keeps a sweep on one stream: the padded rank 16, order 3 and 4 at
+    rank 17, and 8 MB of an order-3 tensor at rank 32."""
+    X, _ = o.make_tensor(dims, 6, seed=12, snr_db=25.0)
+    init = o.gen_factors(dims, R, seed=13)
+    h.set_tensor(X)
+    for form in (P.MTTKRP_STANDARD, P.MTTKRP_DIMTREE):
+        _als_parity(h, X, R, init, mttkrp_form=form, oform=_oform(form), max_iter=6, threshold_error=0.0)
+
+
+@pytest.mark.parametrize("I0", [1, 64, 65, 300])
+@pytest.mark.parametrize("K", [(1, 31), (4, 8), (3, 11), (30, 17), (32, 16), (27, 19), (90, 91)])
+def test_mode0_splits(h, I0, K):
+    """The FP64 contraction of mode 0 about its splits: one (under 64 columns), under and from sixteen
+    (summed in runs), and as many as the rows' blocks leave.  Up to 8190 terms to a sum, each
+    side in its own order: 8190 x 2^-53 = 9e-13 at most."""
+    rng = np.random.default_rng(I0 + K[0])
+    dims = [I0, *K]
+    X = rng.random(dims)
+    h.set_tensor(X, storage=P.TENSOR_BOTH)
+    for R in (5, 33):
+        A = [rng.random((d, R)) for d in dims]
+        M = o.mttkrp(X, A, 0)
+        assert P.rel_err(h.mttkrp(A, 0), M) <= 1e-12
+        X32 = X.astype(np.float32).astype(np.float64)
+        assert P.rel_err(h.mttkrp(A, 0, arith=P.ARITH_F32_F64), o.mttkrp(X32, A, 0)) <= 1e-12
+
+
 def test_als_c2_full_size_three_sweeps(h):
     """Config 2 at full size (800^3, true rank 32, SNR 20 dB, R = 32, init seed 1): three
     sweeps (the line search runs at sweep 2) of the plain FP64 path, per-mode and tree, against
