@@ -448,7 +448,7 @@ struct Work {
     grams.alloc(h, (size_t)N * R * R, kRaw); agr.alloc(h, (size_t)N * R * R, kRaw);
     Vm.alloc(h, (size_t)(N + 1) * R * R, kRaw); Vacc.alloc(h, (size_t)R * R, kRaw);
     M.alloc(h, maxI * ldr, kRaw); Aold.alloc(h, maxI * ldr, kRaw); colsum.alloc(h, kMaxRank, kRaw);
-    prm.alloc(h, kMaxOrder + 1); mask.alloc(h, nnls_mask_words(maxI), kRaw); flags.alloc(h, 4, kRaw);
+    prm.alloc(h, kMaxOrder + 1, kRaw); mask.alloc(h, nnls_mask_words(maxI), kRaw); flags.alloc(h, 4, kRaw);
     nscr.alloc(h, 2 * kMaxOrder * kMaxRank, kRaw); scal.alloc(h, 8, kRaw);
     betas.alloc(h, (size_t)(N + 1) * (kMaxInner + 1), kRaw);
     gpart.alloc(h, (size_t)((maxI + 31) / 32) * R * R, kRaw);
@@ -893,18 +893,14 @@ void frob_norm(ptn_handle h) {
   h->frob_valid = true;
 }
 
+// (the caller waits for the stream before it returns: packed_host may be read until then)
 void upload_factors(Work &w, const double *packed_host, double *dst_rows) {
   ptn_handle h = w.h;
   int64_t n = 0;
   for (int k = 0; k < w.N; ++k) n += w.dims[k] * w.R;
   DevBuf<double> tmp(h, n, kRaw);
   HIPCHK(hipMemcpyAsync(tmp.p, packed_host, n * sizeof(double), hipMemcpyHostToDevice, h->stream));
-  int64_t o = 0;
-  for (int k = 0; k < w.N; ++k) {
-    colmajor_to_rows(h->stream, w.dims[k], w.R, w.ldr, tmp.p + o, dst_rows + w.off[k]);
-    o += w.dims[k] * w.R;
-  }
-  HIPCHK(hipStreamSynchronize(h->stream));
+  factors_to_rows(h->stream, w.N, w.dims, w.R, w.ldr, tmp.p, dst_rows);
 }
 
 void download_factors(Work &w, const double *src_rows, double *packed_host) {
@@ -912,11 +908,7 @@ void download_factors(Work &w, const double *src_rows, double *packed_host) {
   int64_t n = 0;
   for (int k = 0; k < w.N; ++k) n += w.dims[k] * w.R;
   DevBuf<double> tmp(h, n, kRaw);
-  int64_t o = 0;
-  for (int k = 0; k < w.N; ++k) {
-    rows_to_colmajor(h->stream, w.dims[k], w.R, w.ldr, src_rows + w.off[k], tmp.p + o);
-    o += w.dims[k] * w.R;
-  }
+  rows_to_factors(h->stream, w.N, w.dims, w.R, w.ldr, src_rows, tmp.p);
   HIPCHK(hipMemcpyAsync(packed_host, tmp.p, n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
 }
@@ -1276,6 +1268,7 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
     }
     if (pair && o.acceleration) w.enable_pair();
     const int N = w.N, last = N - 1;
+    HIPCHK(hipMemsetAsync(w.prm.p, 0, w.prm.n * sizeof(NnlsParams), h->stream));
     upload_factors(w, init_packed, w.fac);
     for (int k = 0; k < N; ++k) gram_of(w, w.F(k), w.dims[k], w.G(k));
 
@@ -1298,9 +1291,10 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
 
     // The side stream forms V_n, its eigenvalues and the momentum coefficients of mode n
     // while the main stream contracts the tensor for mode n (small tensors: the other way
-    // round, eig_first below, or one after the other); during the line-search pass it also forms the accelerated factors' Grams, V_hat, the sweep's cost and both
-    // mode-0 set-ups of the next sweep.  The aux stream forms the order-3 tree's right node
-    // (right_node_early).  All three run at the default priority.
+    // round, eig_first below, or one after the other); during the line-search pass it also
+    // forms the accelerated factors' Grams, V_hat, the sweep's cost and both mode-0 set-ups of
+    // the next sweep.  The aux stream forms the order-3 tree's right node (right_node_early).
+    // All three run at the default priority.
     // A hop between the streams costs the host two calls and the device 5 to 10 us of waiting, so
     // where a mode's contraction is shorter than that and little of the eigen routine everything
     // stays on one stream.  Sweeps on one / on two, R <= 16: 20^3 160 / 210 us, 64^3 180 / 216,

@@ -176,6 +176,9 @@ int cost_explicit_partials(hipStream_t s, int N, const int64_t *dims, int R, int
 void fill_zero(hipStream_t s, void *p, int64_t words);
 void colmajor_to_rows(hipStream_t s, int64_t I, int R, int ldr, const double *src, double *dst);
 void rows_to_colmajor(hipStream_t s, int64_t I, int R, int ldr, const double *src, double *dst);
+// N factors at once: packed column-major <-> rows one factor after the other
+void factors_to_rows(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *packed, double *rows);
+void rows_to_factors(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const double *rows, double *packed);
 void rows_to_f32(hipStream_t s, int64_t n, const double *src, float *dst);
 
 // ---- MTTKRP building blocks (mttkrp_kernels.hip) ----
