@@ -30,15 +30,26 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // products of a step of 1024 rows: 15.0 us, with the two groups but fragments fetched where they
 // lie 14.1 us, so 8.9 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_gemm_nt(int M, int N, int K, const __bf16 *__restrict__ A, int lda,
-                                                const __bf16 *__restrict__ B, int ldb, const float *__restrict__ bias,
-                                                const __bf16 *__restrict__ gate, int ldg, int relu,
-                                                float *__restrict__ C, int ldc, __bf16 *__restrict__ Cb, int ldcb,
-                                                __bf16 *__restrict__ Cbt, int ldcbt) {
-  constexpr int KG = 128, LD = KG + 8;
-  __shared__ __align__(16) __bf16 tile[64 * LD];         // 32 rows of A, 32 of B
+struct GemmNt {
+  int M, N, K, lda, ldb, ldg, relu, ldc, ldcb, ldcbt;
+  const __bf16 *A, *B;
+  const float *bias;
+  const __bf16 *gate;
+  float *C;
+  __bf16 *Cb, *Cbt;
+  __host__ __device__ int tiles_n() const { return (N + 31) / 32; }
+  __host__ __device__ int tiles() const { return tiles_n() * ((M + 31) / 32); }
+};
+constexpr int kGemmLd = 128 + 8, kGemmLds = 64 * kGemmLd * 2;   // bytes: 32 rows of A, 32 of B
+__device__ __forceinline__ void gemm_tile(const GemmNt &g, int b, __bf16 *tile) {
+  const int M = g.M, N = g.N, K = g.K, lda = g.lda, ldb = g.ldb;
+  const __bf16 *__restrict__ A = g.A, *__restrict__ B = g.B, *__restrict__ gate = g.gate;
+  const float *__restrict__ bias = g.bias;
+  float *__restrict__ C = g.C;
+  __bf16 *__restrict__ Cb = g.Cb, *__restrict__ Cbt = g.Cbt;
+  constexpr int KG = 128, LD = kGemmLd;
   const int lane = threadIdx.x, i = lane & 31, kg = lane >> 5;
-  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+  const int m0 = b / g.tiles_n() * 32, n0 = b % g.tiles_n() * 32;
   const int fr = lane >> 4, fc = 8 * (lane & 15);        // fetching: row within four, first column
   const __bf16 *pa[8], *pb[8];
 #pragma unroll
@@ -98,15 +109,15 @@ __global__ __launch_bounds__(64) void k_gemm_nt(int M, int N, int K, const __bf1
       const int m = m0 + 8 * q + 4 * kg + r;
       float x = acc[4 * q + r] + bn;
       if (m < M) {
-        if (gate && !((float)gate[(int64_t)m * ldg + n] > 0.f)) x = 0.f;
-        if (relu) x = x > 0.f ? x : 0.f;
-        if (C) C[(int64_t)m * ldc + n] = x;
-        if (Cb) Cb[(int64_t)m * ldcb + n] = (__bf16)x;
+        if (gate && !((float)gate[(int64_t)m * g.ldg + n] > 0.f)) x = 0.f;
+        if (g.relu) x = x > 0.f ? x : 0.f;
+        if (C) C[(int64_t)m * g.ldc + n] = x;
+        if (Cb) Cb[(int64_t)m * g.ldcb + n] = (__bf16)x;
       }
       t4[r] = (__bf16)x;
     }
     // (M is a multiple of 4 wherever a transposed copy is asked for)
-    if (Cbt && m0 + 8 * q + 4 * kg < M) *(bf16x4 *)(Cbt + (int64_t)n * ldcbt + m0 + 8 * q + 4 * kg) = t4;
+    if (Cbt && m0 + 8 * q + 4 * kg < M) *(bf16x4 *)(Cbt + (int64_t)n * g.ldcbt + m0 + 8 * q + 4 * kg) = t4;
   }
 }
 
@@ -276,29 +287,34 @@ __global__ __launch_bounds__(256) void k_mse_grad(int B, const float *__restrict
 
 // Bias gradient: out[n] = sum_m G[m][n] (FP32 or bf16 rows), rows added in order in FP32: a chain
 // of M dependent adds per column, which bounds it.  A block owns 16 columns (N and ldg are
-// multiples of 16, rows 16-byte aligned): its 256 threads fetch 256 rows at a time with 16-byte
-// loads, one row each, and leave them column by column in LDS, where 16 lanes walk their columns
+// multiples of 16, rows 16-byte aligned): its 64 threads fetch 256 rows at a time with 16-byte
+// loads, four rows each, and leave them column by column in LDS, where 16 lanes walk their columns
 // four rows per read while the next 256 rows are on their way.  One thread per column reading
-// its rows from memory one by one waited for every load: 1024 rows of 256 columns 224 us, here
+// its rows from memory one by one waited for every load: 1024 rows of 256 columns 224 us, so
 // 6.4 us (an epoch of 8192 rows in batches of 1024: 7.2 -> 1.9 ms).  Rows past M enter as +0,
 // which leaves a sum that starts at +0 as it is.
+struct Colsum {
+  int M, N, ldg;
+  const void *G;
+  float *out;
+  __host__ __device__ int tiles() const { return N / 16; }
+};
+constexpr int kColsumLd = 256 + 4, kColsumLds = 16 * kColsumLd * 4;   // 16 lanes x 16-byte reads touch every bank once
 template <typename TG>
-__global__ __launch_bounds__(256) void k_colsum(int M, const TG *__restrict__ G, int ldg, float *__restrict__ out) {
-  constexpr int LD = 256 + 4;                   // 16 lanes x 16-byte reads touch every bank once
-  __shared__ __align__(16) float tile[16 * LD];
+__device__ __forceinline__ void colsum_tile(const Colsum &cs, int b, float *tile) {
+  constexpr int LD = kColsumLd;
   typedef TG v8 __attribute__((ext_vector_type(16 / sizeof(TG))));
   constexpr int NV = 16 * sizeof(TG) / 16;      // 16-byte loads per row
-  const int t = threadIdx.x, n0 = blockIdx.x * 16;
-  v8 pre[NV];
+  const int M = cs.M, ldg = cs.ldg, t = threadIdx.x, n0 = b * 16;
+  const TG *G = (const TG *)cs.G;
+  v8 pre[4][NV];
   auto fetch = [&](int m0) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q)
+    for (int u = 0; u < 4; ++u) {
+      const int m = m0 + 64 * u + t;
+      const v8 *p = (const v8 *)(G + (int64_t)(m < M ? m : M - 1) * ldg + n0);
 #pragma unroll
-      for (int j = 0; j < 16 / NV; ++j) pre[q][j] = (TG)0.f;
-    if (m0 + t < M) {
-      const v8 *p = (const v8 *)(G + (int64_t)(m0 + t) * ldg + n0);
-#pragma unroll
-      for (int q = 0; q < NV; ++q) pre[q] = p[q];
+      for (int q = 0; q < NV; ++q) pre[u][q] = p[q];
     }
   };
   float s = 0.f;
@@ -306,7 +322,12 @@ __global__ __launch_bounds__(256) void k_colsum(int M, const TG *__restrict__ G,
   for (int m0 = 0; m0 < M; m0 += 256) {
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < 16; ++c) tile[c * LD + t] = (float)pre[c / (16 / NV)][c % (16 / NV)];
+    for (int u = 0; u < 4; ++u) {
+      const bool in = m0 + 64 * u + t < M;
+#pragma unroll
+      for (int c = 0; c < 16; ++c)
+        tile[c * LD + 64 * u + t] = in ? (float)pre[u][c / (16 / NV)][c % (16 / NV)] : 0.f;
+    }
     __syncthreads();
     if (m0 + 256 < M) fetch(m0 + 256);
     if (t < 16) {
@@ -321,7 +342,24 @@ __global__ __launch_bounds__(256) void k_colsum(int M, const TG *__restrict__ G,
       }
     }
   }
-  if (t < 16) out[n0 + t] = s;
+  if (t < 16) cs.out[n0 + t] = s;
+}
+
+// One launch for what a step can do at once: the column sums' blocks first (the longest chain),
+// then the tiles of up to two products.  Each fills a part of the chip for 5 to 9 us, so their
+// launches one after the other were half of a backward pass (epoch as above: 1251 -> 987 us).
+template <typename TG>
+__global__ __launch_bounds__(64) void k_layers(Colsum cs, GemmNt g0, GemmNt g1) {
+  __shared__ __align__(16) unsigned char lds[kGemmLds > kColsumLds ? kGemmLds : kColsumLds];
+  int b = blockIdx.x;
+  const int nc = cs.tiles();
+  if (b < nc) {
+    colsum_tile<TG>(cs, b, (float *)lds);
+    return;
+  }
+  b -= nc;
+  if (b < g0.tiles()) gemm_tile(g0, b, (__bf16 *)lds);
+  else gemm_tile(g1, b - g0.tiles(), (__bf16 *)lds);
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 master weights; the bf16 copies of the three weight
@@ -367,11 +405,19 @@ __global__ __launch_bounds__(256) void k_gather(int B, const int *__restrict__ i
 
 }  // namespace
 
-void gemm_nt(hipStream_t s, int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *bias,
-             const void *gate, int ldg, int relu, float *C, int ldc, void *Cb, int ldcb, void *Cbt, int ldcbt) {
-  dim3 grid((N + 31) / 32, (M + 31) / 32);
-  k_gemm_nt<<<grid, 64, 0, s>>>(M, N, K, (const __bf16 *)A, lda, (const __bf16 *)B, ldb, bias, (const __bf16 *)gate,
-                                 ldg, relu, C, ldc, (__bf16 *)Cb, ldcb, (__bf16 *)Cbt, ldcbt);
+namespace {
+GemmNt gemm_args(const LayerProduct &p) {
+  return GemmNt{p.M, p.N, p.K, p.lda, p.ldb, p.ldg, p.relu, p.ldc, p.ldcb, p.ldcbt, (const __bf16 *)p.A,
+                (const __bf16 *)p.B, p.bias, (const __bf16 *)p.gate, p.C, (__bf16 *)p.Cb, (__bf16 *)p.Cbt};
+}
+}  // namespace
+
+void layer_products(hipStream_t s, const LayerProduct &p0, const LayerProduct *p1, const ColumnSums *sums) {
+  const GemmNt g0 = gemm_args(p0), g1 = p1 ? gemm_args(*p1) : GemmNt{};
+  const Colsum cs = sums ? Colsum{sums->M, sums->N, sums->N, sums->G, sums->out} : Colsum{};
+  const unsigned grid = (unsigned)(cs.tiles() + g0.tiles() + g1.tiles());
+  if (sums && sums->f32) k_layers<float><<<grid, 64, 0, s>>>(cs, g0, g1);
+  else k_layers<__bf16><<<grid, 64, 0, s>>>(cs, g0, g1);
 }
 
 void transposes_bf16(hipStream_t s, int n, const TransposeBf16 *m) {
@@ -403,14 +449,6 @@ void warm_select(hipStream_t s, int64_t I, int R, int ldr, const double *V, Nnls
 void mse_grad(hipStream_t s, int B, const float *Y, const float *T, const unsigned char *rank, float inv_count,
               void *dYb, float *dY, double *part, int nparts) {
   k_mse_grad<<<nparts, 256, 0, s>>>(B, Y, T, rank, inv_count, (__bf16 *)dYb, dY, part);
-}
-
-void colsum_f32(hipStream_t s, int M, int N, const float *G, int ldg, float *out) {
-  k_colsum<float><<<N / 16, 256, 0, s>>>(M, G, ldg, out);
-}
-
-void colsum_bf16(hipStream_t s, int M, int N, const void *G, int ldg, float *out) {
-  k_colsum<__bf16><<<N / 16, 256, 0, s>>>(M, (const __bf16 *)G, ldg, out);
 }
 
 void adam_step(hipStream_t s, int64_t n, float *w, const float *g, float *m1, float *m2, float lr, float b1, float b2,

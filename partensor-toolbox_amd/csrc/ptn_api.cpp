@@ -338,12 +338,24 @@ struct MlpState {
   // Y = network(X) for B rows; back (B a multiple of 32): the activations are kept for the
   // backward pass, upright and transposed
   void forward(hipStream_t s, int B, bool back) {
-    gemm_nt(s, B, kMlpH, kMlpIn, X.p, kMlpIn, wb.p + kMlpW1b, kMlpIn, w.p + kMlpB1, nullptr, 0, 1, nullptr, 0, H1.p,
-            kMlpH, back ? H1T.p : nullptr, B);
-    gemm_nt(s, B, kMlpH, kMlpH, H1.p, kMlpH, wb.p + kMlpW2b, kMlpH, w.p + kMlpB2, nullptr, 0, 1, nullptr, 0, H2.p,
-            kMlpH, back ? H2T.p : nullptr, B);
-    gemm_nt(s, B, kMlpR, kMlpH, H2.p, kMlpH, wb.p + kMlpW3b, kMlpH, w.p + kMlpB3, nullptr, 0, 0, Y.p, kMlpR, nullptr,
-            0, nullptr, 0);
+    LayerProduct p1{B, kMlpH, kMlpIn, X.p, kMlpIn, wb.p + kMlpW1b, kMlpIn};
+    p1.bias = w.p + kMlpB1;
+    p1.relu = 1;
+    p1.Cb = H1.p; p1.ldcb = kMlpH;
+    LayerProduct p2{B, kMlpH, kMlpH, H1.p, kMlpH, wb.p + kMlpW2b, kMlpH};
+    p2.bias = w.p + kMlpB2;
+    p2.relu = 1;
+    p2.Cb = H2.p; p2.ldcb = kMlpH;
+    LayerProduct p3{B, kMlpR, kMlpH, H2.p, kMlpH, wb.p + kMlpW3b, kMlpH};
+    p3.bias = w.p + kMlpB3;
+    p3.C = Y.p; p3.ldc = kMlpR;
+    if (back) {
+      p1.Cbt = H1T.p; p1.ldcbt = B;
+      p2.Cbt = H2T.p; p2.ldcbt = B;
+    }
+    layer_products(s, p1, nullptr, nullptr);
+    layer_products(s, p2, nullptr, nullptr);
+    layer_products(s, p3, nullptr, nullptr);
   }
   // gradient of the masked mean squared error into g (after forward(s, B, true)); per-block
   // partial losses in part[0..64)
@@ -354,18 +366,26 @@ struct MlpState {
                                  {kMlpH, kMlpH, wb.p + kMlpW2b, w2t.p},
                                  {kMlpR, kMlpH, wb.p + kMlpW3b, w3t.p}};
     transposes_bf16(s, 4, tr);
-    colsum_f32(s, B, kMlpR, dYf.p, kMlpR, g.p + kMlpB3);
-    gemm_nt(s, kMlpR, kMlpH, B, dYT.p, B, H2T.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW3, kMlpH, nullptr, 0, nullptr, 0);
-    gemm_nt(s, B, kMlpH, kMlpR, dYb.p, kMlpR, w3t.p, kMlpR, nullptr, H2.p, kMlpH, 0, nullptr, 0, dH2.p, kMlpH, dH2T.p,
-            B);
-    colsum_bf16(s, B, kMlpH, dH2.p, kMlpH, g.p + kMlpB2);
-    gemm_nt(s, kMlpH, kMlpH, B, dH2T.p, B, H1T.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW2, kMlpH, nullptr, 0, nullptr,
-            0);
-    gemm_nt(s, B, kMlpH, kMlpH, dH2.p, kMlpH, w2t.p, kMlpH, nullptr, H1.p, kMlpH, 0, nullptr, 0, dH1.p, kMlpH, dH1T.p,
-            B);
-    colsum_bf16(s, B, kMlpH, dH1.p, kMlpH, g.p + kMlpB1);
-    gemm_nt(s, kMlpH, kMlpIn, B, dH1T.p, B, XT.p, B, nullptr, nullptr, 0, 0, g.p + kMlpW1, kMlpIn, nullptr, 0, nullptr,
-            0);
+    auto weights = [&](int M, int N, uint16_t *dT, uint16_t *inT, float *out) {   // (M x N) = dT in
+      LayerProduct p{M, N, B, dT, B, inT, B};
+      p.C = out; p.ldc = N;
+      return p;
+    };
+    auto hidden = [&](int K, uint16_t *d, uint16_t *wt, uint16_t *act, uint16_t *out, uint16_t *outT) {
+      LayerProduct p{B, kMlpH, K, d, K, wt, K};
+      p.gate = act; p.ldg = kMlpH;
+      p.Cb = out; p.ldcb = kMlpH;
+      p.Cbt = outT; p.ldcbt = B;
+      return p;
+    };
+    // each launch: a layer's weight and bias gradients beside the gradient of the layer before it
+    const ColumnSums b3{B, kMlpR, dYf.p, true, g.p + kMlpB3}, b2{B, kMlpH, dH2.p, false, g.p + kMlpB2},
+        b1{B, kMlpH, dH1.p, false, g.p + kMlpB1};
+    const LayerProduct h2 = hidden(kMlpR, dYb.p, w3t.p, H2.p, dH2.p, dH2T.p);
+    layer_products(s, weights(kMlpR, kMlpH, dYT.p, H2T.p, g.p + kMlpW3), &h2, &b3);
+    const LayerProduct h1 = hidden(kMlpH, dH2.p, w2t.p, H1.p, dH1.p, dH1T.p);
+    layer_products(s, weights(kMlpH, kMlpH, dH2T.p, H1T.p, g.p + kMlpW2), &h1, &b2);
+    layer_products(s, weights(kMlpH, kMlpIn, dH1T.p, XT.p, g.p + kMlpW1), nullptr, &b1);
   }
 };
 

@@ -132,8 +132,33 @@ __host__ __device__ inline int64_t mlp_bf16_index(int64_t e) {
   if (e >= kMlpW3 && e < kMlpB3) return e - kMlpW3 + kMlpW3b;
   return -1;
 }
-void gemm_nt(hipStream_t s, int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *bias,
-             const void *gate, int ldg, int relu, float *C, int ldc, void *Cb, int ldcb, void *Cbt, int ldcbt);
+// One product of the network (mlp_kernels.hip): C[m][n] = sum_k A[m][k] B[n][k], bf16 operands with
+// k contiguous; + bias[n], zero where gate[m][n] <= 0, ReLU, as asked; into FP32 C, bf16 Cb and a
+// transposed bf16 Cbt, whichever are given.
+struct LayerProduct {
+  int M, N, K;
+  const void *A;
+  int lda;
+  const void *B;
+  int ldb;
+  const float *bias = nullptr;
+  const void *gate = nullptr;
+  int ldg = 0, relu = 0;
+  float *C = nullptr;
+  int ldc = 0;
+  void *Cb = nullptr;
+  int ldcb = 0;
+  void *Cbt = nullptr;
+  int ldcbt = 0;
+};
+struct ColumnSums {                          // out[n] = sum_m G[m][n], rows of N values, FP32 or bf16
+  int M, N;
+  const void *G;
+  bool f32;
+  float *out;
+};
+// one launch; p1 and sums may be null
+void layer_products(hipStream_t s, const LayerProduct &p0, const LayerProduct *p1, const ColumnSums *sums);
 struct TransposeBf16 {                       // out (cols x rows) = in^T (rows x cols), both contiguous
   int rows, cols;
   const void *in;
@@ -148,8 +173,6 @@ void warm_select(hipStream_t s, int64_t I, int R, int ldr, const double *V, Nnls
                  int *count);
 void mse_grad(hipStream_t s, int B, const float *Y, const float *T, const unsigned char *rank, float inv_count,
               void *dYb, float *dY, double *part, int nparts);
-void colsum_f32(hipStream_t s, int M, int N, const float *G, int ldg, float *out);
-void colsum_bf16(hipStream_t s, int M, int N, const void *G, int ldg, float *out);
 void adam_step(hipStream_t s, int64_t n, float *w, const float *g, float *m1, float *m2, float lr, float b1, float b2,
                float eps, int step, void *wb);
 void weights_bf16(hipStream_t s, int64_t n, const float *w, void *wb);
