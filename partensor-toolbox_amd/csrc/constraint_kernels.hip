@@ -11,6 +11,8 @@ namespace ptn {
 
 namespace {
 
+#include "wave_common.inc"
+
 constexpr double kDblEps = 2.220446049250313e-16;
 
 // LU with partial pivoting (the largest |entry| of the column, first one on ties), then
@@ -76,140 +78,204 @@ __global__ __launch_bounds__(256) void k_lu_inverse(int R, const double *__restr
   for (int e = t; e < R * R; e += 256) Vi[e] = x[e];
 }
 
-__device__ __forceinline__ int rr_slot(int k, int t, int n) { return k == 0 ? 0 : ((k - 1 + t) % (n - 1)) + 1; }
-
 // Parallel-order cyclic Jacobi (Golub & Van Loan 8.5, Brent-Luk round-robin order): each
 // round applies the n/2 disjoint rotations, rows first (J^T A), then columns (A J) and the
 // eigenvector accumulation; a rotation is skipped when |a_pq| <= eps sqrt(|a_pp a_qq|).
 // Up to 60 sweeps, stopping after a sweep without rotations.  evals = diag, Q = vectors.
 //
-// The chain of rounds bounds it (n - 1 rounds a sweep, some 8 sweeps), so a round is made
-// short: lane k of the first wave forms rotation k (its divisions and square roots side by
-// side with the others' instead of one after another on one thread), and a thread applies a
-// round to one 2 x 2 block at a time, the rows of one pair by the columns of another, in
-// registers: rows first, then columns, as before, with no barrier between the two.  Two
-// barriers a round instead of six; R = 24: 1161 -> 199 us.  RB: R rounded up to 16, 32 or 64,
-// so that a thread's blocks are fixed before the loop.
+// The chain of rounds bounds it (n - 1 rounds a sweep, some 8 sweeps), and a round is two halves
+// of some 1000 clocks.  In the first the lanes of a wave of their own form the rotations side by
+// side (divisions and square roots, the short ones where the operands allow); meanwhile the
+// other four waves fetch the round's entries, a 2 x 2 block to a thread, the rows of one pair by the
+// columns of another, and apply the round before to the vectors.  In the second they apply both
+// rotations to their blocks in registers, rows first, with no barrier between the two and no
+// branch on which pairs rotate.  A pair's members move on by one slot a round (the first stays), so
+// no round computes them.  R = 24: 1161 us with one thread's rotations and six barriers a round,
+// 199 with the rotations side by side before the blocks and the vectors, 163 so.  RB: R rounded up
+// to 16, 32 or 64, so that a thread's blocks are fixed before the loop.
 template <int RB>
-__global__ __launch_bounds__(256) void k_jacobi_eig(int R, const double *__restrict__ A, double *__restrict__ evals,
+__global__ __launch_bounds__(320) void k_jacobi_eig(int R, const double *__restrict__ A, double *__restrict__ evals,
                                                     double *__restrict__ Q) {
   __shared__ double a[RB * RB], v[RB * RB];
-  __shared__ double cs[RB / 2], sn[RB / 2];
-  __shared__ int pp[RB / 2], qq[RB / 2];
+  __shared__ double cs[2][RB / 2], sn[2][RB / 2];   // of this round and the last
   __shared__ unsigned long long act;                 // the pairs that rotate this round
   constexpr int NA = (RB / 2 * (RB / 2) + 255) / 256, NV = (RB * (RB / 2) + 255) / 256;
   const int t = threadIdx.x;
   const int n = R + (R & 1), U = n / 2;              // odd R: the pair with index R stands still
-  int ma[NA], mb[NA], vi[NV], vm[NV];                // blocks (row pair, column pair) and (row of v, pair)
-#pragma unroll
-  for (int u = 0; u < NA; ++u) {
-    const int e = t + 256 * u;
-    ma[u] = e < U * U ? e % U : -1;
-    mb[u] = e / U;
-  }
-#pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int e = t + 256 * u;
-    vi[u] = e < R * U ? e % R : -1;
-    vm[u] = e / R;
-  }
-  for (int e = t; e < R * R; e += 256) {
+  // pair k of round r: slots k and n - 1 - k, where slot 0 holds 0 and the others turn
+  struct Pair {
+    int k, x, y;
+    __device__ int p() const { return x < y ? x : y; }
+    __device__ int q() const { return x < y ? y : x; }
+  };
+  auto pair = [&](int k) { return Pair{k, k, n - 1 - k}; };
+  auto turn = [&](Pair &P) {
+    P.x = P.k == 0 ? 0 : P.x == n - 1 ? 1 : P.x + 1;
+    P.y = P.y == n - 1 ? 1 : P.y + 1;
+  };
+  for (int e = t; e < R * R; e += 320) {
     a[e] = A[e];
     v[e] = (e % R == e / R) ? 1.0 : 0.0;
   }
-  for (int sweep = 0; sweep < 60; ++sweep) {
-    bool rotated = false;
-    for (int r = 0; r < n - 1; ++r) {
-      __syncthreads();                               // the last round's blocks are stored
-      if (t < 64) {
-        int p = 0, q = 0;
-        bool on = t < U;
-        double cc = 1.0, ss = 0.0;
-        if (on) {
-          p = rr_slot(t, r, n);
-          q = rr_slot(n - 1 - t, r, n);
-          if (p > q) {
-            const int tmp = p;
-            p = q;
-            q = tmp;
-          }
-          pp[t] = p;
-          qq[t] = q;
-          on = q < R;
+  if (t >= 256) {                                    // the rotations
+    const int l = t - 256;
+    Pair P = pair(l < U ? l : 0);
+    int par = 0;
+    for (int sweep = 0; sweep < 60; ++sweep) {
+      bool rotated = false;
+      for (int r = 0; r < n - 1; ++r) {
+        const int p = P.p(), q = P.q();
+        const bool whole = l < U && q < R;
+        const int qc = q < R ? q : p;
+        __syncthreads();                             // the last round's blocks are stored
+        const double apq = a[p + R * qc], app = a[p + R * p], aqq = a[qc + R * qc];
+        // lanes without a rotation take the numbers of one, so that the wave need not leave the
+        // short operations for them
+        const bool some = whole && apq != 0.0;
+        const double den = some ? 2.0 * apq : 2.0, num = some ? aqq - app : 0.0, pr = some ? fabs(app * aqq) : 1.0;
+        double small, cc, ss;
+        bool plain = !(mid_range(den) && mid_range(pr) && (num == 0.0 || mid_range(num)));
+        const double th = short_quotient(num, den);
+        plain |= !(fabs(th) < 0x1p199);
+        if (!__any(plain)) {
+          small = kDblEps * short_sqrt(pr);
+          double tt = short_quotient(1.0, fabs(th) + short_sqrt(fma(th, th, 1.0)));
+          tt = th < 0.0 ? -tt : tt;
+          cc = short_quotient(1.0, short_sqrt(fma(tt, tt, 1.0)));
+          ss = tt * cc;
+        } else {
+          small = kDblEps * sqrt(pr);
+          const double theta = num / den;
+          double tt = 1.0 / (fabs(theta) + sqrt(fma(theta, theta, 1.0)));
+          if (fabs(theta) > 1e150) tt = 0.5 / theta;
+          else if (theta < 0.0) tt = -tt;
+          cc = 1.0 / sqrt(fma(tt, tt, 1.0));
+          ss = tt * cc;
         }
+        const bool on = whole && !(apq == 0.0 || fabs(apq) <= small);
         if (on) {
-          const double apq = a[p + R * q], app = a[p + R * p], aqq = a[q + R * q];
-          if (apq == 0.0 || fabs(apq) <= kDblEps * sqrt(fabs(app * aqq))) {
-            on = false;
-          } else {
-            const double theta = (aqq - app) / (2.0 * apq);
-            double tt;
-            if (fabs(theta) > 1e150) tt = 0.5 / theta;
-            else {
-              tt = 1.0 / (fabs(theta) + sqrt(fma(theta, theta, 1.0)));
-              if (theta < 0.0) tt = -tt;
-            }
-            cc = 1.0 / sqrt(fma(tt, tt, 1.0));
-            ss = tt * cc;
-            cs[t] = cc;
-            sn[t] = ss;
-          }
+          cs[par][l] = cc;
+          sn[par][l] = ss;
         }
         const unsigned long long m = __ballot(on);
-        if (t == 0) act = m;
+        if (l == 0) act = m;
+        __syncthreads();
+        rotated |= m != 0;
+        turn(P);
+        par ^= 1;
       }
-      __syncthreads();
-      const unsigned long long m = act;
-      if (m == 0) continue;                          // uniform: written again after the next barrier
-      rotated = true;
+      if (!rotated) break;                           // the same in every wave
+    }
+  } else {
+    Pair ra[NA], ca[NA], cv[NV];                     // blocks (row pair, column pair); (row of v, pair)
+    int vi[NV];
 #pragma unroll
-      for (int u = 0; u < NA; ++u) {
-        if (ma[u] < 0) continue;
-        const bool ron = (m >> ma[u]) & 1, con = (m >> mb[u]) & 1;
-        if (!ron && !con) continue;
-        const int p = pp[ma[u]], q = qq[ma[u]], p2 = pp[mb[u]], q2 = qq[mb[u]];
-        const bool hq = q < R, hq2 = q2 < R;         // (a standing pair has one member)
-        double x00 = a[p + R * p2], x10 = hq ? a[q + R * p2] : 0.0;
-        double x01 = hq2 ? a[p + R * q2] : 0.0, x11 = hq && hq2 ? a[q + R * q2] : 0.0;
-        if (ron) {                                   // rows p, q
-          const double c = cs[ma[u]], s = sn[ma[u]];
-          const double y00 = fma(c, x00, -(s * x10)), y10 = fma(s, x00, c * x10);
-          const double y01 = fma(c, x01, -(s * x11)), y11 = fma(s, x01, c * x11);
-          x00 = y00;
-          x10 = y10;
-          x01 = y01;
-          x11 = y11;
-        }
-        if (con) {                                   // columns p2, q2
-          const double c = cs[mb[u]], s = sn[mb[u]];
-          const double y00 = fma(c, x00, -(s * x01)), y01 = fma(s, x00, c * x01);
-          const double y10 = fma(c, x10, -(s * x11)), y11 = fma(s, x10, c * x11);
-          x00 = y00;
-          x10 = y10;
-          x01 = y01;
-          x11 = y11;
-          if (ma[u] == mb[u]) x01 = x10 = 0.0;
-        }
-        a[p + R * p2] = x00;
-        if (hq) a[q + R * p2] = x10;
-        if (hq2) a[p + R * q2] = x01;
-        if (hq && hq2) a[q + R * q2] = x11;
-      }
+    for (int u = 0; u < NA; ++u) {
+      const int e = t + 256 * u;
+      ra[u] = pair(e < U * U ? e % U : 0);
+      ca[u] = pair(e < U * U ? e / U : 0);
+    }
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int e = t + 256 * u;
+      vi[u] = e < R * U ? e % R : -1;
+      cv[u] = pair(e < R * U ? e / R : 0);
+    }
+    // the rotations of round `par`, pairs m, applied to the vectors
+    auto vectors = [&](unsigned long long m, int par) {
 #pragma unroll
       for (int u = 0; u < NV; ++u) {
-        if (vi[u] < 0 || !((m >> vm[u]) & 1)) continue;
-        const int i = vi[u], p = pp[vm[u]], q = qq[vm[u]];
-        const double c = cs[vm[u]], s = sn[vm[u]];
-        const double vx = v[i + R * p], vy = v[i + R * q];
-        v[i + R * p] = fma(c, vx, -(s * vy));
-        v[i + R * q] = fma(s, vx, c * vy);
+        const int k = cv[u].k;
+        if (vi[u] >= 0 && ((m >> k) & 1)) {
+          const int i = vi[u], p = cv[u].p(), q = cv[u].q();
+          const double c = cs[par][k], s = sn[par][k], vx = v[i + R * p], vy = v[i + R * q];
+          v[i + R * p] = fma(c, vx, -(s * vy));
+          v[i + R * q] = fma(s, vx, c * vy);
+        }
+        turn(cv[u]);
       }
+    };
+    unsigned long long last = 0;                     // the pairs of the round before
+    int par = 0;
+    bool first = true;
+    for (int sweep = 0; sweep < 60; ++sweep) {
+      bool rotated = false;
+      for (int r = 0; r < n - 1; ++r) {
+        double x00[NA], x10[NA], x01[NA], x11[NA];
+        int e00[NA], e10[NA], e01[NA], e11[NA];
+        bool hq[NA], hq2[NA];                        // (a standing pair has one member: its other reads it too)
+        __syncthreads();                             // the last round's blocks are stored
+#pragma unroll
+        for (int u = 0; u < NA; ++u) {
+          const int p = ra[u].p(), p2 = ca[u].p();
+          hq[u] = ra[u].q() < R;
+          hq2[u] = ca[u].q() < R;
+          const int q = hq[u] ? ra[u].q() : p, q2 = hq2[u] ? ca[u].q() : p2;
+          e00[u] = p + R * p2;
+          e10[u] = q + R * p2;
+          e01[u] = p + R * q2;
+          e11[u] = q + R * q2;
+          x00[u] = a[e00[u]];
+          x10[u] = a[e10[u]];
+          x01[u] = a[e01[u]];
+          x11[u] = a[e11[u]];
+          turn(ra[u]);
+          turn(ca[u]);
+        }
+        if (!first) vectors(last, par ^ 1);
+        first = false;
+        __syncthreads();
+        const unsigned long long m = act;
+        double cr[NA], sr[NA], cc[NA], sc[NA];
+#pragma unroll
+        for (int u = 0; u < NA; ++u) {
+          cr[u] = cs[par][ra[u].k];
+          sr[u] = sn[par][ra[u].k];
+          cc[u] = cs[par][ca[u].k];
+          sc[u] = sn[par][ca[u].k];
+        }
+        if (m != 0) {
+          rotated = true;
+#pragma unroll
+          for (int u = 0; u < NA; ++u) {
+            if (t + 256 * u >= U * U) continue;
+            const int kr = ra[u].k, kc = ca[u].k;
+            const bool ron = (m >> kr) & 1, con = (m >> kc) & 1;
+            {                                        // rows p, q (a pair that rotates has both)
+              const double c = cr[u], s = sr[u];
+              const double y00 = fma(c, x00[u], -(s * x10[u])), y10 = fma(s, x00[u], c * x10[u]);
+              const double y01 = fma(c, x01[u], -(s * x11[u])), y11 = fma(s, x01[u], c * x11[u]);
+              x00[u] = ron ? y00 : x00[u];
+              x10[u] = ron ? y10 : x10[u];
+              x01[u] = ron ? y01 : x01[u];
+              x11[u] = ron ? y11 : x11[u];
+            }
+            {                                        // columns p2, q2
+              const double c = cc[u], s = sc[u];
+              const double y00 = fma(c, x00[u], -(s * x01[u])), y01 = fma(s, x00[u], c * x01[u]);
+              const double y10 = fma(c, x10[u], -(s * x11[u])), y11 = fma(s, x10[u], c * x11[u]);
+              const bool own = con && kr == kc;      // the rotated pair's own entries: zero
+              x00[u] = con ? y00 : x00[u];
+              x10[u] = own ? 0.0 : con ? y10 : x10[u];
+              x01[u] = own ? 0.0 : con ? y01 : x01[u];
+              x11[u] = con ? y11 : x11[u];
+            }
+            a[e00[u]] = x00[u];
+            if (hq[u]) a[e10[u]] = x10[u];
+            if (hq2[u]) a[e01[u]] = x01[u];
+            if (hq[u] && hq2[u]) a[e11[u]] = x11[u];
+          }
+        }
+        last = m;
+        par ^= 1;
+      }
+      if (!rotated) break;
     }
-    if (!rotated) break;                             // uniform
+    vectors(last, par ^ 1);
   }
   __syncthreads();
-  for (int e = t; e < R * R; e += 256) Q[e] = v[e];
-  for (int i = t; i < R; i += 256) evals[i] = a[i + R * i];
+  for (int e = t; e < R * R; e += 320) Q[e] = v[e];
+  for (int i = t; i < R; i += 320) evals[i] = a[i + R * i];
 }
 
 // T[a][b] = sum_k Q[a][k] sqrt(1 / ev[k]) Q[b][k]  ((M^T M)^{-1/2})
@@ -251,9 +317,9 @@ __global__ void k_params_no_nnls(NnlsParams *p) {
 void lu_inverse(hipStream_t s, int R, const double *V, double *Vi) { k_lu_inverse<<<1, 256, 0, s>>>(R, V, Vi); }
 
 void jacobi_eig(hipStream_t s, int R, const double *A, double *evals, double *Q) {
-  if (R <= 16) k_jacobi_eig<16><<<1, 256, 0, s>>>(R, A, evals, Q);
-  else if (R <= 32) k_jacobi_eig<32><<<1, 256, 0, s>>>(R, A, evals, Q);
-  else k_jacobi_eig<64><<<1, 256, 0, s>>>(R, A, evals, Q);
+  if (R <= 16) k_jacobi_eig<16><<<1, 320, 0, s>>>(R, A, evals, Q);
+  else if (R <= 32) k_jacobi_eig<32><<<1, 320, 0, s>>>(R, A, evals, Q);
+  else k_jacobi_eig<64><<<1, 320, 0, s>>>(R, A, evals, Q);
 }
 
 void inv_sqrt_matrix(hipStream_t s, int R, const double *Q, const double *ev, double *T) {
