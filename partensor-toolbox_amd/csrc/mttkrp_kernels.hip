@@ -346,6 +346,10 @@ __global__ __launch_bounds__(64, NT * S <= 8 ? 2 : 1) void k_gemm_ck_f64(const T
 // contract_rows: block (i, split) sums, for output index i, the rows of T whose
 // remaining digits fall in the split, weighted by the other modes' factor rows.
 // Threads: r = tid % RP, group = tid / RP; groups are summed in LDS in order.
+//
+// A row's digits took two 64-bit divisions each, and the row was waited for before the next
+// one's.  With two other modes (order-4 tensors) the digits are carried along from row to row and
+// four rows are on their way at once (TWO: 190 x 155 x 61 x 24 at rank 12, mode 2, 23.7 -> 12.1 us).
 // ---------------------------------------------------------------------------
 struct RowSpec {
   int nm, outmode;
@@ -354,7 +358,7 @@ struct RowSpec {
   const double *fac[kMaxOrder];
 };
 
-template <typename TT>
+template <typename TT, bool TWO>
 __global__ __launch_bounds__(256) void k_contract_rows(const TT *__restrict__ T, int64_t ldt, RowSpec sp, int RP,
                                                        int ldr, int64_t cchunk, int64_t Cother,
                                                        double *__restrict__ partials, const int *sel,
@@ -366,7 +370,40 @@ __global__ __launch_bounds__(256) void k_contract_rows(const TT *__restrict__ T,
   const int64_t c0 = (int64_t)blockIdx.y * cchunk;
   const int64_t c1 = c0 + cchunk < Cother ? c0 + cchunk : Cother;
   double acc = 0.0;
-  if (grp < ngrp) {
+  if constexpr (TWO) {
+    const int ja = sp.outmode == 0 ? 1 : 0, jb = sp.outmode == 2 ? 1 : 2;
+    const uint32_t Da = sp.dim[ja];
+    const int64_t sa = sp.stride[ja] * ldt, sb = sp.stride[jb] * ldt;
+    const double *fa = sp.fac[ja] + r, *fb = sp.fac[jb] + r;
+    const TT *Ti = T + (int64_t)i * sp.stride[sp.outmode] * ldt + r;
+    if (grp < ngrp && c0 + grp < c1) {
+      uint32_t da = (uint32_t)((uint64_t)(c0 + grp) % Da), db = (uint32_t)((uint64_t)(c0 + grp) / Da);
+      auto advance = [&] {
+        da += ngrp;
+        while (da >= Da) {
+          da -= Da;
+          ++db;
+        }
+      };
+      int64_t n = (c1 - c0 - grp + ngrp - 1) / ngrp;    // the thread's rows
+      for (; n >= 4; n -= 4) {
+        double x[4], wa[4], wb[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          x[u] = (double)Ti[da * sa + db * sb];
+          wa[u] = fa[(int64_t)da * ldr];
+          wb[u] = fb[(int64_t)db * ldr];
+          advance();
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = fma(x[u], wa[u] * wb[u], acc);
+      }
+      for (; n > 0; --n) {
+        acc = fma((double)Ti[da * sa + db * sb], fa[(int64_t)da * ldr] * fb[(int64_t)db * ldr], acc);
+        advance();
+      }
+    }
+  } else if (grp < ngrp) {
     for (int64_t c = c0 + grp; c < c1; c += ngrp) {
       uint64_t rem = (uint64_t)c;
       int64_t row = (int64_t)i * sp.stride[sp.outmode];
@@ -648,8 +685,16 @@ void contract_rows(hipStream_t s, const double *T64, const float *T32, int64_t l
   int RP = ldr;
   int64_t cchunk = (Cother + splits - 1) / splits;
   dim3 grid((unsigned)spec.dim[outmode], (unsigned)splits);
-  if (T64) k_contract_rows<double><<<grid, 256, 0, s>>>(T64, ldt, sp, RP, ldr, cchunk, Cother, partials, sel, sel_off);
-  else     k_contract_rows<float><<<grid, 256, 0, s>>>(T32, ldt, sp, RP, ldr, cchunk, Cother, partials, sel, sel_off);
+#define PTN_CR(TTV, PTR)                                                                                        \
+  do {                                                                                                          \
+    if (spec.nm == 3)                                                                                           \
+      k_contract_rows<TTV, true><<<grid, 256, 0, s>>>(PTR, ldt, sp, RP, ldr, cchunk, Cother, partials, sel, sel_off); \
+    else                                                                                                        \
+      k_contract_rows<TTV, false><<<grid, 256, 0, s>>>(PTR, ldt, sp, RP, ldr, cchunk, Cother, partials, sel, sel_off); \
+  } while (0)
+  if (T64) PTN_CR(double, T64);
+  else PTN_CR(float, T32);
+#undef PTN_CR
 }
 
 void contract2(hipStream_t s, const double *Y64, const float *Y32, int64_t ld, int64_t D0, int64_t D1, int outmode,

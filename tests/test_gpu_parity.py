@@ -432,6 +432,22 @@ def test_mode0_splits(h, I0, K):
         assert P.rel_err(h.mttkrp(A, 0, arith=P.ARITH_F32_F64), o.mttkrp(X32, A, 0)) <= 1e-12
 
 
+@pytest.mark.parametrize("dims", [[5, 1, 7, 3], [4, 2, 1, 9], [3, 1, 1, 1], [6, 17, 5, 2], [2, 3, 40, 33], [9, 64, 3, 70]])
+@pytest.mark.parametrize("R", [3, 16, 17, 33, 64])
+def test_order4_leaf_contractions(h, dims, R):
+    """The row contraction with two other modes about its groups of rows: single and short modes,
+    fewer rows than groups, remainders of four.  FP64 sums of at most 4480 x 9 positive terms in
+    either order (1e-12), FP32 products over a mode of at most 9 (9 x 2^-23 and the data's rounding)."""
+    rng = np.random.default_rng(R + dims[1])
+    X = rng.random(dims)
+    A = [rng.random((d, R)) for d in dims]
+    h.set_tensor(X, storage=P.TENSOR_BOTH)
+    for mode in (1, 2, 3):
+        M = o.mttkrp(X, A, mode)
+        assert P.rel_err(h.mttkrp(A, mode), M) <= 1e-12
+        assert P.rel_err(h.mttkrp(A, mode, arith=P.ARITH_F32), M) <= 2e-6
+
+
 def test_als_c2_full_size_three_sweeps(h):
     """Config 2 at full size (800^3, true rank 32, SNR 20 dB, R = 32, init seed 1): three
     sweeps (the line search runs at sweep 2) of the plain FP64 path, per-mode and tree, against
