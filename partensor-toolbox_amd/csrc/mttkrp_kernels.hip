@@ -29,6 +29,33 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 namespace {
 
+#include "wave_common.inc"
+
+// The set-up of an NNLS update by one wave, as k_eig_extremes<16> does it.  In a kernel of its own
+// it stands in the stream between two contractions and leaves the chip to one block; as one more
+// block of the contraction (template parameter SETUP) it is hidden by, or hides, that: sweeps
+// of 100^3 at rank 10 205 -> 188 us, 301 x 205 x 150 at 10 257 -> 215, order 4 60 x 50 x 40 x 30 at 8
+// 275 -> 246.
+__device__ __forceinline__ void nnls_setup_wave(const NnlsSetup &u) {
+  __shared__ EigLds<16> S;
+  const int l = threadIdx.x & 63;
+  for (int x = l; x < 256; x += 64) {
+    const int r = x / 16, c = x % 16;
+    double v = 0.0;
+    if (r < u.R && c < u.R) {
+      const int e = r * u.R + c;
+      v = u.g[0][e];
+      for (int j = 1; j < u.ng; ++j) v = u.g[j][e] * v;
+      u.V[e] = v;
+    }
+    S.t[x] = v;
+  }
+  PTN_WAVE_SYNC();
+  double amax, amin;
+  eig_extremes_wave(u.R, S, amax, amin);
+  glambda_betas(amax, amin, u.prm, u.max_inner, u.betas);
+}
+
 struct KrArgs {
   int nm;
   uint32_t dim[kMaxOrder];
@@ -52,9 +79,16 @@ __device__ __forceinline__ double ld(const TX *p) { return (double)*p; }
 // gemm_cm: a block owns 64 consecutive rows and one k-chunk; its 4 waves take
 // interleaved k-steps of 4 columns and are summed through LDS at the end.
 // ---------------------------------------------------------------------------
-template <typename TX, int NT>
+template <typename TX, int NT, bool SETUP>
 __global__ __launch_bounds__(256, 2) void k_gemm_cm_f64(const TX *__restrict__ X, int64_t Mrows, int64_t Ktot,
-                                                     KrArgs w, int ldr, int64_t kchunk, double *__restrict__ out) {
+                                                     KrArgs w, int ldr, int64_t kchunk, double *__restrict__ out,
+                                                     NnlsSetup setup) {
+  if constexpr (SETUP) {
+    if (blockIdx.x + 1 == gridDim.x) {
+      if (blockIdx.y == 0 && threadIdx.x < 64) nnls_setup_wave(setup);
+      return;
+    }
+  }
   constexpr int RP = NT * 16;
   __shared__ double red[64 * RP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -215,13 +249,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm_cm_f64(const TX *__restrict__ X
 // the registers of a wave (245 000 fibers 44 against 52 us), 1 below 16 384 (10 000: 5.8 us
 // against 6.2 and 7.9).
 // ---------------------------------------------------------------------------
-template <typename TX, int NT, int S>
+template <typename TX, int NT, int S, bool SETUP>
 __global__ __launch_bounds__(64, NT * S <= 8 ? 2 : 1) void k_gemm_ck_f64(const TX *__restrict__ X, int64_t L,
                                                                          int64_t C, KrArgs w, int ldr,
-                                                                         double *__restrict__ T) {
+                                                                         double *__restrict__ T, NnlsSetup setup) {
+  if (SETUP && blockIdx.x == 0) {
+    nnls_setup_wave(setup);
+    return;
+  }
   const int lane = threadIdx.x;
   const int g = lane >> 4, f = lane & 15;
-  const int64_t cb = (int64_t)blockIdx.x * (16 * S);
+  const int64_t cb = (int64_t)(blockIdx.x - (SETUP ? 1 : 0)) * (16 * S);
 
   f64x4 acc[S][NT];
 #pragma unroll
@@ -631,15 +669,21 @@ __global__ __launch_bounds__(256) void k_reduce_splits_runs(const f64x2 *__restr
 }  // namespace
 
 void gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mrows, int64_t Ktot, const KrSpec &w,
-                 int ldr, int splits, double *out) {
+                 int ldr, int splits, double *out, const NnlsSetup *setup) {
   KrArgs a = to_args(w);
   int64_t kchunk = (Ktot + splits - 1) / splits;
   dim3 grid((unsigned)((Mrows + 63) / 64), (unsigned)splits);
   const int NT = ldr / 16;
+  if (setup) {                                     // ldr = 16
+    grid.x += 1;
+    if (x64) k_gemm_cm_f64<double, 1, true><<<grid, 256, 0, s>>>(x64, Mrows, Ktot, a, ldr, kchunk, out, *setup);
+    else     k_gemm_cm_f64<float, 1, true><<<grid, 256, 0, s>>>(x32, Mrows, Ktot, a, ldr, kchunk, out, *setup);
+    return;
+  }
 #define PTN_CM(NTV)                                                                              \
   if (NT == NTV) {                                                                               \
-    if (x64) k_gemm_cm_f64<double, NTV><<<grid, 256, 0, s>>>(x64, Mrows, Ktot, a, ldr, kchunk, out); \
-    else     k_gemm_cm_f64<float, NTV><<<grid, 256, 0, s>>>(x32, Mrows, Ktot, a, ldr, kchunk, out);  \
+    if (x64) k_gemm_cm_f64<double, NTV, false><<<grid, 256, 0, s>>>(x64, Mrows, Ktot, a, ldr, kchunk, out, {}); \
+    else     k_gemm_cm_f64<float, NTV, false><<<grid, 256, 0, s>>>(x32, Mrows, Ktot, a, ldr, kchunk, out, {});  \
     return;                                                                                      \
   }
   PTN_CM(1) PTN_CM(2) PTN_CM(3) PTN_CM(4)
@@ -647,24 +691,26 @@ void gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mro
 }
 
 void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, int64_t C, const KrSpec &w, int ldr,
-                 double *T) {
+                 double *T, const NnlsSetup *setup) {
   KrArgs a = to_args(w);
   const int NT = ldr / 16;
   // Fibers per wave: many share each Khatri-Rao fragment, few leave more waves for the 1024
   // SIMDs (k_gemm_ck_f64)
   const int S = C >= 65536 && x64 ? 4 : C >= 16384 ? 2 : 1;
-  const unsigned grid = (unsigned)((C + 16 * S - 1) / (16 * S));
-#define PTN_CKS(NTV, SV)                                                          \
-  if (x64) k_gemm_ck_f64<double, NTV, SV><<<grid, 64, 0, s>>>(x64, L, C, a, ldr, T); \
-  else     k_gemm_ck_f64<float, NTV, SV><<<grid, 64, 0, s>>>(x32, L, C, a, ldr, T);
-#define PTN_CK(NTV)              \
+  const unsigned grid = (unsigned)((C + 16 * S - 1) / (16 * S)) + (setup ? 1 : 0);
+  const NnlsSetup none{};
+#define PTN_CKS(NTV, SV, UV)                                                                              \
+  if (x64) k_gemm_ck_f64<double, NTV, SV, UV><<<grid, 64, 0, s>>>(x64, L, C, a, ldr, T, UV ? *setup : none); \
+  else     k_gemm_ck_f64<float, NTV, SV, UV><<<grid, 64, 0, s>>>(x32, L, C, a, ldr, T, UV ? *setup : none);
+#define PTN_CK(NTV, UV)              \
   if (NT == NTV) {               \
-    if (S == 4) { PTN_CKS(NTV, 4) } \
-    else if (S == 2) { PTN_CKS(NTV, 2) } \
-    else { PTN_CKS(NTV, 1) }     \
+    if (S == 4) { PTN_CKS(NTV, 4, UV) } \
+    else if (S == 2) { PTN_CKS(NTV, 2, UV) } \
+    else { PTN_CKS(NTV, 1, UV) }     \
     return;                      \
   }
-  PTN_CK(1) PTN_CK(2) PTN_CK(3) PTN_CK(4)
+  if (setup) { PTN_CK(1, true) }
+  PTN_CK(1, false) PTN_CK(2, false) PTN_CK(3, false) PTN_CK(4, false)
 #undef PTN_CK
 #undef PTN_CKS
 }

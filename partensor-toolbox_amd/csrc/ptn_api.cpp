@@ -436,6 +436,7 @@ struct Work {
     const int *sel = nullptr;
     int64_t sel_off = 0;
   } left, right;                             // dimension-tree nodes cached between the modes of a sweep
+  NnlsSetup setup{};                         // ng > 0: the next FP64 contraction takes it along
   bool left_ready = false;                   // left node already formed for the coming mode 0 (line-search pass)
   bool right_ready = false;                  // order-3 right node X x_0 A_0 already formed (aux stream)
   bool m0_ready = false;                     // mode-0 MTTKRP already in M (paired pass, chosen on the device)
@@ -598,17 +599,21 @@ int pick_splits_cm(const Work &w, int64_t Mrows, int64_t K) {
   return s < 1 ? 1 : (int)s;
 }
 
+// the set-up waiting to be taken along by a contraction that is about to be launched, or null
+struct TakeSetup {
+  NnlsSetup u;
+  explicit TakeSetup(Work &w) : u(w.setup) { w.setup.ng = 0; }
+  const NnlsSetup *get() const { return u.ng ? &u : nullptr; }
+};
+
 Node node_cm(Work &w, const KrSpec &k, int64_t Mrows, int64_t K, int S, double *dst64, float *dst32,
              int timed = -1) {
   ptn_handle h = w.h;
   hipStream_t s = h->stream;
   if (!w.mfma32) {
     w.pass_mark(timed, false, s);
-    if (S == 1) gemm_cm_f64(s, w.x64(), w.x32(), Mrows, K, k, w.ldr, 1, dst64);
-    else {
-      REQUIRE(S * Mrows * w.ldr <= w.part_cap, PTN_ERR_INVALID, "partial buffer too small");
-      gemm_cm_f64(s, w.x64(), w.x32(), Mrows, K, k, w.ldr, S, w.part);
-    }
+    if (S > 1) REQUIRE(S * Mrows * w.ldr <= w.part_cap, PTN_ERR_INVALID, "partial buffer too small");
+    gemm_cm_f64(s, w.x64(), w.x32(), Mrows, K, k, w.ldr, S, S == 1 ? dst64 : w.part.p, TakeSetup(w).get());
     w.pass_mark(timed, true, s);
     if (S > 1) reduce_splits(s, w.part, S, Mrows * w.ldr, dst64, true);
     return Node{dst64, nullptr, w.ldr};
@@ -631,7 +636,7 @@ Node node_ck(Work &w, const KrSpec &k, int64_t L, int64_t C, hipStream_t s = nul
   if (!s) s = h->stream;
   if (!w.mfma32) {
     w.pass_mark(timed, false, s);
-    gemm_ck_f64(s, w.x64(), w.x32(), L, C, k, w.ldr, w.T);
+    gemm_ck_f64(s, w.x64(), w.x32(), L, C, k, w.ldr, w.T, TakeSetup(w).get());
     w.pass_mark(timed, true, s);
     return Node{w.T.p, nullptr, w.ldr};
   }
@@ -700,7 +705,7 @@ void mttkrp_standard(Work &w, double *base, int mode, double *M) {
       // 501 x 403 x 307 at 33 183 and 174; 640^3 at 48 641 us, with 512 blocks 665).
       const int64_t blocks = (I0 + 63) / 64, target = w.total < ((int64_t)1 << 27) ? 512 : 2048;
       const int S = (int)std::max<int64_t>(1, std::min(std::min<int64_t>(target / blocks, 256), Ktot / 32));
-      gemm_cm_f64(w.h->stream, w.x64(), w.x32(), I0, Ktot, k, w.ldr, S, w.part);
+      gemm_cm_f64(w.h->stream, w.x64(), w.x32(), I0, Ktot, k, w.ldr, S, w.part, TakeSetup(w).get());
       reduce_splits(w.h->stream, w.part, S, I0 * w.ldr, M, true);
     } else {
       // FP32 partials summed in FP64 by the row contraction of a 1-digit node per split
@@ -1316,15 +1321,17 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
     // the next sweep.  The aux stream forms the order-3 tree's right node (right_node_early).
     // All three run at the default priority.
     // A hop between the streams costs the host two calls and the device 5 to 10 us of waiting, so
-    // where a mode's contraction is shorter than that and little of the eigen routine everything
-    // stays on one stream.  Sweeps on one / on two, R <= 16: 20^3 160 / 210 us, 64^3 180 / 216,
-    // 100^3 205 / 215, 301 x 205 x 150 (74 MB) 258 / 278, 300^3 (216 MB) 365 / 339; R <= 32, where
-    // the eigen routine takes 50 us, order 3 on the FP64 matrix cores: 64^3 296 / 321, 100^3 (8 MB)
-    // 320 / 326, 150^3 (27 MB) the same, 200^3 (64 MB) 318 / 304, but with the more and longer
-    // kernels of other contractions beside it 64^3 BF16x3 299 / 282, 30^4 437 / 422, FP32 438 / 392;
-    // R > 32 (116 us): 100^3 560 / 549.
+    // where a mode's contraction is shorter than that and little of the eigen routine, or takes the
+    // set-up along as one of its blocks (FP64 contractions, R <= 16), everything stays on one
+    // stream.  Sweeps on one / on two, R <= 16, FP64: 20^3 147 / 210 us, 64^3 168 / 216, 100^3 188 /
+    // 215, 301 x 205 x 150 (74 MB) 215 / 278, 300^3 (216 MB) 298 / 343, 400^3 (512 MB) 580 / 585 and
+    // in the tree 483 / 511, 500 x 500 x 400 (800 MB) 921 / 907; FP32 100^3 253 / 270, 240^3 (55 MB)
+    // the same.  R <= 32, where the eigen routine takes 50 us, order 3 on the FP64 matrix cores:
+    // 64^3 296 / 321, 100^3 (8 MB) 320 / 326, 150^3 (27 MB) the same, 200^3 (64 MB) 318 / 304, but
+    // with the more and longer kernels of other contractions beside it 64^3 BF16x3 299 / 282, 30^4
+    // 437 / 422, FP32 438 / 392; R > 32 (116 us): 100^3 560 / 549.
     const bool early_right = tree && w.mfma32 && N == 3;
-    const int64_t one_bytes = (int64_t)(R <= 16 ? 96 : R <= 32 && N == 3 && !w.mfma32 ? 8 : 0) << 20;
+    const int64_t one_bytes = (int64_t)(R <= 16 ? (w.mfma32 ? 96 : 600) : R <= 32 && N == 3 && !w.mfma32 ? 8 : 0) << 20;
     const bool one_stream = !early_right && w.total * (w.f32 ? 4 : 8) <= one_bytes;
     hipStream_t ms = h->stream, ss = one_stream ? ms : h->side;
     auto fork = [&] {      // side waits for the main stream's work so far
@@ -1389,12 +1396,12 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
       // decision, so it runs on the side stream beside the next pass (Normalize leaves
       // the last factor and its Gram as they are unless it is the weight factor)
       const bool side_cost = step_now && pair && !(o.normalization && !all_orth && wf == last);
-      // A tensor that is read in less time than the eigen routine takes (28, 65 and 150 us at
+      // A tensor that is read in less time than the eigen routine takes (22, 49 and 116 us at
       // the three padded ranks; a contraction reads about 4.5 TB/s): the set-up, then the longer
       // of the two, follows the Gram on the main stream, and the contraction crosses to the side
       // stream and back beside it, so neither hop is waited for.  Sweeps per this and the other
-      // order: 100^3 R = 10 229 / 269 us, 200^3 R = 20 342 / 375, 400^3 R = 64 (512 MB) 1232 /
-      // 1452; 300^3 R = 16 (216 MB) 394 / 387, 400^3 R = 16 635 / 598.
+      // order (with a routine of 28, 65 and 150 us): 200^3 R = 20 342 / 375, 400^3 R = 64 (512 MB)
+      // 1232 / 1452, 100^3 R = 10 229 / 269; 300^3 R = 16 (216 MB) 394 / 387.
       const int64_t eig_bytes = (int64_t)(R <= 16 ? 128 : R <= 32 ? 288 : 640) << 20;
       const bool short_read = !early_right && !one_stream && w.total * (w.f32 ? 4 : 8) <= eig_bytes;
       for (int n = 0; n < N; ++n) {
@@ -1407,7 +1414,19 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
         if (set_up) {
           sel[n] = slot(w, n);
           fork();
-          prep_mode(w, w.grams, n, tree, sel[n], o, eig_first ? ms : ss);
+          // on one stream the set-up of rank <= 16 goes along with the FP64 contraction
+          if (one_stream && !w.mfma32 && R <= 16 && o.constraints[n] == PTN_NONNEGATIVITY) {
+            int list[kMaxOrder];
+            w.setup.ng = v_order(N, n, tree, list);
+            for (int j = 0; j < w.setup.ng; ++j) w.setup.g[j] = w.G(list[j]);
+            w.setup.R = R;
+            w.setup.max_inner = o.max_inner;
+            w.setup.V = sel[n].V;
+            w.setup.prm = sel[n].p;
+            w.setup.betas = sel[n].betas;
+          } else {
+            prep_mode(w, w.grams, n, tree, sel[n], o, eig_first ? ms : ss);
+          }
         }
         if (set_up && eig_first) {
           StreamsSwapped swapped(h);
@@ -1422,6 +1441,11 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
           // waits then pass before the leaf contraction instead of one on each side of it
           if (n == 2 && early_right) join();
           contract();
+          // (a mode that contracts a node formed before has not taken it)
+          if (w.setup.ng) {
+            w.setup.ng = 0;
+            prep_mode(w, w.grams, n, tree, sel[n], o, ms);
+          }
         }
         if (set_up && !(n == 2 && early_right)) join();   // mode 0: joined after the line-search pass
         update_factor(w, n, o, sel[n]);

@@ -205,12 +205,22 @@ void rows_to_factors(hipStream_t s, int N, const int64_t *dims, int R, int ldr, 
 void rows_to_f32(hipStream_t s, int64_t n, const double *src, float *dst);
 
 // ---- MTTKRP building blocks (mttkrp_kernels.hip) ----
+// The set-up of an NNLS update (nnls_setup) for R <= 16, taken along by a contraction as one more
+// block: V from the ng Grams, its constants and momentum coefficients.
+struct NnlsSetup {
+  const double *g[kMaxOrder];
+  int ng, R, max_inner;
+  double *V;
+  NnlsParams *prm;
+  double *betas;
+};
 // out[split][m][r] = sum_{k in split} X[m + Mrows*k] * W(k)[r];  W = Khatri-Rao row of `w`.
 void gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mrows, int64_t Ktot,
-                 const KrSpec &w, int ldr, int splits, double *out);
-// T[c][r] = sum_{a < L} X[a + L*c] * W(a)[r]   for c < C;  W = Khatri-Rao row of `w` (a < 2^32)
+                 const KrSpec &w, int ldr, int splits, double *out, const NnlsSetup *setup = nullptr);
+// T[c][r] = sum_{a < L} X[a + L*c] * W(a)[r]   for c < C;  W = Khatri-Rao row of `w` (a < 2^32).
+// setup (ldr = 16 only): runs beside the contraction
 void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, int64_t C,
-                 const KrSpec &w, int ldr, double *T);
+                 const KrSpec &w, int ldr, double *T, const NnlsSetup *setup = nullptr);
 // out[i][r] (+)= sum over rows t of T whose output digit is i of T[t][r] * prod of the
 // other digits' factor rows.  `t` enumerates spec modes lowest fastest; `outmode` is the
 // position in spec of the output index.  Rows of T are ldt apart; T may be FP64 or FP32.
