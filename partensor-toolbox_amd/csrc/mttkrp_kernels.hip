@@ -598,6 +598,41 @@ __global__ __launch_bounds__(256) void k_contract2_r4(const float *__restrict__ 
   }
 }
 
+// A small FP64 node contracted over one digit, a block to an output row: the columns' threads in
+// 256 / ldr groups, each taking every so many-th row with four in flight, the groups summed in LDS in
+// order.  k_contract2 splits such a node to fill the chip and has the splits summed by another
+// launch, 2 to 5 us of the 6 to 20 that both take (MTTKRP of 200^3 at rank 16 68 -> 64 us, the rule for
+// it in contract_node).
+__global__ __launch_bounds__(256) void k_contract2_rows(const double *__restrict__ Y, int64_t rstride, int64_t ostride,
+                                                        int n, const double *__restrict__ F, int ldr,
+                                                        double *__restrict__ out) {
+  __shared__ double red[256];
+  const int r = threadIdx.x % ldr, g = threadIdx.x / ldr, G = 256 / ldr;
+  const double *y = Y + blockIdx.x * ostride + r, *f = F + r;
+  double acc = 0.0;
+  if (g < G) {
+    int j = g;
+    for (; j + 3 * G < n; j += 4 * G) {
+      double x[4], w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        x[u] = y[(j + u * G) * rstride];
+        w[u] = f[(int64_t)(j + u * G) * ldr];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = fma(x[u], w[u], acc);
+    }
+    for (; j < n; j += G) acc = fma(y[j * rstride], f[(int64_t)j * ldr], acc);
+  }
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  if ((int)threadIdx.x < ldr) {
+    double s = red[threadIdx.x];
+    for (int q = 1; q < G; ++q) s += red[q * ldr + threadIdx.x];
+    out[(int64_t)blockIdx.x * ldr + threadIdx.x] = s;
+  }
+}
+
 __global__ void k_reduce_splits(const double *__restrict__ partials, int splits, int64_t n, double *__restrict__ out) {
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
     double s = 0.0;
@@ -757,6 +792,12 @@ void contract2(hipStream_t s, const double *Y64, const float *Y32, int64_t ld, i
   else
     k_contract2<float><<<grid, 256, 0, s>>>(Y32, ld, D0, D1, outmode, F, ldr, R, slen, part, sel, sel_off, nullptr,
                                             nullptr);
+}
+
+void contract2_rows(hipStream_t s, const double *Y, int64_t ld, int64_t D0, int64_t D1, int outmode, const double *F,
+                    int ldr, double *out) {
+  if (outmode == 0) k_contract2_rows<<<(unsigned)D0, 256, 0, s>>>(Y, D0 * ld, ld, (int)D1, F, ldr, out);
+  else k_contract2_rows<<<(unsigned)D1, 256, 0, s>>>(Y, ld, D0 * ld, (int)D0, F, ldr, out);
 }
 
 void contract2_pair(hipStream_t s, const float *Ya, const float *Yb, int64_t ld, int64_t D0, int64_t D1, int outmode,

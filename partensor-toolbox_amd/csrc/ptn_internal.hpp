@@ -237,6 +237,9 @@ void reduce_splits(hipStream_t s, const double *partials, int splits, int64_t n,
 void contract2(hipStream_t s, const double *Y64, const float *Y32, int64_t ld, int64_t D0, int64_t D1, int outmode,
                const double *F, int ldr, int R, int splits, double *part, const int *sel = nullptr,
                int64_t sel_off = 0);
+// the same of an FP64 node, a block to an output row, straight into out (ldr values a row)
+void contract2_rows(hipStream_t s, const double *Y, int64_t ld, int64_t D0, int64_t D1, int outmode, const double *F,
+                    int ldr, double *out);
 // contract2 of two FP32 nodes of one shape in one launch: part[split][0 / 1][i][ldr] for
 // (Ya, Fa) / (Yb, Fb); reduce_splits over 2 x D_out x ldr then gives both results.
 void contract2_pair(hipStream_t s, const float *Ya, const float *Yb, int64_t ld, int64_t D0, int64_t D1, int outmode,

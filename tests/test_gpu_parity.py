@@ -448,6 +448,23 @@ def test_order4_leaf_contractions(h, dims, R):
         assert P.rel_err(h.mttkrp(A, mode, arith=P.ARITH_F32), M) <= 2e-6
 
 
+@pytest.mark.parametrize("dims", [[3, 1, 1], [3, 7, 512], [3, 7, 513], [3, 513, 7], [2, 255, 300], [2, 256, 300],
+                                  [2, 300, 257], [5, 64, 65]])
+@pytest.mark.parametrize("R", [1, 16, 17, 48, 64])
+def test_leaf_contractions_a_block_to_a_row(h, dims, R):
+    """Order 3, modes 1 and 2: both sides of the rule that gives an FP64 node's output row a block of
+    its own, fewer rows than groups of threads and remainders of their fours.  At most 513 x 5
+    positive FP64 terms in either order (1e-12)."""
+    rng = np.random.default_rng(R + dims[2])
+    X = rng.random(dims)
+    A = [rng.random((d, R)) for d in dims]
+    h.set_tensor(X)
+    for mode in (1, 2):
+        assert P.rel_err(h.mttkrp(A, mode), o.mttkrp(X, A, mode)) <= 1e-12
+    for a, b in zip(h.mttkrp_dimtree(A), [o.mttkrp(X, A, m) for m in range(3)]):
+        assert P.rel_err(a, b) <= 1e-12
+
+
 def test_als_c2_full_size_three_sweeps(h):
     """Config 2 at full size (800^3, true rank 32, SNR 20 dB, R = 32, init seed 1): three
     sweeps (the line search runs at sweep 2) of the plain FP64 path, per-mode and tree, against
