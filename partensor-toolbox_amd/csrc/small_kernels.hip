@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kEigThreads<RB>) void k_eig_extremes(int R, const d
 
 
 
-// One 64-lane wave per factor row; lane r holds column r and keeps column r of
+// One 64-lane wave per factor row; lane r (mod RB) holds column r and keeps column r of
 // Zt = V + lambda I in registers.  Each step the row y is broadcast through LDS and
 // (Y Zt)(i, r) accumulates four interleaved partial sums over k mod 4, combined
 // pairwise, as the CPU restatement does; lanes and k beyond R hold exact zeros, which
@@ -201,6 +201,10 @@ __global__ __launch_bounds__(kEigThreads<RB>) void k_eig_extremes(int R, const d
 // (max |G.Y| <= d1 and min G >= -d2 hold iff they hold entry-wise).  Iterate A_k goes
 // to hist[k]; the common stopping point is selected afterwards.  The momentum
 // coefficients depend only on q and come precomputed (momentum_wave).
+//
+// The chain of steps bounds it, and a step is as long as what a wave issues in it.  With R <= 32 the
+// 64 lanes hold two or four copies of the row, and each copy forms its own two or one of the
+// four partial sums (100 rows at rank 10 15.0 -> 12.5 us, 301 at 24 21.0 -> 16.3; every lane all four).
 template <int RB>
 __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr, const double *__restrict__ V,
                                                       const NnlsParams *__restrict__ prm,
@@ -211,7 +215,10 @@ __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr,
                                                       double *colsum) {
   __shared__ double sbeta[kMaxInner + 1];
   if (blockIdx.x == 0 && (int)threadIdx.x < R) colsum[threadIdx.x] = 0.0;   // summed by k_nnls_select
-  __shared__ double ybuf[4][RB];
+  constexpr int GP = 64 / RB, NC = 4 / GP, NR = RB / 4;   // groups of RB lanes; chains of a group, their length
+  // y, by chain where a group has some of them: y_k at SQ (k mod 4) + SJ (k / 4)
+  constexpr int SQ = RB == 64 ? 1 : NR, SJ = RB == 64 ? 4 : 1;
+  __shared__ __align__(16) double ybuf[4][RB];
   __shared__ unsigned long long wbits[4][4];
   for (int k = threadIdx.x; k < max_inner; k += blockDim.x) sbeta[k] = betas[k];
   __syncthreads();
@@ -221,14 +228,18 @@ __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr,
   if (row < I) {
   const double lambda = prm->lambda, L = prm->L;
   const double invL = 1.0 / L;
-  const bool on = lane < R;
-  const int r = on ? lane : 0;
-  double z[RB];
+  const int c = lane % RB, grp = RB == 64 ? 0 : lane / RB;
+  const bool on = c < R;
+  const int r = on ? c : 0;
+  double z[NC][NR];
 #pragma unroll
-  for (int k = 0; k < RB; ++k) {
-    const double vk = (on && k < R) ? V[k * R + r] : 0.0;
-    z[k] = (k == r && on) ? vk + lambda : vk;
-  }
+  for (int q = 0; q < NC; ++q)
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+      const int k = 4 * j + grp * NC + q;
+      const double vk = (on && k < R) ? V[k * R + r] : 0.0;
+      z[q][j] = (k == r && on) ? vk + lambda : vk;
+    }
   // lanes >= R: zero start, zero column of Zt and zero Wt keep every iterate at +0.
   // The anchor of W~ is always the previous row A; the start is A or the warm start S.
   const double anc = on ? A[row * ldr + r] : 0.0;
@@ -244,13 +255,22 @@ __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr,
     for (int kb = 0; kb < kend; ++kb) {
       const int k = 64 * kw + kb;
       const double beta = sbeta[k];
-      if (lane < RB) ybuf[wave][lane] = y;
+      if (lane < RB) ybuf[wave][SQ * (c & 3) + SJ * (c >> 2)] = y;
       __builtin_amdgcn_wave_barrier();
-      double s4[4] = {0.0, 0.0, 0.0, 0.0};
+      double sq[NC];
 #pragma unroll
-      for (int kk = 0; kk < RB; ++kk) s4[kk & 3] = fma(ybuf[wave][kk], z[kk], s4[kk & 3]);
+      for (int q = 0; q < NC; ++q) sq[q] = 0.0;
+      const double *yb = ybuf[wave] + (RB == 64 ? 0 : grp * NC * NR);
+#pragma unroll
+      for (int j = 0; j < NR; ++j)
+#pragma unroll
+        for (int q = 0; q < NC; ++q) sq[q] = fma(yb[SQ * q + SJ * j], z[q][j], sq[q]);
       __builtin_amdgcn_wave_barrier();
-      const double g = ((s4[0] + s4[1]) + (s4[2] + s4[3])) - wt;
+      double dot;
+      if constexpr (RB == 16) dot = add_other_half<32>(add_other_half<16>(sq[0]));
+      else if constexpr (RB == 32) dot = add_other_half<32>(sq[0] + sq[1]);
+      else dot = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+      const double g = dot - wt;
       const bool fail = on && ((fabs(g * y) > d1) || (g < -d2));
       if (__ballot(fail) == 0ull) m |= 1ull << kb;       // the row passes check k
       // g / L as RN(g / L): reciprocal, then one exact-residual correction (Markstein)

@@ -252,6 +252,20 @@ def test_nesterov_matches_oracle(h, I, R, d):
     assert np.array_equal(Ag, Ao)                          # row arithmetic mirrors the oracle
 
 
+@pytest.mark.parametrize("R", [1, 2, 3, 15, 16, 17, 31, 32, 33])
+def test_nesterov_at_the_edges_of_the_padded_ranks(h, R):
+    # bitwise the oracle's where a wave holds one, two and four copies of a row
+    rng = np.random.default_rng(60 + R)
+    B = rng.random((3 * R, R))
+    for I in (1, 5):
+        W = rng.standard_normal((I, R)) * 4 + 2
+        A0 = rng.random((I, R))
+        Ag, itg, Lg, mug = h.nesterov(B.T @ B, W, A0, 1e-2, 1e-2, 70)
+        Ao, ito, Lo, muo = o.nesterov(B.T @ B, W, A0, 1e-2, 1e-2, 70)
+        assert itg == ito and (Lg, mug) == (Lo, muo)
+        assert np.array_equal(Ag, Ao)
+
+
 @pytest.mark.parametrize("wf", [0, 1, 2, 3])
 def test_normalize_matches_oracle(h, wf):
     """Normalize with the weights loaded on factor wf (Normalize.hpp:92-174): bitwise the
