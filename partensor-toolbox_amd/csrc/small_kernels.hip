@@ -204,7 +204,8 @@ __global__ __launch_bounds__(kEigThreads<RB>) void k_eig_extremes(int R, const d
 //
 // The chain of steps bounds it, and a step is as long as what a wave issues in it.  With R <= 32 the
 // 64 lanes hold two or four copies of the row, and each copy forms its own two or one of the
-// four partial sums (100 rows at rank 10 15.0 -> 12.5 us, 301 at 24 21.0 -> 16.3; every lane all four).
+// four partial sums (all four by every copy: 100 rows at rank 10 15.0 us, so 12.5; 301 at 24 21.0
+// and 16.3).
 template <int RB>
 __global__ __launch_bounds__(256) void k_nnls_iterate(int64_t I, int R, int ldr, const double *__restrict__ V,
                                                       const NnlsParams *__restrict__ prm,
