@@ -676,10 +676,11 @@ void contract_node(Work &w, const Node &nd, const KrSpec &sp, int outmode, doubl
     // An FP64 node takes a block to an output row, without the splits' launch, where a block's rows are
     // few or the blocks fill the chip (MTTKRP through the C entry with splits / so: 37 x 23 x 41 mode 1
     // 48.5 / 44.7 us, 200^3 at R = 16 68 / 64, 300^3 at 48 168 / 165, 400^3 at 64 (82 MB) 353 / 351,
-    // 800^3 at 32 (164 MB) 914 / 916; but 30 rows of 2000 82 / 96).  FP32 nodes keep the order of
-    // their sums.
+    // 800^3 at 32 (164 MB) 914 / 916, 5000 rows of 100 at 5 120 / 109; but 30 rows of 2000 82 / 96).
+    // Up to 96 MB: larger nodes are read for longer than a launch.  FP32 nodes keep the order of their
+    // sums.
     const int64_t Dc = outmode == 0 ? D1 : D0;
-    if (nd.p64 && !nd.sel && (Dc <= 32 * (256 / w.ldr) || (In >= 256 && D0 * D1 * nd.ld * 8 <= (int64_t)96 << 20))) {
+    if (nd.p64 && !nd.sel && D0 * D1 * nd.ld * 8 <= (int64_t)96 << 20 && (Dc <= 32 * (256 / w.ldr) || In >= 256)) {
       contract2_rows(s, nd.p64, nd.ld, D0, D1, outmode, sp.fac[1 - outmode], w.ldr, M);
       return;
     }
