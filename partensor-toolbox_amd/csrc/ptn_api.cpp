@@ -1144,7 +1144,12 @@ ptn_status run(ptn_handle h, const std::function<void()> &fn) {
   if (!h) return PTN_ERR_INVALID;
   struct AtEnd {                             // also on the way out of an error
     ptn_handle h;
-    ~AtEnd() { give_back_spent(h); }
+    bool failed = true;
+    ~AtEnd() {
+      give_back_spent(h);
+      // the runtime keeps an error until it is asked for, and the next call asks
+      if (failed) (void)hipGetLastError();
+    }
   } at_end{h};
   try {
     if (h->stream) {
@@ -1155,6 +1160,7 @@ ptn_status run(ptn_handle h, const std::function<void()> &fn) {
       }
     }
     fn();
+    at_end.failed = false;
     return PTN_OK;
   } catch (const Fail &f) {
     return f.code;
@@ -1760,6 +1766,7 @@ ptn_status run_direct(ptn_handle h, F &&fn) {
     fn();
     return PTN_OK;
   } catch (const Fail &f) {
+    (void)hipGetLastError();                 // (as run() does)
     return f.code;
   } catch (...) {
     h->err = "unexpected exception";

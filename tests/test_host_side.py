@@ -1,0 +1,123 @@
+"""What the library does around its kernels - device memory, streams, waits, the order of its
+launches - on a host model of the HIP runtime (hip_model.c), without a GPU.  Each test runs in a
+process of its own, which loads the model in the runtime's place before the library; kernels do
+nothing there, copies and fills are carried out as late as the streams' rules allow."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+import ptn_hip
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+model = ctypes.CDLL(%r, ctypes.RTLD_GLOBAL)
+model.model_trace.restype = ctypes.c_char_p
+for f in (model.model_in_use, model.model_peak):
+    f.restype = ctypes.c_size_t
+model.model_limit.argtypes = [ctypes.c_size_t]
+for f in (model.model_mallocs, model.model_frees):
+    f.restype = ctypes.c_long
+model.model_fail_after.argtypes = [ctypes.c_long]
+sys.path.insert(0, %r)
+import numpy as np
+import ptn_hip as P
+MB = 1 << 20
+
+def trace():
+    return [model.model_trace(i).decode() for i in range(model.model_trace_size())]
+
+def factors(dims, R):
+    return [np.random.default_rng(I).random((I, R)) for I in dims]
+
+def tensor(h, dims, storage=P.TENSOR_BOTH):
+    # (the model's kernels do nothing: no values, only the memory)
+    h.generate_tensor(list(dims), 3, seed=1, storage=storage)
+"""
+
+
+@pytest.fixture(scope="module")
+def on_model(tmp_path_factory):
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None:
+        pytest.skip("no host C compiler")
+    so = str(tmp_path_factory.mktemp("model") / "libhip_model.so")
+    subprocess.run([cc, "-O1", "-Wall", "-Wextra", "-Werror", "-shared", "-fPIC", "-o", so,
+                    os.path.join(HERE, "hip_model.c"), "-lpthread"], check=True)
+    prelude = PRELUDE % (so, os.path.dirname(ptn_hip.LIB_PATH))
+
+    def run(code):
+        r = subprocess.run([sys.executable, "-c", prelude + textwrap.dedent(code)], capture_output=True, text=True,
+                           timeout=300)
+        assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-4000:]
+        return r.stdout
+
+    return run
+
+
+CALLS = """
+def network_rows(n):
+    return np.zeros((n, P.MLP_IN), np.float32), np.zeros((n, P.MLP_OUT), np.float32), np.full(n, 7, np.uint8)
+
+def calls(h):
+    d3, d4 = (60, 50, 40), (12, 11, 10, 9)
+    kw = dict(max_iter=3, threshold_error=0.0, time_passes=1)    # (timed runs wait for events, not for kernels' stores)
+    tree = dict(kw, mttkrp_form=P.MTTKRP_DIMTREE)
+    return [
+        lambda: h.set_tensor(np.ones(d3), storage=P.TENSOR_BOTH), lambda: h.set_tensor(np.ones(d3), storage=P.TENSOR_F32),
+        lambda: tensor(h, d3), lambda: h.norm_sq(), lambda: h.mttkrp(factors(d3, 5), 0),
+        lambda: h.mttkrp(factors(d3, 40), 1, arith=P.ARITH_BF16X3), lambda: h.mttkrp_dimtree(factors(d3, 20)),
+        lambda: h.cost_explicit(factors(d3, 5)), lambda: h.cpd(5, factors(d3, 5), **kw),
+        lambda: h.cpd(33, factors(d3, 33), constraints=[1, 2, 0], **tree),
+        lambda: h.cpd(20, factors(d3, 20), arith=P.ARITH_F32, fuse_accel=1, **tree),
+        lambda: tensor(h, d4), lambda: h.mttkrp_dimtree(factors(d4, 9), arith=P.ARITH_F32),
+        lambda: h.cpd(9, factors(d4, 9), arith=P.ARITH_BF16X3, fuse_accel=1, **tree),
+        lambda: h.cpd(9, factors(d4, 9), **kw),
+        lambda: h.nesterov(np.eye(6), np.ones((30, 6)), np.ones((30, 6))), lambda: h.sym_extremes(np.eye(6)),
+        lambda: h.mlp_init(1), lambda: h.mlp_set_params(np.zeros(P.MLP_PARAMS, np.float32)), lambda: h.mlp_params(),
+        lambda: h.mlp_forward(np.zeros((3, P.MLP_IN), np.float32)), lambda: h.mlp_data_add(*network_rows(40)),
+        lambda: h.mlp_data_add(*network_rows(90)), lambda: h.mlp_loss_grad(*network_rows(70)),
+        lambda: h.mlp_train(1, batch=32, lr=1e-3, seed=7),
+        lambda: h.cpd(9, factors(d4, 9), mlp_harvest=1, warm_start=1, **kw),
+        lambda: h.batch_generate([(20, 19, 18), (17, 16, 21)], [4, 5], seed=1),
+        lambda: h.batch_init_factors(seed=2), lambda: h.cpd_batch(h.batch_init_factors(seed=2), max_iter=2),
+    ]
+"""
+
+
+FAILING = CALLS + """
+# every call with its allocations failing from the k-th on: yields (call, k) after the failure
+def failing_calls():
+    for i in range(len(calls(None))):
+        for k in (0, 1, 2, 3, 5, 8, 13, 21):
+            with P.Handle(0) as h:
+                cs = calls(h)
+                for j in (2, 11, 17, 21, 26):                  # what the later calls need
+                    if j < i:
+                        cs[j]()
+                model.model_fail_after(k)
+                try:
+                    cs[i]()
+                except P.PtnError as e:
+                    assert e.code == 2, (i, k, e)
+                    model.model_fail_after(-1)
+                    yield cs[i], (i, k)
+                model.model_fail_after(-1)
+"""
+
+
+def test_a_call_that_ran_out_of_memory_does_not_fail_the_next(on_model):
+    """The runtime remembers an error until it is asked for; the next call on the thread must not
+    take it for its own."""
+    on_model(FAILING + textwrap.dedent("""
+        n = 0
+        for c, at in failing_calls():
+            c()
+            n += 1
+        assert n > 50, n
+        """))
