@@ -184,8 +184,9 @@ void pool_give(int device, void *p, size_t bytes) {
 }
 
 // the end of a call: what it has finished with returns to the pool once its streams are idle
-void give_back_spent(ptn_handle h) {
-  if (h->spent.empty()) return;
+// (a failed call may leave work queued that it did not get to wait for)
+void give_back_spent(ptn_handle h, bool failed = false) {
+  if (h->spent.empty() && !failed) return;
   bool idle = true;
   for (hipStream_t s : {h->stream, h->side, h->aux})
     if (s && hipStreamSynchronize(s) != hipSuccess) idle = false;
@@ -327,10 +328,10 @@ struct MlpState {
     DevBuf<float> nt(h, (size_t)nc * kMlpR);
     DevBuf<unsigned char> nr(h, (size_t)nc);
     HIPCHK(hipStreamSynchronize(h->stream));
-    if (n > 0) {
-      HIPCHK(hipMemcpy(nx.p, dx.p, (size_t)n * kMlpIn * 2, hipMemcpyDeviceToDevice));
-      HIPCHK(hipMemcpy(nt.p, dt.p, (size_t)n * kMlpR * 4, hipMemcpyDeviceToDevice));
-      HIPCHK(hipMemcpy(nr.p, drank.p, (size_t)n, hipMemcpyDeviceToDevice));
+    if (n > 0) {                             // (on the handle's stream: the call waits for it before the old set goes)
+      HIPCHK(hipMemcpyAsync(nx.p, dx.p, (size_t)n * kMlpIn * 2, hipMemcpyDeviceToDevice, h->stream));
+      HIPCHK(hipMemcpyAsync(nt.p, dt.p, (size_t)n * kMlpR * 4, hipMemcpyDeviceToDevice, h->stream));
+      HIPCHK(hipMemcpyAsync(nr.p, drank.p, (size_t)n, hipMemcpyDeviceToDevice, h->stream));
     }
     dx.swap(nx); dt.swap(nt); drank.swap(nr);
     cap = nc;
@@ -1146,7 +1147,7 @@ ptn_status run(ptn_handle h, const std::function<void()> &fn) {
     ptn_handle h;
     bool failed = true;
     ~AtEnd() {
-      give_back_spent(h);
+      give_back_spent(h, failed);
       // the runtime keeps an error until it is asked for, and the next call asks
       if (failed) (void)hipGetLastError();
     }
@@ -2473,8 +2474,8 @@ ptn_status ptn_mlp_init(ptn_handle h, uint64_t seed) {
     fill(kMlpW2, (int64_t)kMlpH * kMlpH, kMlpH);
     fill(kMlpW3, (int64_t)kMlpR * kMlpH, kMlpH);
     HIPCHK(hipMemcpy(ms.w.p, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(ms.m1.p, 0, kMlpParams * sizeof(float)));
-    HIPCHK(hipMemset(ms.m2.p, 0, kMlpParams * sizeof(float)));
+    HIPCHK(hipMemsetAsync(ms.m1.p, 0, kMlpParams * sizeof(float), h->stream));
+    HIPCHK(hipMemsetAsync(ms.m2.p, 0, kMlpParams * sizeof(float), h->stream));
     weights_bf16(h->stream, kMlpParams, ms.w.p, ms.wb.p);
     HIPCHK(hipStreamSynchronize(h->stream));
     ms.step = 0;
@@ -2487,8 +2488,8 @@ ptn_status ptn_mlp_set_params(ptn_handle h, const float *params) {
     REQUIRE(params, PTN_ERR_INVALID, "params is null");
     MlpState &ms = mlp_of(h);
     HIPCHK(hipMemcpy(ms.w.p, params, kMlpParams * sizeof(float), hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(ms.m1.p, 0, kMlpParams * sizeof(float)));
-    HIPCHK(hipMemset(ms.m2.p, 0, kMlpParams * sizeof(float)));
+    HIPCHK(hipMemsetAsync(ms.m1.p, 0, kMlpParams * sizeof(float), h->stream));
+    HIPCHK(hipMemsetAsync(ms.m2.p, 0, kMlpParams * sizeof(float), h->stream));
     weights_bf16(h->stream, kMlpParams, ms.w.p, ms.wb.p);
     HIPCHK(hipStreamSynchronize(h->stream));
     ms.step = 0;

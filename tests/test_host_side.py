@@ -83,7 +83,7 @@ def calls(h):
         lambda: h.mlp_forward(np.zeros((3, P.MLP_IN), np.float32)), lambda: h.mlp_data_add(*network_rows(40)),
         lambda: h.mlp_data_add(*network_rows(90)), lambda: h.mlp_loss_grad(*network_rows(70)),
         lambda: h.mlp_train(1, batch=32, lr=1e-3, seed=7),
-        lambda: h.cpd(9, factors(d4, 9), mlp_harvest=1, warm_start=1, **kw),
+        lambda: h.cpd(9, factors(d4, 9), arith=P.ARITH_F32, fuse_accel=1, mlp_harvest=1, warm_start=1, **tree),
         lambda: h.batch_generate([(20, 19, 18), (17, 16, 21)], [4, 5], seed=1),
         lambda: h.batch_init_factors(seed=2), lambda: h.cpd_batch(h.batch_init_factors(seed=2), max_iter=2),
     ]
@@ -91,23 +91,28 @@ def calls(h):
 
 
 FAILING = CALLS + """
-# every call with its allocations failing from the k-th on: yields (call, k) after the failure
+# every call with its allocations failing from the k-th on, for every k: yields (call, (its index, k))
+# after each failure
 def failing_calls():
     for i in range(len(calls(None))):
-        for k in (0, 1, 2, 3, 5, 8, 13, 21):
+        k, failed = 0, True
+        while failed:
             with P.Handle(0) as h:
                 cs = calls(h)
-                for j in (2, 11, 17, 21, 26):                  # what the later calls need
+                for j in (2, 11, 17, 21, 26):                # what the later calls need
                     if j < i:
                         cs[j]()
                 model.model_fail_after(k)
+                failed = False
                 try:
                     cs[i]()
                 except P.PtnError as e:
                     assert e.code == 2, (i, k, e)
-                    model.model_fail_after(-1)
-                    yield cs[i], (i, k)
+                    failed = True
                 model.model_fail_after(-1)
+                if failed:
+                    yield cs[i], (i, k)
+            k += 1
 """
 
 
@@ -119,5 +124,22 @@ def test_a_call_that_ran_out_of_memory_does_not_fail_the_next(on_model):
         for c, at in failing_calls():
             c()
             n += 1
-        assert n > 50, n
+        assert n > 200, n
+        """))
+
+
+def test_no_work_is_left_queued_when_a_call_returns(on_model):
+    """A returned call's memory may go to another handle, so nothing that reads or writes it may
+    still wait in a stream, the null stream included; nor after a call that ran out of memory."""
+    on_model(FAILING + textwrap.dedent("""
+        left = []
+        with P.Handle(0) as h:
+            for i, c in enumerate(calls(h)):
+                c()
+                if model.model_pending():
+                    left.append((i, model.model_pending()))
+        for c, at in failing_calls():
+            if model.model_pending():
+                left.append((at, model.model_pending()))
+        assert not left, left
         """))
