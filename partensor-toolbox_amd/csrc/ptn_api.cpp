@@ -1185,8 +1185,7 @@ void alloc_tensor(ptn_handle h, int N, const int64_t *dims, int storage) {
   REQUIRE(storage >= 1 && storage <= 3, PTN_ERR_INVALID, "storage must be F64, F32 or BOTH");
   check_dims(h, N, dims);
   drop_tensor(h);                             // (the calls that read it have waited for their streams)
-  h->N = N;
-  for (int k = 0; k < N; ++k) h->dims[k] = dims[k];
+  h->N = 0;                                   // no tensor until its memory is there
   h->total = prod(dims, N);
   h->frob_valid = false;
   // kTensorPad zero elements after the tensor: the contiguous-K contractions read whole
@@ -1199,6 +1198,8 @@ void alloc_tensor(ptn_handle h, int N, const int64_t *dims, int storage) {
     HIPCHK(pool_take(h->device, pool_size((h->total + kTensorPad) * sizeof(float)), (void **)&h->x32, &h->x32_bytes));
     HIPCHK(hipMemsetAsync(h->x32 + h->total, 0, kTensorPad * sizeof(float), h->stream));
   }
+  for (int k = 0; k < N; ++k) h->dims[k] = dims[k];
+  h->N = N;
 }
 
 void check_arith(ptn_handle h, int arith) {

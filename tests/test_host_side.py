@@ -143,3 +143,35 @@ def test_no_work_is_left_queued_when_a_call_returns(on_model):
                 left.append((at, model.model_pending()))
         assert not left, left
         """))
+
+
+def test_a_tensor_that_did_not_fit_leaves_none(on_model):
+    """Setting a tensor gives up the one before; when the memory for the new one is not there, the
+    handle has none, and calls that need one say so instead of reading it."""
+    on_model("""
+        for storage in (P.TENSOR_F64, P.TENSOR_F32, P.TENSOR_BOTH):
+            for k in (0, 1, 2):
+                with P.Handle(0) as h:
+                    tensor(h, (20, 10, 5), storage)
+                    dims = h.dims
+                    model.model_fail_after(k)
+                    fits = False
+                    try:
+                        tensor(h, (60, 50, 40), storage)
+                        fits = True
+                    except P.PtnError as e:
+                        assert e.code == 2, e
+                    model.model_fail_after(-1)
+                    if fits:
+                        continue
+                    h.dims = dims
+                    for c in (h.norm_sq, lambda: h.cost_explicit(factors(dims, 3)),
+                              lambda: h.mttkrp(factors(dims, 3), 0), lambda: h.cpd(3, factors(dims, 3), max_iter=1)):
+                        try:
+                            c()
+                            raise AssertionError((storage, k))
+                        except P.PtnError as e:
+                            assert e.code == 5, (storage, k, e)
+                    tensor(h, dims, storage)
+                    h.norm_sq()
+        """)
