@@ -312,6 +312,7 @@ struct MlpState {
     r = (r + 31) / 32 * 32;
     if (r <= rows) return;
     HIPCHK(hipDeviceSynchronize());
+    rows = 0;                                 // (a buffer that does not fit leaves the set incomplete)
     const size_t rin = (size_t)r * kMlpIn, rh = (size_t)r * kMlpH, ro = (size_t)r * kMlpR;
     grow(h, X, rin); grow(h, XT, rin); grow(h, H1, rh); grow(h, H2, rh); grow(h, H1T, rh); grow(h, H2T, rh);
     grow(h, dYb, ro); grow(h, dYT, ro); grow(h, dH1, rh); grow(h, dH1T, rh); grow(h, dH2, rh); grow(h, dH2T, rh);

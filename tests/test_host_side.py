@@ -175,3 +175,27 @@ def test_a_tensor_that_did_not_fit_leaves_none(on_model):
                     tensor(h, dims, storage)
                     h.norm_sq()
         """)
+
+
+def test_activation_buffers_that_did_not_fit_are_taken_again(on_model):
+    """The network's buffers grow by giving up the smaller ones.  When a larger one does not fit, a
+    later call of the old size must not go on with the missing one (the model copies to the address
+    it is given)."""
+    on_model("""
+        for k in range(40):
+            with P.Handle(0) as h:
+                h.mlp_init(1)
+                h.mlp_forward(np.zeros((3, P.MLP_IN), np.float32))
+                model.model_fail_after(k)
+                failed = False
+                try:
+                    h.mlp_forward(np.zeros((3000, P.MLP_IN), np.float32))
+                except P.PtnError as e:
+                    assert e.code == 2, e
+                    failed = True
+                model.model_fail_after(-1)
+                h.mlp_forward(np.zeros((3, P.MLP_IN), np.float32))
+                if not failed:
+                    assert k > 10
+                    break
+        """)
