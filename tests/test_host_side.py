@@ -199,3 +199,37 @@ def test_activation_buffers_that_did_not_fit_are_taken_again(on_model):
                     assert k > 10
                     break
         """)
+
+
+def test_a_tensor_given_up_is_given_back(on_model):
+    """Setting another tensor, or another storage, returns the old one's memory to the device at once,
+    a tensor of the same size takes it over, and the work buffers kept between calls stay."""
+    on_model("""
+        big, small = (1000, 800, 600), (30, 20, 10)
+        nb, ns = 480000000, 6000
+        with P.Handle(0) as h:
+            tensor(h, small)
+            none = model.model_in_use()
+            tensor(h, big)
+            full = model.model_in_use()
+            assert full > none + 12 * (nb - ns)
+            mallocs = model.model_mallocs()
+            tensor(h, big)
+            tensor(h, (800, 1000, 600))
+            assert (model.model_mallocs(), model.model_in_use()) == (mallocs, full)
+            tensor(h, big, P.TENSOR_F32)
+            assert model.model_in_use() <= full - 8 * nb
+            tensor(h, small)
+            assert model.model_in_use() < none + MB, (model.model_in_use(), none)
+            h.mttkrp(factors(small, 5), 0)                   # work buffers
+            tensor(h, big)
+            h.mttkrp(factors(big, 5), 0)
+            tensor(h, small)
+            mallocs, used = model.model_mallocs(), model.model_in_use()
+            assert used < none + 6000 * MB, used
+            h.mttkrp(factors(small, 5), 0)
+            tensor(h, big)
+            h.mttkrp(factors(big, 5), 0)
+            assert model.model_mallocs() == mallocs + 2      # the two copies of the tensor
+        assert model.model_in_use() == 0
+        """)
