@@ -1231,10 +1231,14 @@ ptn_status ptn_set_tensor(ptn_handle h, int N, const int64_t *dims, const double
       HIPCHK(hipMemcpyAsync(h->x64, X, h->total * sizeof(double), hipMemcpyHostToDevice, h->stream));
       if (h->x32) cast_f64_to_f32(h->stream, h->total, h->x64, h->x32);
     } else {
-      DevBuf<double> tmp(h, h->total, kRaw);
-      HIPCHK(hipMemcpyAsync(tmp.p, X, h->total * sizeof(double), hipMemcpyHostToDevice, h->stream));
-      cast_f64_to_f32(h->stream, h->total, tmp.p, h->x32);
-      HIPCHK(hipStreamSynchronize(h->stream));
+      // through a buffer of at most 64 MB (the pool keeps it), the copies and casts in stream order
+      const int64_t part = std::min<int64_t>(h->total, (int64_t)8 << 20);
+      DevBuf<double> tmp(h, part, kRaw);
+      for (int64_t e = 0; e < h->total; e += part) {
+        const int64_t n = std::min(part, h->total - e);
+        HIPCHK(hipMemcpyAsync(tmp.p, X + e, n * sizeof(double), hipMemcpyHostToDevice, h->stream));
+        cast_f64_to_f32(h->stream, n, tmp.p, h->x32 + e);
+      }
     }
     HIPCHK(hipStreamSynchronize(h->stream));
   });

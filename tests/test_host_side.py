@@ -233,3 +233,18 @@ def test_a_tensor_given_up_is_given_back(on_model):
             assert model.model_mallocs() == mallocs + 2      # the two copies of the tensor
         assert model.model_in_use() == 0
         """)
+
+
+def test_an_fp32_tensor_is_not_staged_whole(on_model):
+    """FP64 host data for an FP32 tensor passes through a buffer of a bounded size, which is what stays
+    in the pool of work buffers afterwards."""
+    on_model("""
+        with P.Handle(0) as h:
+            before = model.model_in_use()
+            X = np.zeros((300, 300, 333), order="F")         # 240 MB, 120 MB in FP32
+            h.set_tensor(X, storage=P.TENSOR_F32)
+            assert model.model_peak() <= before + X.size * 4 + 80 * MB, model.model_peak()
+            copies = [int(t.split("bytes=")[1].split()[0]) for t in trace() if t.startswith("copy kind=1")]
+            casts = [t for t in trace() if "k_cast" in t]
+            assert sum(copies) == 8 * X.size and len(casts) == len(copies) > 1
+        """)
