@@ -132,23 +132,38 @@ void pool_trim(DevicePool &P, size_t keep) {
   P.blocks.erase(P.blocks.begin(), P.blocks.begin() + (std::ptrdiff_t)n);
 }
 
-// hipMalloc that gives the pool's memory back before it reports that there is none
-hipError_t device_malloc(int device, void **p, size_t bytes) {
+// the handle's three streams have finished what was queued
+bool wait_for_streams(ptn_handle h) {
+  bool idle = true;
+  for (hipStream_t s : {h->stream, h->side, h->aux})
+    if (s && hipStreamSynchronize(s) != hipSuccess) idle = false;
+  return idle;
+}
+
+// hipMalloc that, before it reports that there is no memory, gives back the pool's and then what
+// the handle's call has finished with
+hipError_t device_malloc(ptn_handle h, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   (void)hipGetLastError();
-  DevicePool &P = pools[device];
+  DevicePool &P = pools[h->device];
   {
     std::lock_guard<std::mutex> lock(P.mu);
     pool_trim(P, 0);
   }
+  e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || h->spent.empty()) return e;
+  (void)hipGetLastError();
+  (void)wait_for_streams(h);
+  for (const auto &b : h->spent) (void)hipFree(b.first);
+  h->spent.clear();
   return hipMalloc(p, bytes);
 }
 
 // a block of at least `size` (a pool_size) bytes; a larger one serves while less than a
 // quarter of it would lie idle
-hipError_t pool_take(int device, size_t size, void **p, size_t *got) {
-  DevicePool &P = pools[device];
+hipError_t pool_take(ptn_handle h, size_t size, void **p, size_t *got) {
+  DevicePool &P = pools[h->device];
   {
     std::lock_guard<std::mutex> lock(P.mu);
     size_t best = P.blocks.size();
@@ -165,7 +180,7 @@ hipError_t pool_take(int device, size_t size, void **p, size_t *got) {
     }
   }
   *got = size;
-  return device_malloc(device, p, size);
+  return device_malloc(h, p, size);
 }
 
 void pool_give(int device, void *p, size_t bytes) {
@@ -187,9 +202,7 @@ void pool_give(int device, void *p, size_t bytes) {
 // (a failed call may leave work queued that it did not get to wait for)
 void give_back_spent(ptn_handle h, bool failed = false) {
   if (h->spent.empty() && !failed) return;
-  bool idle = true;
-  for (hipStream_t s : {h->stream, h->side, h->aux})
-    if (s && hipStreamSynchronize(s) != hipSuccess) idle = false;
+  const bool idle = wait_for_streams(h);
   for (const auto &b : h->spent) {
     if (idle) pool_give(h->device, b.first, b.second);
     else (void)hipFree(b.first);
@@ -219,7 +232,7 @@ struct DevBuf {
     h = hh;
     n = count ? count : 1;
     h->spent.reserve(h->spent.size() + 64);  // the destructor's push does not allocate
-    HIPCHK(pool_take(h->device, pool_size(n * sizeof(T)), (void **)&p, &bytes));
+    HIPCHK(pool_take(h, pool_size(n * sizeof(T)), (void **)&p, &bytes));
     if (fill == kZero) HIPCHK(hipMemsetAsync(p, 0, n * sizeof(T), h->stream));
   }
   ~DevBuf() {
@@ -453,7 +466,7 @@ struct Work {
     if (end) kev_used[tslot][q] = true;
   }
 
-  Work(ptn_handle hh, int R_, int arith_, bool need_tree)
+  Work(ptn_handle hh, int R_, int arith_, bool need_tree, bool pair = false)
       : h(hh), N(hh->N), R(R_), ldr(round_up16(R_)), rpf((R_ + 31) / 32 * 32), arith(arith_) {
     f32 = arith != PTN_ARITH_F64;
     mfma32 = arith == PTN_ARITH_F32 || arith == PTN_ARITH_BF16X3;
@@ -489,23 +502,16 @@ struct Work {
       if (need_tree) YL.alloc(h, yl * ldr, kRaw);
     } else {
       part32_cap = 256 * dims[0] * rpf;
-      if (need_tree && N >= 4) part32_cap = std::max<int64_t>(part32_cap, 64 * yl * rpf);
+      if (need_tree && N >= 4) part32_cap = std::max<int64_t>(part32_cap, 64 * yl * (pair ? 2 : 1) * rpf);
       part32.alloc(h, part32_cap, kRaw);
       T32.alloc(h, std::max(C, dims[0]) * rpf, kRaw);
       if (need_tree) YL32.alloc(h, yl * rpf, kRaw);
+      if (pair) {                            // the paired left-node pass
+        YL2.alloc(h, yl * 2 * rpf, kRaw);
+        M2.alloc(h, 2 * dims[0] * ldr, kRaw);        // [Mhat | M] of mode 0
+      }
     }
     part.alloc(h, part_cap, kRaw);
-  }
-  // buffers of the paired left-node pass (dimension tree, FP32-output contractions)
-  void enable_pair() {
-    const int64_t yl = left_rows();
-    YL2.alloc(h, yl * 2 * rpf, kRaw);
-    M2.alloc(h, 2 * dims[0] * ldr, kRaw);          // [Mhat | M] of mode 0 from the paired pass
-    if (N >= 4 && 64 * yl * 2 * rpf > part32_cap) {
-      part32.~DevBuf(); new (&part32) DevBuf<float>();
-      part32_cap = 64 * yl * 2 * rpf;
-      part32.alloc(h, part32_cap, kRaw);
-    }
   }
   // the tree's root splits at half = ceil(N / 2) (DIM_HALF_SIZE, DimTrees.hpp:274): the left
   // node holds modes [0, half), the right node modes [half, N)
@@ -1199,12 +1205,12 @@ void alloc_tensor(ptn_handle h, int N, const int64_t *dims, int storage) {
   // kTensorPad zero elements after the tensor: the contiguous-K contractions read whole
   // 32-element steps, which may run past the end of the last fiber
   if (storage & PTN_TENSOR_F64) {
-    if (!h->x64) HIPCHK(device_malloc(h->device, (void **)&h->x64, b64));
+    if (!h->x64) HIPCHK(device_malloc(h, (void **)&h->x64, b64));
     h->x64_bytes = b64;
     HIPCHK(hipMemsetAsync(h->x64 + h->total, 0, kTensorPad * sizeof(double), h->stream));
   }
   if (storage & PTN_TENSOR_F32) {
-    if (!h->x32) HIPCHK(device_malloc(h->device, (void **)&h->x32, b32));
+    if (!h->x32) HIPCHK(device_malloc(h, (void **)&h->x32, b32));
     h->x32_bytes = b32;
     HIPCHK(hipMemsetAsync(h->x32 + h->total, 0, kTensorPad * sizeof(float), h->stream));
   }
@@ -1314,7 +1320,7 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
     REQUIRE(o.warm_refine >= 0 && o.warm_refine <= o.max_inner, PTN_ERR_INVALID,
             "warm_refine must be in 0 .. max_inner");
 
-    Work w(h, R, o.arith, tree);
+    Work w(h, R, o.arith, tree, pair && o.acceleration);
     if (o.warm_start || o.mlp_harvest) {
       MlpState &mst = mlp_of(h);
       mst.ensure_rows((int)w.maxI);
@@ -1324,7 +1330,6 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
         mst.ensure_data(mst.n + per * o.max_iter);
       }
     }
-    if (pair && o.acceleration) w.enable_pair();
     const int N = w.N, last = N - 1;
     HIPCHK(hipMemsetAsync(w.prm.p, 0, w.prm.n * sizeof(NnlsParams), h->stream));
     upload_factors(w, init_packed, w.fac);
@@ -2023,7 +2028,7 @@ void batch_layout(ptn_handle h, int nprob, const int *dims, const int *ranks) {
   b->nx = xo;
   b->nrows = fo;
   // three copies: mode 0 fastest (the tensors as given), mode 1 fastest, mode 2 fastest
-  HIPCHK(device_malloc(h->device, (void **)&b->x32, 3 * xo * sizeof(float)));
+  HIPCHK(device_malloc(h, (void **)&b->x32, 3 * xo * sizeof(float)));
   HIPCHK(hipMemsetAsync(b->x32, 0, 3 * xo * sizeof(float), h->stream));
   delete h->batch;
   h->batch = b.release();

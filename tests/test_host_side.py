@@ -248,3 +248,39 @@ def test_an_fp32_tensor_is_not_staged_whole(on_model):
             casts = [t for t in trace() if "k_cast" in t]
             assert sum(copies) == 8 * X.size and len(casts) == len(copies) > 1
         """)
+
+
+def test_a_call_needs_no_memory_for_what_it_has_replaced(on_model):
+    """A buffer that a call replaces by a larger one is kept until the call's work is done with it, but
+    not when its memory is needed: with room for the larger buffers alone the call still runs.  The
+    paired line search of order 4 takes its larger partial sums at once."""
+    on_model("""
+        def rows(n):
+            return np.zeros((n, P.MLP_IN), np.float32)
+        with P.Handle(0) as h:
+            h.mlp_init(1)
+            h.mlp_forward(rows(8000))
+            need = model.model_in_use()
+        with P.Handle(0) as h:
+            h.mlp_init(1)
+            h.mlp_forward(rows(6000))
+            model.model_limit(need + MB)
+            h.mlp_forward(rows(8000))
+            model.model_limit(1 << 62)
+            assert model.model_pending() == 0
+
+        # partial sums of 64 splits of (I0 I1) rows of 64 (paired: 128) floats
+        dims, R = (200, 200, 20, 20), 64
+        kw = dict(max_iter=3, threshold_error=0.0, time_passes=1, mttkrp_form=P.MTTKRP_DIMTREE, arith=P.ARITH_F32)
+        part = 64 * 200 * 200 * 64 * 4
+        peak = []
+        for fuse in (0, 1):
+            with P.Handle(0) as h:
+                tensor(h, dims, P.TENSOR_F32)
+                model.model_reset_peak()
+                h.cpd(R, factors(dims, R), fuse_accel=fuse, **kw)
+                peak.append(model.model_peak())
+        # paired: twice the partial sums, the pair of left nodes (as large as 2 of the 64 splits), the
+        # pair of mode-0 results and the packed operand for both
+        assert peak[1] - peak[0] < part + part // 32 + 40 * MB, [p // MB for p in peak]
+        """)
