@@ -160,26 +160,20 @@ hipError_t device_malloc(ptn_handle h, void **p, size_t bytes) {
   return hipMalloc(p, bytes);
 }
 
-// a block of at least `size` (a pool_size) bytes; a larger one serves while less than a
-// quarter of it would lie idle
-hipError_t pool_take(ptn_handle h, size_t size, void **p, size_t *got) {
+// a block of `size` (a pool_size) bytes.  A larger one would serve, but its idle part would be
+// missing near the limit of the memory, where a call that fits by itself must still run
+hipError_t pool_take(ptn_handle h, size_t size, void **p) {
   DevicePool &P = pools[h->device];
   {
     std::lock_guard<std::mutex> lock(P.mu);
-    size_t best = P.blocks.size();
-    for (size_t i = 0; i < P.blocks.size(); ++i) {
-      const size_t b = P.blocks[i].second;
-      if (b >= size && b - size <= b / 4 && (best == P.blocks.size() || b < P.blocks[best].second)) best = i;
-    }
-    if (best < P.blocks.size()) {
-      *p = P.blocks[best].first;
-      *got = P.blocks[best].second;
-      P.held -= *got;
-      P.blocks.erase(P.blocks.begin() + (std::ptrdiff_t)best);
-      return hipSuccess;
-    }
+    for (size_t i = 0; i < P.blocks.size(); ++i)
+      if (P.blocks[i].second == size) {
+        *p = P.blocks[i].first;
+        P.held -= size;
+        P.blocks.erase(P.blocks.begin() + (std::ptrdiff_t)i);
+        return hipSuccess;
+      }
   }
-  *got = size;
   return device_malloc(h, p, size);
 }
 
@@ -232,7 +226,8 @@ struct DevBuf {
     h = hh;
     n = count ? count : 1;
     h->spent.reserve(h->spent.size() + 64);  // the destructor's push does not allocate
-    HIPCHK(pool_take(h, pool_size(n * sizeof(T)), (void **)&p, &bytes));
+    bytes = pool_size(n * sizeof(T));
+    HIPCHK(pool_take(h, bytes, (void **)&p));
     if (fill == kZero) HIPCHK(hipMemsetAsync(p, 0, n * sizeof(T), h->stream));
   }
   ~DevBuf() {

@@ -284,3 +284,22 @@ def test_a_call_needs_no_memory_for_what_it_has_replaced(on_model):
         # pair of mode-0 results and the packed operand for both
         assert peak[1] - peak[0] < part + part // 32 + 40 * MB, [p // MB for p in peak]
         """)
+
+
+def test_blocks_of_other_calls_do_not_crowd_out_a_call(on_model):
+    """A call that fits the memory by itself fits after larger calls too: it does not hold their larger
+    blocks in the place of its own."""
+    on_model("""
+        dims, R = (40, 1500, 1500), 20
+        with P.Handle(0) as h:
+            tensor(h, dims)
+            h.mttkrp(factors(dims, R), 1)
+            need = model.model_peak()
+        larger = (40, 1600, 1800)
+        with P.Handle(0) as h:
+            tensor(h, larger)
+            h.mttkrp(factors(larger, R), 1)
+            tensor(h, dims)
+            model.model_limit(need + MB)
+            h.mttkrp(factors(dims, R), 1)
+        """)
