@@ -121,15 +121,20 @@ size_t pool_size(size_t bytes) {
   return s;
 }
 
-// frees the oldest blocks until at most `keep` bytes are held
+// frees the oldest blocks until at most `keep` bytes are held, one at a time and with the pool
+// unlocked: hipFree waits for the device, and the other handles' calls need not
 void pool_trim(DevicePool &P, size_t keep) {
-  size_t n = 0;
-  while (n < P.blocks.size() && P.held > keep) {
-    (void)hipFree(P.blocks[n].first);
-    P.held -= P.blocks[n].second;
-    ++n;
+  for (;;) {
+    void *p = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(P.mu);
+      if (P.held <= keep) return;
+      p = P.blocks.front().first;
+      P.held -= P.blocks.front().second;
+      P.blocks.erase(P.blocks.begin());
+    }
+    (void)hipFree(p);
   }
-  P.blocks.erase(P.blocks.begin(), P.blocks.begin() + (std::ptrdiff_t)n);
 }
 
 // the handle's three streams have finished what was queued
@@ -146,11 +151,7 @@ hipError_t device_malloc(ptn_handle h, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   (void)hipGetLastError();
-  DevicePool &P = pools[h->device];
-  {
-    std::lock_guard<std::mutex> lock(P.mu);
-    pool_trim(P, 0);
-  }
+  pool_trim(pools[h->device], 0);
   e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory || h->spent.empty()) return e;
   (void)hipGetLastError();
@@ -179,14 +180,16 @@ hipError_t pool_take(ptn_handle h, size_t size, void **p) {
 
 void pool_give(int device, void *p, size_t bytes) {
   DevicePool &P = pools[device];
-  std::lock_guard<std::mutex> lock(P.mu);
-  if (bytes <= kPoolMax) {
+  while (bytes <= kPoolMax) {
     pool_trim(P, kPoolMax - bytes);
+    std::lock_guard<std::mutex> lock(P.mu);
+    if (P.held > kPoolMax - bytes) continue;   // (another call gave a block back meanwhile)
     try {
       P.blocks.emplace_back(p, bytes);
       P.held += bytes;
       return;
     } catch (const std::bad_alloc &) {
+      break;
     }
   }
   (void)hipFree(p);
@@ -1124,8 +1127,12 @@ void ptn_destroy(ptn_handle h) {
     if (r) (void)hipHostFree(r);
   if (h->pooled) {
     DevicePool &P = pools[h->device];
-    std::lock_guard<std::mutex> lock(P.mu);
-    if (--P.handles == 0) pool_trim(P, 0);
+    bool last;
+    {
+      std::lock_guard<std::mutex> lock(P.mu);
+      last = --P.handles == 0;
+    }
+    if (last) pool_trim(P, 0);
   }
   if (h->scal) (void)hipFree(h->scal);
   if (h->part) (void)hipFree(h->part);

@@ -159,7 +159,10 @@ int hipFree(void *p) {
     hold_free = 2;
     struct timespec t = {0, 1000000};
     nanosleep(&t, NULL);
-    if (ms == 1999) free_timed_out = 1;
+    if (ms == 1999) {
+      free_timed_out = 1;
+      hold_free = 0;
+    }
   }
   pthread_mutex_lock(&mu);
   drain_all();                                /* hipFree waits for the device */

@@ -303,3 +303,30 @@ def test_blocks_of_other_calls_do_not_crowd_out_a_call(on_model):
             model.model_limit(need + MB)
             h.mttkrp(factors(dims, R), 1)
         """)
+
+
+def test_freeing_blocks_does_not_stop_other_handles(on_model):
+    """hipFree waits for the device.  While one handle's call frees blocks of the pool, another handle's
+    calls go on (the model holds the hipFree until they have, or two seconds)."""
+    on_model("""
+        import threading
+        dims = (30, 20, 10)
+        a, b = P.Handle(0), P.Handle(0)
+        tensor(a, dims)
+        tensor(b, dims)
+        b.mttkrp(factors(dims, 5), 0)
+        big = (4000, 3000, 2)                                # work buffers beyond what the pool keeps
+        tensor(a, big, P.TENSOR_F64)
+        a.mttkrp(factors(big, 5), 0)
+        model.model_limit(model.model_in_use() + 40 * MB)
+        model.model_hold_free(1)
+        t = threading.Thread(target=lambda: a.nesterov(np.eye(60), np.ones((3000, 60)), np.ones((3000, 60))))
+        t.start()                                            # finds no memory: the pool is emptied
+        while not model.model_free_held():
+            assert t.is_alive() or model.model_free_timed_out()
+        b.mttkrp(factors(dims, 5), 1)
+        b.sym_extremes(np.eye(5))
+        assert not model.model_free_timed_out()
+        model.model_hold_free(0)
+        t.join()
+        """)
