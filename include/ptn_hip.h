@@ -5,8 +5,9 @@
  * Layouts are the reference's (Tensor.hpp:42,63-64): tensors column-major with
  * mode 0 fastest, factors I_n x R column-major, "packed" factor buffers =
  * factor 0, factor 1, ... back to back.  Host buffers stay owned by the caller;
- * a handle owns all device memory and streams and is used by one host thread
- * at a time (handles are independent of each other).
+ * a handle owns its tensor, its network and its streams and is used by one host
+ * thread at a time (handles are independent of each other; those of one GPU share
+ * a pool of work buffers, ptn_release_memory).
  */
 #ifndef PTN_HIP_H
 #define PTN_HIP_H
@@ -102,6 +103,12 @@ typedef struct {
 /* ---- handle ---- */
 ptn_status  ptn_create(ptn_handle *h, int device);
 void        ptn_destroy(ptn_handle h);
+/* Work buffers of finished calls stay on the device for the next calls of any handle of the same
+   GPU, at most 8 GiB of them, until the GPU's last handle is destroyed or an allocation of this
+   library finds no memory.  This gives them back at once (for another allocator in the process);
+   tensors, networks and training sets stay.  It may be called at any time between a handle's
+   calls, also while other handles' calls run. */
+ptn_status  ptn_release_memory(ptn_handle h);
 const char *ptn_last_error(ptn_handle h);
 void        ptn_default_options(ptn_options *o);
 int         ptn_abi_version(void);

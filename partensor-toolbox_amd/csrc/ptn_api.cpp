@@ -101,8 +101,8 @@ struct Fail {
 // with a large node: MTTKRP of 37 x 23 x 41 189 -> 65 us, of 501 x 403 x 307 at
 // R = 33 759 -> 268 us, the order-4 tree at 200^4, R = 64 from between 7 and 95 ms to 5.3 ms.
 // The pool holds at most kPoolMax bytes (the oldest blocks are freed first), gives
-// everything back when an allocation fails or the GPU's last handle is destroyed, and is
-// guarded by a mutex.
+// everything back when an allocation fails, the GPU's last handle is destroyed or the caller
+// asks for it (ptn_release_memory), and is guarded by a mutex.
 constexpr size_t kPoolMax = (size_t)8 << 30;
 struct DevicePool {
   std::mutex mu;
@@ -1142,6 +1142,10 @@ void ptn_destroy(ptn_handle h) {
   for (hipEvent_t e : h->ev)
     if (e) (void)hipEventDestroy(e);
   delete h;
+}
+
+ptn_status ptn_release_memory(ptn_handle h) {
+  return run(h, [&] { pool_trim(pools[h->device], 0); });
 }
 
 const char *ptn_last_error(ptn_handle h) { return h ? h->err.c_str() : "null handle"; }

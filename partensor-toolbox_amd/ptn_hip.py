@@ -25,7 +25,7 @@ MTTKRP_STANDARD, MTTKRP_DIMTREE = 0, 2
 ARITH_F64, ARITH_F32, ARITH_BF16X3, ARITH_F32_F64 = 0, 1, 2, 3
 
 EXPORTED = [
-    "ptn_create", "ptn_destroy", "ptn_last_error", "ptn_default_options", "ptn_abi_version",
+    "ptn_create", "ptn_destroy", "ptn_release_memory", "ptn_last_error", "ptn_default_options", "ptn_abi_version",
     "ptn_set_tensor", "ptn_generate_tensor", "ptn_generate_factors", "ptn_tensor_norm_sq",
     "ptn_cpd", "ptn_mttkrp", "ptn_mttkrp_dimtree", "ptn_nesterov_mnls", "ptn_nesterov_mnls_noalloc",
     "ptn_sym_extremes",
@@ -95,6 +95,7 @@ def lib():
         L.ptn_create.argtypes = [ctypes.POINTER(_vp), _i]
         L.ptn_destroy.argtypes = [_vp]
         L.ptn_destroy.restype = None
+        L.ptn_release_memory.argtypes = [_vp]
         L.ptn_last_error.argtypes = [_vp]
         L.ptn_last_error.restype = ctypes.c_char_p
         L.ptn_default_options.argtypes = [ctypes.POINTER(Options)]
@@ -190,6 +191,11 @@ class Handle:
         if self._h:
             lib().ptn_destroy(self._h)
             self._h = _vp()
+
+    def release_memory(self):
+        """Give back the work buffers that calls on this GPU's handles keep between them (at most
+        8 GiB), for another allocator in the process; tensors and networks stay."""
+        self._check(lib().ptn_release_memory(self._h))
 
     def __enter__(self):
         return self

@@ -330,3 +330,28 @@ def test_freeing_blocks_does_not_stop_other_handles(on_model):
         model.model_hold_free(0)
         t.join()
         """)
+
+
+def test_the_kept_work_buffers_can_be_given_back(on_model):
+    """Up to 8 GiB of work buffers stay on the device between calls; release_memory returns them, of
+    every handle of the GPU, and leaves the tensors, the network and the calls alone."""
+    on_model(CALLS + textwrap.dedent("""
+        a, b = P.Handle(0), P.Handle(0)
+        tensor(a, (60, 50, 40))
+        tensor(b, (60, 50, 40))
+        a.release_memory()
+        before = model.model_in_use()
+        for c in calls(a)[3:11]:
+            c()
+        b.mttkrp(factors((60, 50, 40), 5), 1)
+        assert before + 4 * MB < model.model_in_use() < before + 8192 * MB
+        b.release_memory()
+        assert model.model_in_use() == before
+        for c in calls(a)[3:11]:
+            c()
+        a.release_memory()
+        assert model.model_in_use() == before
+        a.close()
+        b.close()
+        assert model.model_in_use() == 0
+        """))
