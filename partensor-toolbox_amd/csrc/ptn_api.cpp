@@ -1458,8 +1458,9 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
         if (set_up) {
           sel[n] = slot(w, n);
           fork();
-          // on one stream the set-up of rank <= 16 goes along with the FP64 contraction
-          if (one_stream && !w.mfma32 && R <= 16 && o.constraints[n] == PTN_NONNEGATIVITY) {
+          // on one stream the set-up of rank <= 16 goes along with the FP64 contraction (not into a
+          // timed pass, whose time is the contraction's alone)
+          if (one_stream && !w.mfma32 && R <= 16 && o.constraints[n] == PTN_NONNEGATIVITY && !w.kev) {
             int list[kMaxOrder];
             w.setup.ng = v_order(N, n, tree, list);
             for (int j = 0; j < w.setup.ng; ++j) w.setup.g[j] = w.G(list[j]);

@@ -590,6 +590,26 @@ def test_time_passes_events_leave_results_unchanged(h):
         t_prev = l["t_end"]
 
 
+@pytest.mark.parametrize("R", [3, 16])
+@pytest.mark.parametrize("arith", [P.ARITH_F64, P.ARITH_F32_F64])
+def test_time_passes_fp64_leaves_results_unchanged(h, arith, R):
+    """FP64 contractions of rank <= 16 take the NNLS set-up along as one of their blocks, timed ones
+    do not: the same operations in either place, so the same bits."""
+    dims = [60, 45, 50]
+    X, _ = o.make_tensor(dims, R, seed=4, snr_db=30.0)
+    init = o.gen_factors(dims, R, seed=5)
+    h.set_tensor(X, storage=P.TENSOR_BOTH)
+    for form in (P.MTTKRP_STANDARD, P.MTTKRP_DIMTREE):
+        kw = dict(max_iter=8, threshold_error=0.0, mttkrp_form=form, arith=arith)
+        F0, st0, lg0 = h.cpd(R, init, **kw)
+        F1, st1, lg1 = h.cpd(R, init, time_passes=1, **kw)
+        assert st0["f_value"] == st1["f_value"]
+        assert [(l["f_value"], l["f_accel"], l["lipschitz"], l["mu"]) for l in lg0] == \
+            [(l["f_value"], l["f_accel"], l["lipschitz"], l["mu"]) for l in lg1]
+        for a, b in zip(F0, F1):
+            assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("dims,R,seed,sweeps", [([5, 4, 6, 3, 4], 3, 5, 9), ([4, 3, 5, 3, 4, 2], 3, 6, 10),
                                                 ([3, 4, 5, 3, 2, 3], 2, 7, 10)])
 def test_als_higher_order_standard_form(h, dims, R, seed, sweeps):

@@ -355,3 +355,32 @@ def test_the_kept_work_buffers_can_be_given_back(on_model):
         b.close()
         assert model.model_in_use() == 0
         """))
+
+
+def test_timed_passes_hold_the_contraction_alone(on_model):
+    """t_pass_ms is the device time of the tensor passes: the NNLS set-up that rides along with an FP64
+    contraction of rank <= 16 (the instances whose last template parameter is true) stays out of a
+    timed one."""
+    on_model("""
+        dims, R = (60, 50, 40), 10
+        with P.Handle(0) as h:
+            tensor(h, dims)
+            for arith in (P.ARITH_F64, P.ARITH_F32_F64):
+                model.model_trace_clear()
+                kw = dict(max_iter=3, threshold_error=0.0, mttkrp_form=P.MTTKRP_DIMTREE, arith=arith)
+                try:
+                    h.cpd(R, factors(dims, R), **kw)         # (ends in an error: no kernel publishes the sweep)
+                except P.PtnError as e:
+                    assert e.code == 3
+                assert any("k_gemm" in t and "Lb1EEE" in t for t in trace())
+                model.model_trace_clear()
+                _, _, log = h.cpd(R, factors(dims, R), time_passes=1, **kw)
+                assert all(t > 0 for l in log for t in l["t_pass_ms"])
+                lines = [t for t in trace() if not t.startswith("copy")]
+                timed = [t for a, t, b in zip(lines, lines[1:], lines[2:])
+                         if a.startswith("record") and b.startswith("record")]
+                assert len([t for t in timed if "k_gemm_cm_f64" in t]) == 3
+                assert len([t for t in timed if "k_gemm_ck_f64" in t]) == 3
+                assert not any("k_gemm" in t and "Lb1EEE" in t for t in lines)
+                assert any("k_eig_extremes" in t for t in lines)
+        """)
