@@ -703,32 +703,34 @@ __global__ __launch_bounds__(256) void k_reduce_splits_runs(const f64x2 *__restr
 
 }  // namespace
 
-void gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mrows, int64_t Ktot, const KrSpec &w,
+bool gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mrows, int64_t Ktot, const KrSpec &w,
                  int ldr, int splits, double *out, const NnlsSetup *setup) {
   KrArgs a = to_args(w);
   int64_t kchunk = (Ktot + splits - 1) / splits;
   dim3 grid((unsigned)((Mrows + 63) / 64), (unsigned)splits);
   const int NT = ldr / 16;
-  if (setup) {                                     // ldr = 16
+  if (setup && NT == 1) {                          // one more block
     grid.x += 1;
     if (x64) k_gemm_cm_f64<double, 1, true><<<grid, 256, 0, s>>>(x64, Mrows, Ktot, a, ldr, kchunk, out, *setup);
     else     k_gemm_cm_f64<float, 1, true><<<grid, 256, 0, s>>>(x32, Mrows, Ktot, a, ldr, kchunk, out, *setup);
-    return;
+    return true;
   }
 #define PTN_CM(NTV)                                                                              \
   if (NT == NTV) {                                                                               \
     if (x64) k_gemm_cm_f64<double, NTV, false><<<grid, 256, 0, s>>>(x64, Mrows, Ktot, a, ldr, kchunk, out, {}); \
     else     k_gemm_cm_f64<float, NTV, false><<<grid, 256, 0, s>>>(x32, Mrows, Ktot, a, ldr, kchunk, out, {});  \
-    return;                                                                                      \
+    return false;                                                                                \
   }
   PTN_CM(1) PTN_CM(2) PTN_CM(3) PTN_CM(4)
 #undef PTN_CM
+  return false;
 }
 
-void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, int64_t C, const KrSpec &w, int ldr,
+bool gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, int64_t C, const KrSpec &w, int ldr,
                  double *T, const NnlsSetup *setup) {
   KrArgs a = to_args(w);
   const int NT = ldr / 16;
+  if (NT != 1) setup = nullptr;
   // Fibers per wave: many share each Khatri-Rao fragment, few leave more waves for the 1024
   // SIMDs (k_gemm_ck_f64)
   const int S = C >= 65536 && x64 ? 4 : C >= 16384 ? 2 : 1;
@@ -742,12 +744,13 @@ void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, 
     if (S == 4) { PTN_CKS(NTV, 4, UV) } \
     else if (S == 2) { PTN_CKS(NTV, 2, UV) } \
     else { PTN_CKS(NTV, 1, UV) }     \
-    return;                      \
+    return setup != nullptr;     \
   }
   if (setup) { PTN_CK(1, true) }
   PTN_CK(1, false) PTN_CK(2, false) PTN_CK(3, false) PTN_CK(4, false)
 #undef PTN_CK
 #undef PTN_CKS
+  return false;
 }
 
 void contract_rows(hipStream_t s, const double *T64, const float *T32, int64_t ldt, const KrSpec &spec, int outmode,

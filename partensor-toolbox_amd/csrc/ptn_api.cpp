@@ -605,12 +605,11 @@ int pick_splits_cm(const Work &w, int64_t Mrows, int64_t K) {
   return s < 1 ? 1 : (int)s;
 }
 
-// the set-up waiting to be taken along by a contraction that is about to be launched, or null
-struct TakeSetup {
-  NnlsSetup u;
-  explicit TakeSetup(Work &w) : u(w.setup) { w.setup.ng = 0; }
-  const NnlsSetup *get() const { return u.ng ? &u : nullptr; }
-};
+// the set-up waiting to be taken along by the contraction that is about to be launched, or null
+const NnlsSetup *waiting_setup(const Work &w) { return w.setup.ng ? &w.setup : nullptr; }
+void setup_taken(Work &w, bool taken) {
+  if (taken) w.setup.ng = 0;
+}
 
 Node node_cm(Work &w, const KrSpec &k, int64_t Mrows, int64_t K, int S, double *dst64, float *dst32,
              int timed = -1) {
@@ -619,7 +618,8 @@ Node node_cm(Work &w, const KrSpec &k, int64_t Mrows, int64_t K, int S, double *
   if (!w.mfma32) {
     w.pass_mark(timed, false, s);
     if (S > 1) REQUIRE(S * Mrows * w.ldr <= w.part_cap, PTN_ERR_INVALID, "partial buffer too small");
-    gemm_cm_f64(s, w.x64(), w.x32(), Mrows, K, k, w.ldr, S, S == 1 ? dst64 : w.part.p, TakeSetup(w).get());
+    setup_taken(w, gemm_cm_f64(s, w.x64(), w.x32(), Mrows, K, k, w.ldr, S, S == 1 ? dst64 : w.part.p,
+                               waiting_setup(w)));
     w.pass_mark(timed, true, s);
     if (S > 1) reduce_splits(s, w.part, S, Mrows * w.ldr, dst64, true);
     return Node{dst64, nullptr, w.ldr};
@@ -642,7 +642,7 @@ Node node_ck(Work &w, const KrSpec &k, int64_t L, int64_t C, hipStream_t s = nul
   if (!s) s = h->stream;
   if (!w.mfma32) {
     w.pass_mark(timed, false, s);
-    gemm_ck_f64(s, w.x64(), w.x32(), L, C, k, w.ldr, w.T, TakeSetup(w).get());
+    setup_taken(w, gemm_ck_f64(s, w.x64(), w.x32(), L, C, k, w.ldr, w.T, waiting_setup(w)));
     w.pass_mark(timed, true, s);
     return Node{w.T.p, nullptr, w.ldr};
   }
@@ -722,7 +722,7 @@ void mttkrp_standard(Work &w, double *base, int mode, double *M) {
       // 501 x 403 x 307 at 33 183 and 174; 640^3 at 48 641 us, with 512 blocks 665).
       const int64_t blocks = (I0 + 63) / 64, target = w.total < ((int64_t)1 << 27) ? 512 : 2048;
       const int S = (int)std::max<int64_t>(1, std::min(std::min<int64_t>(target / blocks, 256), Ktot / 32));
-      gemm_cm_f64(w.h->stream, w.x64(), w.x32(), I0, Ktot, k, w.ldr, S, w.part, TakeSetup(w).get());
+      setup_taken(w, gemm_cm_f64(w.h->stream, w.x64(), w.x32(), I0, Ktot, k, w.ldr, S, w.part, waiting_setup(w)));
       reduce_splits(w.h->stream, w.part, S, I0 * w.ldr, M, true);
     } else {
       // FP32 partials summed in FP64 by the row contraction of a 1-digit node per split
@@ -1486,7 +1486,7 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
           // waits then pass before the leaf contraction instead of one on each side of it
           if (n == 2 && early_right) join();
           contract();
-          // (a mode that contracts a node formed before has not taken it)
+          // (not taken by a mode that contracts a node formed before)
           if (w.setup.ng) {
             w.setup.ng = 0;
             prep_mode(w, w.grams, n, tree, sel[n], o, ms);

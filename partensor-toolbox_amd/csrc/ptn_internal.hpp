@@ -215,11 +215,13 @@ struct NnlsSetup {
   double *betas;
 };
 // out[split][m][r] = sum_{k in split} X[m + Mrows*k] * W(k)[r];  W = Khatri-Rao row of `w`.
-void gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mrows, int64_t Ktot,
+// A given set-up runs beside the contraction where ldr = 16; returns whether it does (otherwise it
+// is the caller's still to launch)
+bool gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mrows, int64_t Ktot,
                  const KrSpec &w, int ldr, int splits, double *out, const NnlsSetup *setup = nullptr);
 // T[c][r] = sum_{a < L} X[a + L*c] * W(a)[r]   for c < C;  W = Khatri-Rao row of `w` (a < 2^32).
-// setup (ldr = 16 only): runs beside the contraction
-void gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, int64_t C,
+// The set-up as in gemm_cm_f64.
+bool gemm_ck_f64(hipStream_t s, const double *x64, const float *x32, int64_t L, int64_t C,
                  const KrSpec &w, int ldr, double *T, const NnlsSetup *setup = nullptr);
 // out[i][r] (+)= sum over rows t of T whose output digit is i of T[t][r] * prod of the
 // other digits' factor rows.  `t` enumerates spec modes lowest fastest; `outmode` is the

@@ -384,3 +384,33 @@ def test_timed_passes_hold_the_contraction_alone(on_model):
                 assert not any("k_gemm" in t and "Lb1EEE" in t for t in lines)
                 assert any("k_eig_extremes" in t for t in lines)
         """)
+
+
+def test_a_set_up_that_a_contraction_does_not_take_is_not_lost(on_model):
+    """The FP64 contractions take an NNLS set-up along in their rank-16 instances only, and say whether
+    they did, so that the caller launches it where they did not; and without it they have no block
+    for it."""
+    on_model("""
+        lib = P.lib()
+        buf = ctypes.create_string_buffer(1 << 16)
+        spec = (ctypes.c_int64 * 33)(1, 50)                  # KrSpec: one mode of 50
+        setup = (ctypes.c_int64 * 16)()                      # NnlsSetup
+        at = ctypes.addressof(buf)
+        i64, vp = ctypes.c_int64, ctypes.c_void_p
+        cm = lib["_ZN3ptn11gemm_cm_f64EP12ihipStream_tPKdPKfllRKNS_6KrSpecEiiPdPKNS_9NnlsSetupE"]
+        ck = lib["_ZN3ptn11gemm_ck_f64EP12ihipStream_tPKdPKfllRKNS_6KrSpecEiPdPKNS_9NnlsSetupE"]
+        cm.argtypes = [vp, vp, vp, i64, i64, vp, ctypes.c_int, ctypes.c_int, vp, vp]
+        ck.argtypes = [vp, vp, vp, i64, i64, vp, ctypes.c_int, vp, vp]
+        cm.restype = ck.restype = ctypes.c_bool
+        for x64, x32 in ((at, None), (None, at)):
+            for ldr in (16, 32, 48, 64):
+                for s in (None, setup):
+                    model.model_trace_clear()
+                    took = (cm(None, x64, x32, 640, 50, spec, ldr, 1, at, s),
+                            ck(None, x64, x32, 50, 640, spec, ldr, at, s))
+                    lines = [t for t in trace() if "k_gemm" in t]
+                    want = s is not None and ldr == 16
+                    assert len(lines) == 2 and took == (want, want), (ldr, took)
+                    for t, blocks in zip(lines, (10, 40)):
+                        assert ("Lb1EEE" in t) == want and ("grid=%d," % (blocks + want)) in t, t
+        """)
