@@ -864,6 +864,52 @@ void left_node_pair(Work &w, double *cur, double *acc) {
   w.m0_ready = true;
 }
 
+// How a mode's set-up (V_n, its eigenvalues and the momentum coefficients: 22 us at rank <= 16, 50
+// at 32, 116 at 64) and its contraction share the main and the side stream.
+//   kOneStream: a hop between the streams costs the host two calls and the device 5 to 10 us of
+//     waiting.  It is not worth it where the contraction is short, or takes the set-up along as one
+//     of its blocks (FP64, rank <= 16).
+//   kContractionAside: where the contraction is shorter than the set-up, the set-up follows the Gram
+//     on the main stream and the contraction crosses to the side stream and back beside it, so that
+//     neither hop is waited for.
+//   kSetupAside: otherwise the set-up crosses.
+// The contraction's time goes by the tensor's bytes, and by what follows the reading: in the tree two
+// of a sweep's N contractions read the tensor; in the standard form each does, and from order 4 on
+// its leaf has three digits and more.  Limits in MB; us per sweep of the three (one stream /
+// contraction aside / set-up aside):
+//   tree: 2 to 8 modes alike.  R <= 16 FP64 340^3 (300 MB) 360 / 398 / 385, 97 x 94 x 94 x 91 (595 MB)
+//     1394 / 1465 / 1481; FP32 70 x 67^2 x 64 (77 MB) 389 / 421 / 425; R = 24 FP64 332^3 (279 MB)
+//     463 / 431 / 426; R = 48 70 x 67^2 x 64 (153 MB) 1165 / 1057 / 1112.
+//   standard, R <= 16: FP64 order 3 and 4 389^3 (449 MB) 588 / 627 / 591, 426^3 714 / 746 / 711; order 5
+//     R = 6 27^5 (110 MB) 718 / 811 / 751, R = 16 16^5 (8 MB) 365 / 379 / 419, 21^5 (31 MB) 502 / 520 /
+//     469; order 6 9^6 (4 MB) 464 / 484 / 497, 10^6 548 / 569 / 498.  FP32 and BF16x3 147^3 (12 MB)
+//     263 / 283 / 263, 192^3 (27 MB) 305 / 307 / 295, 70 x 67^2 x 64 (77 MB) 563 / 572 / 526; order 5
+//     12^5 (1 MB) 354 / 385 / 370, 15^5 (3 MB) 417 / 452 / 409.
+//   standard, larger ranks: order 3 FP64 R = 20 257^3 (130 MB) 403 / 376 / 377, 297^3 440 / 413 / 398;
+//     R = 40 307^3 (221 MB) 781 / 634 / 703, 374^3 1055 / 905 / 883; R = 64 435^3 (628 MB) 1558 / 1352 /
+//     1516; BF16x3 R = 20 251^3 (60 MB) 395 / 370 / 380, 276^3 436 / 411 / 397, R = 64 508^3 (500 MB) 1331 /
+//     1046 / 1072.  Order 4 FP64 R = 32 67 x 64^2 x 61 (128 MB) 698 / 576 / 609, 75 x 72^2 x 69 (205 MB)
+//     875 / 750 / 740; FP32 76 x 73^2 x 70 (108 MB) 791 / 683 / 705, 88 x 85^2 x 82 (199 MB) 977 / 856 /
+//     825.  Order 5 FP64 R = 24 16^5 (8 MB) 567 / 476 / 534, 21^5 792 / 710 / 657; FP32 15^5 (3 MB)
+//     582 / 505 / 535, 18^5 (7 MB) 677 / 617 / 583.
+enum Schedule { kOneStream, kContractionAside, kSetupAside };
+Schedule schedule_for(int N, int R, bool tree, bool fp64, int64_t bytes) {
+  int64_t one, aside;
+  if (R <= 16) {
+    aside = tree ? 128 : 0;
+    if (tree || N <= 4) one = fp64 ? 600 : tree ? 96 : 16;
+    else one = fp64 ? (R <= 8 ? 150 : N == 5 ? 12 : 5) : N == 5 ? 4 : 2;
+  } else {
+    one = R <= 32 && N == 3 && fp64 ? 8 : 0;
+    if (tree) aside = R <= 32 ? 288 : 640;
+    else if (N == 3) aside = fp64 ? 12 * (R - 10) : R * R / 7 + 6;
+    else if (N == 4) aside = fp64 ? R * R / 7 + 6 : 5 * (R - 8);
+    else if (N == 5) aside = fp64 ? R / 2 : R / 6;
+    else aside = fp64 ? R / 5 : R / 12;
+  }
+  return bytes <= one << 20 ? kOneStream : bytes <= aside << 20 ? kContractionAside : kSetupAside;
+}
+
 // The main and side streams exchanged while the scope lasts: what is enqueued on the main stream
 // goes to the side stream.
 struct StreamsSwapped {
@@ -1189,7 +1235,7 @@ ptn_status run(ptn_handle h, const std::function<void()> &fn) {
 
 // A tensor's memory is not the pool's: a program that sets a small tensor, or none, in the place of
 // a large one has the memory back for whatever else it runs.  Only a tensor of the same size takes
-// the block over (hipFree and hipMalloc of 0.5 GB: 0.7 ms).
+// the block over (ptn_set_tensor of 100^3 in FP64 238 us so, 283 with hipFree and hipMalloc).
 void drop_tensor(ptn_handle h) {
   if (h->x64) (void)hipFree(h->x64);
   if (h->x32) (void)hipFree(h->x32);
@@ -1360,23 +1406,14 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
 
     // The side stream forms V_n, its eigenvalues and the momentum coefficients of mode n
     // while the main stream contracts the tensor for mode n (small tensors: the other way
-    // round, eig_first below, or one after the other); during the line-search pass it also
+    // round, or one after the other, schedule_for); during the line-search pass it also
     // forms the accelerated factors' Grams, V_hat, the sweep's cost and both mode-0 set-ups of
     // the next sweep.  The aux stream forms the order-3 tree's right node (right_node_early).
     // All three run at the default priority.
-    // A hop between the streams costs the host two calls and the device 5 to 10 us of waiting, so
-    // where a mode's contraction is shorter than that and little of the eigen routine, or takes the
-    // set-up along as one of its blocks (FP64 contractions, R <= 16), everything stays on one
-    // stream.  Sweeps on one / on two, R <= 16, FP64: 20^3 147 / 210 us, 64^3 168 / 216, 100^3 188 /
-    // 215, 301 x 205 x 150 (74 MB) 215 / 278, 300^3 (216 MB) 298 / 343, 400^3 (512 MB) 580 / 585 and
-    // in the tree 483 / 511, 500 x 500 x 400 (800 MB) 921 / 907; FP32 100^3 253 / 270, 240^3 (55 MB)
-    // the same.  R <= 32, where the eigen routine takes 50 us, order 3 on the FP64 matrix cores:
-    // 64^3 296 / 321, 100^3 (8 MB) 320 / 326, 150^3 (27 MB) the same, 200^3 (64 MB) 318 / 304, but
-    // with the more and longer kernels of other contractions beside it 64^3 BF16x3 299 / 282, 30^4
-    // 437 / 422, FP32 438 / 392; R > 32 (116 us): 100^3 560 / 549.
     const bool early_right = tree && w.mfma32 && N == 3;
-    const int64_t one_bytes = (int64_t)(R <= 16 ? (w.mfma32 ? 96 : 600) : R <= 32 && N == 3 && !w.mfma32 ? 8 : 0) << 20;
-    const bool one_stream = !early_right && w.total * (w.f32 ? 4 : 8) <= one_bytes;
+    const Schedule sched =
+        early_right ? kSetupAside : schedule_for(N, R, tree, !w.mfma32, w.total * (w.f32 ? 4 : 8));
+    const bool one_stream = sched == kOneStream;
     hipStream_t ms = h->stream, ss = one_stream ? ms : h->side;
     auto fork = [&] {      // side waits for the main stream's work so far
       if (one_stream) return;
@@ -1440,17 +1477,9 @@ ptn_status ptn_cpd(ptn_handle h, int R, const double *init_packed, const ptn_opt
       // decision, so it runs on the side stream beside the next pass (Normalize leaves
       // the last factor and its Gram as they are unless it is the weight factor)
       const bool side_cost = step_now && pair && !(o.normalization && !all_orth && wf == last);
-      // A tensor that is read in less time than the eigen routine takes (22, 49 and 116 us at
-      // the three padded ranks; a contraction reads about 4.5 TB/s): the set-up, then the longer
-      // of the two, follows the Gram on the main stream, and the contraction crosses to the side
-      // stream and back beside it, so neither hop is waited for.  Sweeps per this and the other
-      // order (with a routine of 28, 65 and 150 us): 200^3 R = 20 342 / 375, 400^3 R = 64 (512 MB)
-      // 1232 / 1452, 100^3 R = 10 229 / 269; 300^3 R = 16 (216 MB) 394 / 387.
-      const int64_t eig_bytes = (int64_t)(R <= 16 ? 128 : R <= 32 ? 288 : 640) << 20;
-      const bool short_read = !early_right && !one_stream && w.total * (w.f32 ? 4 : 8) <= eig_bytes;
       for (int n = 0; n < N; ++n) {
         const bool set_up = !(n == 0 && prepped0);
-        const bool eig_first = short_read && o.constraints[n] == PTN_NONNEGATIVITY;
+        const bool eig_first = sched == kContractionAside && o.constraints[n] == PTN_NONNEGATIVITY;
         auto contract = [&] {
           if (tree) mttkrp_tree(w, w.fac, n, w.M);
           else mttkrp_standard(w, w.fac, n, w.M);

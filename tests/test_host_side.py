@@ -414,3 +414,65 @@ def test_a_set_up_that_a_contraction_does_not_take_is_not_lost(on_model):
                     for t, blocks in zip(lines, (10, 40)):
                         assert ("Lb1EEE" in t) == want and ("grid=%d," % (blocks + want)) in t, t
         """)
+
+
+def test_schedules_of_a_sweep(on_model):
+    """Which streams a sweep's set-ups and contractions take, on both sides of every limit (schedule_for):
+    all on one, the contraction aside, or the set-up aside.  Whatever aside is, the update waits for
+    both."""
+    on_model("""
+        def schedule(h, dims, R, form, arith, cons):
+            model.model_trace_clear()
+            kw = dict(max_iter=2, threshold_error=0.0, mttkrp_form=form, arith=arith, time_passes=1)
+            h.cpd(R, factors(dims, R), constraints=cons, **kw)
+            lines = trace()
+            lines = lines[next(i for i, t in enumerate(lines) if "stream=0 blocking" in t):]    # the sweeps
+            stream = lambda what: [t.split("stream=")[1].split()[0] for t in lines if what in t]
+            update = set(stream("k_nnls_iterate"))
+            assert len(update) == 1
+            nnls = next(k for k, c in enumerate(cons) if c == 1)
+            setup, gemm = set(stream("k_eig_extremes")), stream("k_gemm_c")
+            if not stream("wait"):
+                assert setup == update == set(gemm)
+                return "one"
+            if setup == update:
+                assert set(gemm) - update
+                return "contraction"
+            assert update <= set(gemm) and not setup & set(gemm)
+            return "set-up"
+
+        def cubes(order, mb, size):
+            d = round((mb * MB / size) ** (1.0 / order))
+            return [d] * order
+
+        std, tree = P.MTTKRP_STANDARD, P.MTTKRP_DIMTREE
+        # order, rank, form, FP64?, limit of one stream, limit of the contraction aside (MB)
+        rules = [(3, 16, std, 1, 600, 0), (3, 16, tree, 1, 600, 0), (4, 10, std, 1, 600, 0), (5, 8, std, 1, 150, 0),
+                 (5, 9, std, 1, 12, 0), (6, 16, std, 1, 5, 0), (6, 16, tree, 1, 600, 0), (3, 16, std, 0, 16, 0),
+                 (4, 5, std, 0, 16, 0), (5, 5, std, 0, 4, 0), (6, 5, std, 0, 2, 0), (4, 16, tree, 0, 96, 128),
+                 (3, 17, std, 1, 8, 84), (3, 32, tree, 1, 8, 288), (3, 33, std, 1, 0, 276), (3, 64, tree, 1, 0, 640),
+                 (3, 20, std, 0, 0, 63), (3, 64, std, 0, 0, 591), (4, 20, std, 1, 0, 63), (4, 20, std, 0, 0, 60),
+                 (4, 24, tree, 0, 0, 288), (5, 24, std, 1, 0, 12), (5, 24, std, 0, 0, 4), (6, 25, std, 1, 0, 5),
+                 (6, 24, std, 0, 0, 2), (7, 40, tree, 1, 0, 640)]
+        for order, R, form, fp64, one, aside in rules:
+            seen = []
+            for lim in sorted({one, aside}):
+                for mb in (lim * 0.75, lim * 1.3) if lim else (0.5,):
+                    for arith, size in ((P.ARITH_F64, 8), (P.ARITH_F32_F64, 4)) if fp64 else \\
+                            ((P.ARITH_F32, 4), (P.ARITH_BF16X3, 4)):
+                        dims = cubes(order, mb, size)
+                        got = np.prod([float(d) for d in dims]) * size / MB
+                        if (got - lim) * (mb - lim) <= 0:      # (small orders jump past the limit)
+                            continue
+                        with P.Handle(0) as h:
+                            tensor(h, dims, P.TENSOR_F64 if arith == P.ARITH_F64 else P.TENSOR_F32)
+                            want = "one" if got <= one else "contraction" if got <= aside else "set-up"
+                            got_s = schedule(h, dims, R, form, arith, [1] * order)
+                            assert got_s == want, (order, R, form, arith, dims, got_s, want)
+                            seen.append(want)
+            assert len(set(seen)) == 1 + (one > 0) + (aside > one) or order >= 5, (order, R, seen)
+        # the order-3 tree with FP32 products keeps its own (the right node on a third stream)
+        with P.Handle(0) as h:
+            tensor(h, (30, 30, 30), P.TENSOR_F32)
+            assert schedule(h, (30, 30, 30), 5, tree, P.ARITH_F32, [1, 1, 1]) == "set-up"
+        """)
