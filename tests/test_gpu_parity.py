@@ -428,6 +428,74 @@ def test_als_on_one_stream_and_on_two(h, dims, R):
         _als_parity(h, X, R, init, mttkrp_form=form, oform=_oform(form), max_iter=6, threshold_error=0.0)
 
 
+@pytest.mark.parametrize("arith", [P.ARITH_F32, P.ARITH_BF16X3])
+@pytest.mark.parametrize("dims,R,cons", [
+    ([40, 30, 20], 16, [1, 1, 1]), ([30, 25, 20, 12], 16, [1, 1, 1, 1]),        # one stream
+    ([40, 30, 20], 17, [1, 1, 1]), ([13, 9, 10, 8], 17, [1, 1, 1, 1]),          # the contraction aside
+    ([45, 40, 30, 20], 33, [1, 1, 1, 1]), ([8, 7, 9, 6, 5], 24, [1, 1, 1, 1, 1]),
+    ([175, 170, 160], 10, [1, 1, 1]), ([60, 55, 50, 45], 12, [1, 1, 1, 1]),     # the set-up aside (standard form)
+    ([24, 22, 20, 18, 10], 20, [1, 1, 1, 1, 1]),
+    ([60, 50, 40], 5, [1, 2, 0]), ([60, 50, 40], 20, [0, 1, 2]), ([24, 20, 22, 26], 20, [1, 0, 1, 2])])
+def test_als_fp32_products_on_every_schedule(h, arith, dims, R, cons):
+    """FP32 and BF16x3 contractions on each schedule of a sweep (all on one stream, the contraction
+    aside, the set-up aside), in both forms, fused and unfused, with mixed constraints.  Against the
+    FP64 oracle on the run's own line-search path: FP32 accumulation puts about 1e-6 of ||X||^2 into
+    the fit term of f^2 (1e-5 allowed), a hundred times that where unconstrained factors of large
+    norm cancel (1e-4).  A second run gives the same bits: nothing read early or late."""
+    say("FP32 schedules", dims, R, cons, "arith", arith)
+    nonneg = all(c == 1 for c in cons)
+    X, _ = o.make_tensor(dims, 5, seed=30, snr_db=25.0)
+    init = o.gen_factors(dims, R, seed=31)
+    h.set_tensor(X, storage=P.TENSOR_F32)
+    frob = float(np.sum(X * X))
+    kw = dict(max_iter=4, threshold_error=0.0, constraints=cons)
+    for form, fuse in ((P.MTTKRP_STANDARD, 0), (P.MTTKRP_DIMTREE, 0), (P.MTTKRP_DIMTREE, 1)):
+        Fg, _, lg = h.cpd(R, init, arith=arith, mttkrp_form=form, fuse_accel=fuse, **kw)
+        oform = _oform(form) if len(dims) <= 4 else o.MTTKRP_STANDARD     # (the oracle's tree ends at order 4)
+        _, _, logo = oracle_on_device_path(X, R, init, lg, tie=1e-3, mttkrp_form=oform, cost_form=o.COST_GRAM, **kw)
+        worst = max(abs(a["f_value"] ** 2 - b["f_value"] ** 2) for a, b in zip(lg, logo)) / frob
+        say("form", form, "fused", fuse, "max |f^2 - f_oracle^2| / ||X||^2 = %.2e" % worst)
+        assert worst < (1e-5 if nonneg else 1e-4)
+        Fa, _, la = h.cpd(R, init, arith=arith, mttkrp_form=form, fuse_accel=fuse, **kw)
+        assert [(l["f_value"], l["f_accel"], l["nnls_iters"]) for l in la] == \
+            [(l["f_value"], l["f_accel"], l["nnls_iters"]) for l in lg]
+        for a, b in zip(Fa, Fg):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("arith", [P.ARITH_F32, P.ARITH_BF16X3])
+def test_als_paired_pass_of_order_4_beside_the_set_up(h, arith):
+    """The paired line-search pass at order 4 and rank > 16 on a tensor too large for the contraction to
+    go aside (297 MB in FP32, over the tree's 288): fused and unfused runs take the same steps and
+    agree in every bit while they do."""
+    dims, R = [98, 96, 92, 90], 20
+    h.generate_tensor(dims, R, seed=8, snr_db=20.0, storage=P.TENSOR_F32)
+    init = o.gen_factors(dims, R, seed=9)
+    kw = dict(max_iter=4, threshold_error=0.0, mttkrp_form=P.MTTKRP_DIMTREE, arith=arith)
+    F0, st0, lg0 = h.cpd(R, init, fuse_accel=0, **kw)
+    F1, st1, lg1 = h.cpd(R, init, fuse_accel=1, **kw)
+    acc0, acc1 = [l["accel_accepted"] for l in lg0], [l["accel_accepted"] for l in lg1]
+    say("accept unfused", acc0, "fused", acc1)
+    assert [l["accel_tried"] for l in lg0] == [l["accel_tried"] for l in lg1] and any(l["accel_tried"] for l in lg0)
+    same = next((i for i, (a, b) in enumerate(zip(acc0, acc1)) if a != b), len(acc0))
+    for a, b in list(zip(lg0, lg1))[:same + 1]:
+        assert (a["f_value"], a["nnls_iters"]) == (b["f_value"], b["nnls_iters"])
+    if acc0 == acc1:
+        for a, b in zip(F0, F1):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dims,R", [([17, 17, 16, 17, 16], 24), ([20, 18, 18, 18, 16], 16), ([8, 7, 7, 8, 7, 6], 16),
+                                    ([66, 62, 60, 40], 20)])
+def test_als_fp64_set_up_aside_at_higher_orders(h, dims, R):
+    """FP64 standard-form runs of orders 4 to 6 on both sides of the limits where the set-up goes aside
+    (9.6 and 14 MB at order 5, 1 MB at order 6, 75 MB at order 4)."""
+    X, _ = o.make_tensor(dims, 5, seed=32, snr_db=25.0)
+    init = o.gen_factors(dims, R, seed=33)
+    h.set_tensor(X)
+    _als_parity(h, X, R, init, mttkrp_form=P.MTTKRP_STANDARD, max_iter=4, threshold_error=0.0)
+
+
 @pytest.mark.parametrize("I0", [1, 64, 65, 300])
 @pytest.mark.parametrize("K", [(1, 31), (4, 8), (3, 11), (30, 17), (32, 16), (27, 19), (90, 91)])
 def test_mode0_splits(h, I0, K):
