@@ -774,6 +774,76 @@ def test_work_buffers_shared_between_handles_and_threads():
     assert not bad
 
 
+def test_calls_that_fail_with_work_buffers_taken_leave_the_others_alone():
+    """As above, with calls among them that run out of memory when they already hold work buffers: an
+    NNLS solve whose iterates (256 x 2.6 million rows x 64 doubles, 341 GB) exceed the memory of the
+    GPU after its row buffers were taken, which also empties the pool under the other threads.  Every
+    worker reaches its end, every result has the bits of the call alone, and so have calls of the
+    failing handle and of a new one afterwards."""
+    import ctypes
+    import threading
+    rng = np.random.default_rng(9)
+    shapes = [((37, 23, 41), 5), ((120, 90, 70), 20), ((40, 31, 22, 9), 12), ((300, 64, 50), 40)]
+    square = np.eye(64)
+
+    def out_of_memory(hd):
+        # (the rows are not read before the iterates have their memory)
+        it, L, mu = ctypes.c_int(), ctypes.c_double(), ctypes.c_double()
+        p = square.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+        return P.lib().ptn_nesterov_mnls(hd._h, 2600000, 64, p, p, 1e-2, 1e-2, 255, p, ctypes.byref(it),
+                                         ctypes.byref(L), ctypes.byref(mu))
+
+    def calls_of(hd, dims, A, R):
+        return [lambda: hd.mttkrp(A, 1), lambda: hd.mttkrp_dimtree(A, arith=P.ARITH_F32),
+                lambda: hd.cpd(R, A, max_iter=4, threshold_error=0.0)[0]]
+
+    def equal(got, want):
+        return all(np.array_equal(g, w) for g, w in zip(got, want)) if isinstance(want, list) else \
+            np.array_equal(got, want)
+
+    tensors = [rng.standard_normal(dims) for dims, _ in shapes]
+    starts = [[rng.random((I, R)) for I in dims] for dims, R in shapes]
+    handles, calls = [], []
+    for (dims, R), X, A in zip(shapes, tensors, starts):
+        hd = P.Handle(0)
+        hd.set_tensor(X, storage=P.TENSOR_BOTH)
+        handles.append(hd)
+        calls.append(calls_of(hd, dims, A, R))
+    alone = [[c() for c in cs] for cs in calls]
+    say("failing call alone")
+    assert out_of_memory(handles[0]) == 2
+    bad, done = [], []
+
+    def work(k):
+        try:
+            for i in range(4):
+                if k == 0 and out_of_memory(handles[0]) != 2:
+                    bad.append((k, i, "ran"))
+                for j, (c, want) in enumerate(zip(calls[k], alone[k])):
+                    if not equal(c(), want):
+                        bad.append((k, i, j))
+            done.append(k)
+        except BaseException as e:                          # an exception in a thread fails no test by itself
+            bad.append((k, repr(e)))
+
+    say("four threads")
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(shapes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad and sorted(done) == list(range(len(shapes))), (bad, done)
+    assert out_of_memory(handles[0]) == 2
+    for c, want in zip(calls[0], alone[0]):
+        assert equal(c(), want)
+    with P.Handle(0) as hd:
+        hd.set_tensor(tensors[1], storage=P.TENSOR_BOTH)
+        for c, want in zip(calls_of(hd, shapes[1][0], starts[1], shapes[1][1]), alone[1]):
+            assert equal(c(), want)
+    for hd in handles:
+        hd.close()
+
+
 @pytest.mark.parametrize("R", [3, 32, 33, 64])
 @pytest.mark.parametrize("dims", [(1, 7, 9), (3, 300, 5), (31, 17, 33), (32, 64, 5), (33, 20, 30), (50, 257, 3),
                                   (97, 10, 11), (130, 9, 8)])

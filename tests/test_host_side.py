@@ -476,3 +476,41 @@ def test_schedules_of_a_sweep(on_model):
             tensor(h, (30, 30, 30), P.TENSOR_F32)
             assert schedule(h, (30, 30, 30), 5, tree, P.ARITH_F32, [1, 1, 1]) == "set-up"
         """)
+
+
+def test_failing_calls_on_several_threads(on_model):
+    """Handles on four threads, one of them running out of memory again and again with buffers taken:
+    every other call runs, no block is given to two calls at once (the model's hipFree knows its
+    blocks, and copies through them keep their values), and all memory returns at the end."""
+    on_model("""
+        import threading
+        bad, done = [], []
+        def rows(n):
+            return np.full((n, P.MLP_IN), n, np.float32), np.zeros((n, P.MLP_OUT), np.float32), np.full(n, 7, np.uint8)
+        def work(k):
+            try:
+                with P.Handle(0) as h:
+                    for i in range(12):
+                        tensor(h, (20 + k, 30, 40))
+                        h.mttkrp(factors((20 + k, 30, 40), 5 + 9 * k), i % 3)
+                        n = 30 + 17 * k + i
+                        h.mlp_data_clear()
+                        h.mlp_data_add(*rows(n))
+                        h.mlp_data_add(*rows(n))             # grows: the rows before are copied
+                        assert (h.mlp_data_get(0, 2 * n)[0] == n).all()
+                        if k == 0:
+                            try:
+                                h.nesterov(np.eye(64), np.zeros((20000, 64)), np.zeros((20000, 64)))
+                                bad.append("ran")
+                            except P.PtnError as e:
+                                assert e.code == 2
+                    done.append(k)
+            except BaseException as e:
+                bad.append((k, repr(e)))
+        model.model_limit(300 * MB)                          # (51 iterates of 20000 x 64: 522 MB)
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+        for t in threads: t.start()
+        for t in threads: t.join()
+        assert not bad and sorted(done) == [0, 1, 2, 3], (bad, done)
+        assert model.model_in_use() == 0 and model.model_pending() == 0
+        """)
