@@ -964,6 +964,35 @@ def test_orthogonal_update_is_the_polar_factor_at_every_padded_rank(h, R):
     assert np.abs(F[0].T @ F[0] - np.eye(R)).max() <= 1e-11
 
 
+@pytest.mark.parametrize("R", [2, 5, 16, 17, 33, 64])
+@pytest.mark.parametrize("scale", [0, 230, -230, "graded", "zero column"])
+def test_orthogonal_update_outside_the_short_operations_range(h, R, scale):
+    """The rotations' divisions and roots take short forms while their operands lie within 2^+-400, and the
+    operators elsewhere: tensors scaled by 2^+-230 (diagonals of M^T M about 2^+-460), columns of M from
+    2^-110 to 2^110 of the others (rotation angles beyond 2^199) and a column of zeros.  Small integers times
+    powers of two make M and its scalings exact in any order of sums, and everything after M is the
+    oracle's operation by operation, so the factors agree bit for bit (NaN of a zero column included)."""
+    rng = np.random.default_rng(R)
+    dims = [70, 9, 11]
+    X = rng.integers(-4, 5, dims).astype(np.float64)
+    init = [rng.integers(-3, 4, (I, R)).astype(np.float64) for I in dims]
+    if scale == "graded":
+        init[1] *= 2.0 ** rng.integers(-110, 111, R)
+    elif scale == "zero column":
+        init[1][:, R // 2] = 0.0
+    else:
+        X *= 2.0 ** scale
+    h.set_tensor(X)
+    assert np.array_equal(h.mttkrp(init, 0), o.mttkrp(X, init, 0))
+    kw = dict(max_iter=1, threshold_error=0.0, normalization=0, acceleration=0, constraints=[2, 4, 4])
+    F, _, _ = h.cpd(R, init, **kw)
+    Fo, _, _ = o.cpd(X, R, init, cost_form=o.COST_GRAM, **kw)
+    say("rank", R, scale, "finite", np.isfinite(F[0]).all())
+    assert np.array_equal(F[0], Fo[0], equal_nan=True)
+    if scale not in ("zero column", "graded"):
+        assert np.abs(F[0].T @ F[0] - np.eye(R)).max() <= 1e-9
+
+
 @pytest.mark.parametrize("dims,R", [([6, 5, 7, 4, 5], 3), ([4, 5, 3, 4, 3, 4], 3), ([3, 4, 3, 2, 3, 2, 3], 2),
                                     ([3, 2, 3, 2, 2, 3, 2, 3], 2)])
 def test_dimtree_higher_orders(h, dims, R):

@@ -514,3 +514,18 @@ def test_failing_calls_on_several_threads(on_model):
         assert not bad and sorted(done) == [0, 1, 2, 3], (bad, done)
         assert model.model_in_use() == 0 and model.model_pending() == 0
         """)
+
+
+def test_short_quotient_and_root_equal_the_operators(tmp_path):
+    """The quotient and square root in the kernels' dependent chains (csrc/short_ops.inc) are correctly
+    rounded over the operands their callers keep to: 24 million of each, random, next to powers of two
+    and to the middles between doubles."""
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    exe = str(tmp_path / "short_ops_check")
+    subprocess.run([cxx, "-O2", "-ffp-contract=off", "-std=c++17", "-Wall", "-I",
+                    os.path.join(os.path.dirname(ptn_hip.LIB_PATH), "csrc"), "-o", exe,
+                    os.path.join(HERE, "short_ops_check.cpp")], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout == "0\n", r.stdout
