@@ -103,10 +103,11 @@ typedef struct {
 /* ---- handle ---- */
 ptn_status  ptn_create(ptn_handle *h, int device);
 void        ptn_destroy(ptn_handle h);
-/* Work buffers of finished calls stay on the device for the next calls of any handle of the same
-   GPU, at most 8 GiB of them, until the GPU's last handle is destroyed or an allocation of this
+/* Work buffers of finished calls, and the memory of tensors of up to 128 MB that were replaced or
+   whose handle was destroyed, stay on the device for the next calls of any handle of the same GPU,
+   at most 8 GiB in all, until the GPU's last handle is destroyed or an allocation of this
    library finds no memory.  This gives them back at once (for another allocator in the process);
-   tensors, networks and training sets stay.  It may be called at any time between a handle's
+   the handles' tensors, networks and training sets stay.  It may be called at any time between a handle's
    calls, also while other handles' calls run. */
 ptn_status  ptn_release_memory(ptn_handle h);
 const char *ptn_last_error(ptn_handle h);

@@ -181,16 +181,19 @@ hipError_t pool_take(ptn_handle h, size_t size, void **p) {
 void pool_give(int device, void *p, size_t bytes) {
   DevicePool &P = pools[device];
   while (bytes <= kPoolMax) {
-    pool_trim(P, kPoolMax - bytes);
-    std::lock_guard<std::mutex> lock(P.mu);
-    if (P.held > kPoolMax - bytes) continue;   // (another call gave a block back meanwhile)
-    try {
-      P.blocks.emplace_back(p, bytes);
-      P.held += bytes;
-      return;
-    } catch (const std::bad_alloc &) {
-      break;
+    {
+      std::lock_guard<std::mutex> lock(P.mu);
+      if (P.held <= kPoolMax - bytes) {
+        try {
+          P.blocks.emplace_back(p, bytes);
+          P.held += bytes;
+          return;
+        } catch (const std::bad_alloc &) {
+          break;
+        }
+      }
     }
+    pool_trim(P, kPoolMax - bytes);
   }
   (void)hipFree(p);
 }
@@ -1233,12 +1236,25 @@ ptn_status run(ptn_handle h, const std::function<void()> &fn) {
   }
 }
 
-// A tensor's memory is not the pool's: a program that sets a small tensor, or none, in the place of
-// a large one has the memory back for whatever else it runs.  Only a tensor of the same size takes
-// the block over (ptn_set_tensor of 100^3 in FP64 238 us so, 283 with hipFree and hipMalloc).
-void drop_tensor(ptn_handle h) {
-  if (h->x64) (void)hipFree(h->x64);
-  if (h->x32) (void)hipFree(h->x32);
+// A large tensor's memory is not the pool's: a program that sets a small tensor, or none, in its
+// place has the memory back for whatever else it runs, and only a tensor of the same size takes the
+// block over.  Tensors of up to 128 MB come from the pool and return to it: a handle for each new
+// tensor of 8 MB took 3.0 ms to set up with hipMalloc and hipFree, 2.2 so (of 74 MB 25.4 and 22.6).
+constexpr size_t kPooledTensor = (size_t)128 << 20;
+size_t tensor_block(size_t bytes) { return bytes <= kPooledTensor ? pool_size(bytes) : bytes; }
+
+void take_tensor(ptn_handle h, size_t block, void **p) {
+  HIPCHK(block <= kPooledTensor ? pool_take(h, block, p) : device_malloc(h, p, block));
+}
+
+void drop_tensor(ptn_handle h) {              // (every call has waited for its streams)
+  auto give = [&](void *p, size_t block) {
+    if (!p) return;
+    if (block <= kPooledTensor) pool_give(h->device, p, block);
+    else (void)hipFree(p);
+  };
+  give(h->x64, h->x64_bytes);
+  give(h->x32, h->x32_bytes);
   h->x64 = nullptr;
   h->x32 = nullptr;
   h->x64_bytes = h->x32_bytes = 0;
@@ -1250,19 +1266,19 @@ void alloc_tensor(ptn_handle h, int N, const int64_t *dims, int storage) {
   h->N = 0;                                   // no tensor until its memory is there
   h->total = prod(dims, N);
   const size_t elems = (size_t)(h->total + kTensorPad);
-  const size_t b64 = storage & PTN_TENSOR_F64 ? elems * sizeof(double) : 0;
-  const size_t b32 = storage & PTN_TENSOR_F32 ? elems * sizeof(float) : 0;
+  const size_t b64 = storage & PTN_TENSOR_F64 ? tensor_block(elems * sizeof(double)) : 0;
+  const size_t b32 = storage & PTN_TENSOR_F32 ? tensor_block(elems * sizeof(float)) : 0;
   if (b64 != h->x64_bytes || b32 != h->x32_bytes) drop_tensor(h);
   h->frob_valid = false;
   // kTensorPad zero elements after the tensor: the contiguous-K contractions read whole
   // 32-element steps, which may run past the end of the last fiber
   if (storage & PTN_TENSOR_F64) {
-    if (!h->x64) HIPCHK(device_malloc(h, (void **)&h->x64, b64));
+    if (!h->x64) take_tensor(h, b64, (void **)&h->x64);
     h->x64_bytes = b64;
     HIPCHK(hipMemsetAsync(h->x64 + h->total, 0, kTensorPad * sizeof(double), h->stream));
   }
   if (storage & PTN_TENSOR_F32) {
-    if (!h->x32) HIPCHK(device_malloc(h, (void **)&h->x32, b32));
+    if (!h->x32) take_tensor(h, b32, (void **)&h->x32);
     h->x32_bytes = b32;
     HIPCHK(hipMemsetAsync(h->x32 + h->total, 0, kTensorPad * sizeof(float), h->stream));
   }

@@ -202,8 +202,9 @@ def test_activation_buffers_that_did_not_fit_are_taken_again(on_model):
 
 
 def test_a_tensor_given_up_is_given_back(on_model):
-    """Setting another tensor, or another storage, returns the old one's memory to the device at once,
-    a tensor of the same size takes it over, and the work buffers kept between calls stay."""
+    """Setting another tensor, or another storage, returns the old one's memory to the device at once
+    (tensors of up to 128 MB to the pool), a tensor of the same size takes it over, and the work buffers
+    kept between calls stay."""
     on_model("""
         big, small = (1000, 800, 600), (30, 20, 10)
         nb, ns = 480000000, 6000
@@ -231,6 +232,19 @@ def test_a_tensor_given_up_is_given_back(on_model):
             tensor(h, big)
             h.mttkrp(factors(big, 5), 0)
             assert model.model_mallocs() == mallocs + 2      # the two copies of the tensor
+            # up to 128 MB: kept for the next handle's, and given back when asked for
+            h.release_memory()
+            tensor(h, small)
+            h.release_memory()
+            none = model.model_in_use()
+            tensor(h, (100, 400, 400), P.TENSOR_F64)
+            kept = model.model_in_use()
+            tensor(h, small)
+            with P.Handle(0) as g:
+                tensor(g, (100, 400, 400), P.TENSOR_F64)
+                assert model.model_in_use() < kept + MB, (model.model_in_use(), kept)
+            h.release_memory()
+            assert model.model_in_use() == none, (model.model_in_use(), none)
         assert model.model_in_use() == 0
         """)
 
