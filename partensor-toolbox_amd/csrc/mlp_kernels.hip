@@ -121,9 +121,10 @@ __device__ __forceinline__ void gemm_tile(const GemmNt &g, int b, __bf16 *tile) 
   }
 }
 
-// Several transposes in one launch (an epoch of 8192 rows in batches of 1024: eight launches of
-// 4.7 us a step; the layers' own results are written transposed by their products): out[c][r] = in[r][c] (bf16), 32 x 32 tiles through LDS;
-// block b belongs to the matrix whose tiles start at or before b.
+// Several transposes in one launch: out[c][r] = in[r][c] (bf16), 32 x 32 tiles through LDS; block b
+// belongs to the matrix whose tiles start at or before b.  (Eight launches of 4.7 us a step of an
+// epoch of 8192 rows in batches of 1024; the layers' own results are written transposed by their
+// products.)
 struct Transposes {
   int n;
   int first[5];                                         // first tile of each matrix, then their number

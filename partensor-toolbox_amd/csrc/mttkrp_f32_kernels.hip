@@ -501,11 +501,11 @@ __global__ __launch_bounds__(384 * NT) void k_gemm_ck_few(const float *__restric
   }
   const int64_t nstep = (L + 31) / 32, alast = 32 * (nstep - 1), nfull = nstep / 2;
   f32x4 pre[NQ];
-  auto fetch = [&](int64_t n, int q0, int q1) {
+  auto fetch = [&](int64_t n) {
     int64_t a = KS * n + (k4 & 32);
     a = (a < alast ? a : alast) + (k4 & 31);
 #pragma unroll
-    for (int q = q0; q < q1; ++q) {
+    for (int q = 0; q < NQ; ++q) {
       if constexpr (NTL) pre[q] = __builtin_nontemporal_load((const f32x4 *)(src[q] + a));
       else pre[q] = *(const f32x4u *)(src[q] + a);
     }
@@ -528,9 +528,9 @@ __global__ __launch_bounds__(384 * NT) void k_gemm_ck_few(const float *__restric
     bf16x8 h[4], l[4];
     f32x8 f[4];
   };
-  auto operand = [&](int64_t n, Frag &B, int u0, int u1) {
+  auto operand = [&](int64_t n, Frag &B) {
 #pragma unroll
-    for (int u = u0; u < u1; ++u) {
+    for (int u = 0; u < 4; ++u) {
       const int64_t s16 = 4 * n + u < 2 * nstep ? 4 * n + u : 2 * nstep - 1;
       if constexpr (MODE == kGemmBf16x3) {
         B.h[u] = whi[(s16 * NT + t) * 64 + lane];
@@ -562,8 +562,8 @@ __global__ __launch_bounds__(384 * NT) void k_gemm_ck_few(const float *__restric
   // before it (past the last tile: the last step again, not used)
   auto turn = [&](int64_t n, const Frag &cur, Frag &nxt) {
     store(n + 1);
-    operand(n + 1, nxt, 0, 4);
-    fetch(n + 2, 0, NQ);
+    operand(n + 1, nxt);
+    fetch(n + 2);
     __builtin_amdgcn_sched_barrier(0);          // the requests stay ahead of the products
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
@@ -581,10 +581,10 @@ __global__ __launch_bounds__(384 * NT) void k_gemm_ck_few(const float *__restric
     multiply(xc, 1, cur, 1);
   };
   Frag b0, b1;
-  fetch(0, 0, NQ);
-  operand(0, b0, 0, 4);
+  fetch(0);
+  operand(0, b0);
   store(0);
-  fetch(1, 0, NQ);
+  fetch(1);
   __syncthreads();
   int64_t n = 0;
   for (; n + 2 <= nfull; n += 2) {

@@ -2394,7 +2394,9 @@ ptn_status ptn_cpd_batch(ptn_handle h, const double *init_packed, const ptn_opti
       };
       // The candidates, the one more often best first.  Every problem on a block of its own
       // at once: 512 threads, on one block per CU or per two (8 .. 200 problems of modes
-      // 16 .. 128 were within 5% of each other).  More problems than CUs: 512 threads, or 256
+      // 16 .. 128 were within 5% of each other).  256 threads are slower there at any size of the
+      // modes (us per sweep, 512 / 256 threads: 32 problems of modes 4 .. 12 110 / 113, of 16 206 / 214,
+      // of 16 .. 32 217 / 239, of 32 .. 64 283 / 423; 250 of 16 .. 32 226 / 249).  More problems than CUs: 512 threads, or 256
       // with two blocks per CU, which suits many small problems (2000 of modes 16 .. 32: 1.84
       // against 1.21 ms per sweep; 512 of modes 16 .. 128: 1.18 against 1.78).  256 threads on
       // one block per CU were never best (1.02 .. 1.7 times the best of these), nor half the

@@ -277,10 +277,9 @@ void grams_all(hipStream_t s, int N, const int64_t *dims, int R, int ldr, const 
 // extreme singular values of V, GLambda and (betas != nullptr) the momentum coefficients
 void eig_extremes(hipStream_t s, int R, const double *V, NnlsParams *p, int max_inner, double *betas);
 // V = Hadamard of the ng Grams (list order), its extreme eigenvalues with GLambda, and
-// the max_inner momentum coefficients: everything an NNLS update needs besides M.
+// the max_inner momentum coefficients (betas): everything an NNLS update needs besides M.
 void nnls_setup(hipStream_t s, int R, int ng, const double *const *grams, double *V, NnlsParams *p, int max_inner,
                 double *betas);
-// betas: max_inner doubles
 // satisfaction masks of nnls_iterate: 4 words per block of 4 rows
 inline int64_t nnls_mask_words(int64_t I) { return (I + 3) / 4 * 4; }
 // hist: (max_inner + 1) x I x ldr doubles; mask: nnls_mask_words(I) words
