@@ -320,10 +320,14 @@ __global__ __launch_bounds__(256, NT >= 4 || MODE == kGemmFp32 ? 2 : 1) void k_g
 // elsewhere a line is read by two steps, and cached loads keep it (701 x 555 x 333, R = 20: 383 us
 // when a length that is no multiple of 4 was read element by element from memory, 138 now;
 // 700 x 555 x 333 184 us with non-temporal loads, 143 with cached ones).
-// FUSE: the block's fibers share one index of the last mode (c = i1 + I1 * i2, 64 consecutive
-// i1 per wave) and the epilogue multiplies each fiber row by the FP64 factor row A1[i1] and
+// FUSE: a wave's fibers share one index of the last mode (c = i1 + I1 * i2, 64 consecutive
+// i1) and the epilogue multiplies each fiber row by the FP64 factor row A1[i1] and
 // sums them: the right node of the order-3 dimension tree (X x_0 A_0, then the TTV with A_1,
-// DimTrees.hpp:668-800) in one pass, written as one partial row per (i2, i1-chunk).
+// DimTrees.hpp:668-800) in one pass, written as one partial row per (i2, i1-chunk).  The four waves
+// of a block take four consecutive chunks, whatever their i2: with a block inside one i2, I1 of 64
+// and less left three waves in four without work (13 x 50 x 7925, R = 53, FP32 139 us, with a
+// register-only kernel that packed its waves so 64, here 61; 801 x 40 x 2000 BF16x3 126 and 127,
+// 44; 800^3, R = 32 FP32 469 us, 402).
 // ---------------------------------------------------------------------------
 template <int MODE, int NT, bool FUSE, bool NTL>
 __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X, int64_t L, int64_t C, int64_t I1,
@@ -338,25 +342,31 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
   __shared__ float tile[TF * LDP + PAD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i = lane & 31, kg = lane >> 5;
-  int64_t cb, nfb, i1b = 0, i2 = 0;
-  if (FUSE) {
-    const int64_t bpf = (I1 + TF - 1) / TF;
-    i2 = blockIdx.x / bpf;
-    i1b = (blockIdx.x % bpf) * TF;
-    if (i2 * I1 >= C) return;
-    cb = i1b + I1 * i2;
-    nfb = I1 - i1b < TF ? I1 - i1b : TF;
-  } else {
-    cb = (int64_t)blockIdx.x * TF;
-    nfb = C - cb < TF ? C - cb : TF;
-  }
+  const int64_t cb = (int64_t)blockIdx.x * TF, nfb = C - cb < TF ? C - cb : TF;
+  // FUSE: chunk n of the fibers, its first index of mode 1, and its length (a chunk past the last: fiber 0)
+  const int64_t wpf = FUSE ? (I1 + 63) / 64 : 1, nchunks = FUSE ? C / I1 * wpf : 0;
+  const int64_t chunk = (int64_t)blockIdx.x * 4 + (FUSE ? __builtin_amdgcn_readfirstlane(wave) : 0);
+  auto chunk_of = [&](int64_t n, int64_t &first, int64_t &i1b, int &len) {
+    const int64_t i2 = n < nchunks ? n / wpf : 0;
+    i1b = n < nchunks ? (n - i2 * wpf) * 64 : 0;
+    first = i1b + I1 * i2;
+    len = n < nchunks ? (I1 - i1b < 64 ? (int)(I1 - i1b) : 64) : 1;
+  };
   // global side: instruction q reads fiber 32 q + tid / 8, elements 4 (tid % 8) .. + 3
   const int k4 = 4 * (tid & 7);
   const float *src[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    const int fl = 32 * q + (tid >> 3);
-    src[q] = X + L * (cb + (fl < nfb ? fl : 0)) + k4;
+    if (FUSE) {
+      int64_t first, i1b;
+      int len;
+      chunk_of((int64_t)blockIdx.x * 4 + q / 2, first, i1b, len);
+      const int f = 32 * (q & 1) + (tid >> 3);
+      src[q] = X + L * (first + (f < len ? f : 0)) + k4;
+    } else {
+      const int fl = 32 * q + (tid >> 3);
+      src[q] = X + L * (cb + (fl < nfb ? fl : 0)) + k4;
+    }
   }
   const int64_t alast = ((L - 1) / 32) * 32;
   f32x4 pre[8];
@@ -433,8 +443,8 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
       }
     }
   }
-  const int64_t wb = 64 * wave;               // the wave's first fiber within the block
   if (!FUSE) {
+    const int64_t wb = 64 * wave;             // the wave's first fiber within the block
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -447,9 +457,10 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
       }
     return;
   }
-  if (wb >= nfb) return;                      // wave-uniform
-  const int64_t wpf = (I1 + 63) / 64;
-  const int64_t chunk = i2 * wpf + (i1b + wb) / 64;
+  if (chunk >= nchunks) return;               // wave-uniform
+  int64_t first, i1b;
+  int len;
+  chunk_of(chunk, first, i1b, len);
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int col = 32 * t + i;
@@ -459,8 +470,8 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
       for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int64_t f = wb + 32 * s + 8 * (v / 4) + 4 * kg + (v % 4);
-          if (f < nfb) sum = fma((double)acc[s][t][v], A1[(i1b + f) * ldr + col], sum);
+          const int f = 32 * s + 8 * (v / 4) + 4 * kg + (v % 4);
+          if (f < len) sum = fma((double)acc[s][t][v], A1[(i1b + f) * ldr + col], sum);
         }
     }
     sum += __shfl_xor(sum, 32, 64);
@@ -734,7 +745,7 @@ void gemm_ck_f32(hipStream_t s, GemmMode mode, const float *x32, int64_t L, int6
 #undef PTN_CKF
     return;
   }
-  const int64_t blocks = fuse ? (C / fuse_I1) * ((fuse_I1 + 255) / 256) : (C + 255) / 256;
+  const int64_t blocks = fuse ? ((C / fuse_I1) * ((fuse_I1 + 63) / 64) + 3) / 4 : (C + 255) / 256;
   const dim3 g2((unsigned)blocks);
 #define PTN_CKL(MODEV, NTV, FUSEV)                                                                        \
   do {                                                                                                    \

@@ -543,3 +543,19 @@ def test_short_quotient_and_root_equal_the_operators(tmp_path):
                     os.path.join(HERE, "short_ops_check.cpp")], check=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout == "0\n", r.stdout
+
+
+def test_fused_right_node_has_no_idle_waves(on_model):
+    """The order-3 right node with its leaf contraction in one launch: chunks of 64 fibres of one index of
+    the last mode, four to a block whatever that index is."""
+    on_model("""
+        for dims in ((13, 50, 79), (30, 1, 101), (32, 64, 7), (31, 65, 9), (40, 256, 3), (64, 257, 5), (33, 300, 1)):
+            with P.Handle(0) as h:
+                tensor(h, dims, P.TENSOR_F32)
+                for arith in (P.ARITH_F32, P.ARITH_BF16X3):
+                    for R in (5, 40):
+                        model.model_trace_clear()
+                        h.mttkrp_dimtree(factors(dims, R), arith=arith)
+                        grid = [int(t.split("grid=")[1].split(",")[0]) for t in trace() if "k_gemm_ck_lds" in t]
+                        assert grid == [((dims[1] + 63) // 64 * dims[2] + 3) // 4], (dims, grid)
+        """)
