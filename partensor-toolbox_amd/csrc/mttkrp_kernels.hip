@@ -69,17 +69,25 @@ KrArgs to_args(const KrSpec &w) {
   return a;
 }
 
-// A cached load: where rows are no whole cache lines, neighbouring columns share them, and a
-// non-temporal line is fetched again for each (501 x 403 x 307 at rank 17: 140 us, cached 120;
-// 800^3 at rank 32, whole lines: 877 either way).
-template <typename TX>
-__device__ __forceinline__ double ld(const TX *p) { return (double)*p; }
+// gemm_cm's loads.  Cached ones: where columns are no whole cache lines, neighbouring ones share
+// them, and a non-temporal line is fetched again for each (501 x 403 x 307 at rank 17: 140 us, cached
+// 120), and what the 256 MB of the last-level cache hold stays there from one pass to the next.
+// NTL: non-temporal ones for FP64 columns of whole lines, and many of them, in a larger tensor, which
+// only pass through (left node of 1024^2 x 100 (0.84 GB) at rank 32 260 us cached and 245 so, of 1600 x
+// 1248 x 20 (0.32 GB) at 8 211 and 203, mode 0 of 800 x 300 x 300 at 8 113 and 107; but of 128 x 300 x
+// 1000 (0.31 GB) at 40 108 and 111, the left node of 4096 x 60 x 60 (118 MB) at 8 34 and 39, and in FP32
+// of 640^3 (1 GB) at 8 272 and 293).
+template <bool NTL, typename TX>
+__device__ __forceinline__ double ld(const TX *p) {
+  if constexpr (NTL) return (double)__builtin_nontemporal_load(p);
+  else return (double)*p;
+}
 
 // ---------------------------------------------------------------------------
 // gemm_cm: a block owns 64 consecutive rows and one k-chunk; its 4 waves take
 // interleaved k-steps of 4 columns and are summed through LDS at the end.
 // ---------------------------------------------------------------------------
-template <typename TX, int NT, bool SETUP>
+template <typename TX, int NT, bool NTL, bool SETUP>
 __global__ __launch_bounds__(256, 2) void k_gemm_cm_f64(const TX *__restrict__ X, int64_t Mrows, int64_t Ktot,
                                                      KrArgs w, int ldr, int64_t kchunk, double *__restrict__ out,
                                                      NnlsSetup setup) {
@@ -147,7 +155,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_cm_f64(const TX *__restrict__ X
     kr_next(kv, p, q);
     const TX *xp = X + Mrows * (kv ? kk : kbeg);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) a[s] = ld(xp + roff[s]);
+    for (int s = 0; s < 4; ++s) a[s] = ld<NTL>(xp + roff[s]);
     kk += 16;
   };
   auto mma_step = [&](bool kv, const double (&a)[4], const double (&p)[NT], const double (&q)[NT]) {
@@ -709,20 +717,30 @@ bool gemm_cm_f64(hipStream_t s, const double *x64, const float *x32, int64_t Mro
   int64_t kchunk = (Ktot + splits - 1) / splits;
   dim3 grid((unsigned)((Mrows + 63) / 64), (unsigned)splits);
   const int NT = ldr / 16;
-  if (setup && NT == 1) {                          // one more block
-    grid.x += 1;
-    if (x64) k_gemm_cm_f64<double, 1, true><<<grid, 256, 0, s>>>(x64, Mrows, Ktot, a, ldr, kchunk, out, *setup);
-    else     k_gemm_cm_f64<float, 1, true><<<grid, 256, 0, s>>>(x32, Mrows, Ktot, a, ldr, kchunk, out, *setup);
+  const bool ntl = x64 && Mrows % 16 == 0 && Mrows >= 512 && Mrows * Ktot > ((int64_t)32 << 20);   // (ld)
+  if (setup && NT == 1) grid.x += 1;               // one more block
+#define PTN_CML(TXV, PTR, NTV, NTLV, SETUPV, UP) \
+  k_gemm_cm_f64<TXV, NTV, NTLV, SETUPV><<<grid, 256, 0, s>>>(PTR, Mrows, Ktot, a, ldr, kchunk, out, UP)
+#define PTN_CMK(NTV, SETUPV, UP)                              \
+  do {                                                        \
+    if (ntl) PTN_CML(double, x64, NTV, true, SETUPV, UP);       \
+    else if (x64) PTN_CML(double, x64, NTV, false, SETUPV, UP); \
+    else PTN_CML(float, x32, NTV, false, SETUPV, UP);           \
+  } while (0)
+  if (setup && NT == 1) {
+    PTN_CMK(1, true, *setup);
     return true;
   }
-#define PTN_CM(NTV)                                                                              \
-  if (NT == NTV) {                                                                               \
-    if (x64) k_gemm_cm_f64<double, NTV, false><<<grid, 256, 0, s>>>(x64, Mrows, Ktot, a, ldr, kchunk, out, {}); \
-    else     k_gemm_cm_f64<float, NTV, false><<<grid, 256, 0, s>>>(x32, Mrows, Ktot, a, ldr, kchunk, out, {});  \
-    return false;                                                                                \
+  const NnlsSetup none{};
+#define PTN_CM(NTV)              \
+  if (NT == NTV) {               \
+    PTN_CMK(NTV, false, none);   \
+    return false;                \
   }
   PTN_CM(1) PTN_CM(2) PTN_CM(3) PTN_CM(4)
 #undef PTN_CM
+#undef PTN_CMK
+#undef PTN_CML
   return false;
 }
 

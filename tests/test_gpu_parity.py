@@ -514,6 +514,22 @@ def test_mode0_splits(h, I0, K):
         assert P.rel_err(h.mttkrp(A, 0, arith=P.ARITH_F32_F64), o.mttkrp(X32, A, 0)) <= 1e-12
 
 
+@pytest.mark.parametrize("dims", [(512, 512, 128), (512, 512, 129), (16, 1448, 1500), (257, 256, 511)])
+def test_fp64_column_contraction_at_the_cache_size(h, dims):
+    """Mode 0 and the left node on both sides of 256 MB, where FP64 columns of whole cache lines go over to
+    non-temporal loads.  X = [[B]] from the library's generator, so M_n = B_n (Hadamard of B_k^T A_k):
+    sums of up to 2.2 million positive terms in FP64, about 2e6^0.5 roundings: 1e-12."""
+    R = 17
+    h.generate_tensor(list(dims), 3, seed=5, storage=P.TENSOR_F64)
+    B = o.gen_factors(list(dims), 3, seed=5)
+    rng = np.random.default_rng(3)
+    A = [rng.random((I, R)) for I in dims]
+    want = [B[n] @ np.prod([B[k].T @ A[k] for k in range(3) if k != n], axis=0) for n in range(3)]
+    assert P.rel_err(h.mttkrp(A, 0), want[0]) <= 1e-12
+    for got, w in zip(h.mttkrp_dimtree(A), want):
+        assert P.rel_err(got, w) <= 1e-12
+
+
 @pytest.mark.parametrize("dims", [[5, 1, 7, 3], [4, 2, 1, 9], [3, 1, 1, 1], [6, 17, 5, 2], [2, 3, 40, 33], [9, 64, 3, 70]])
 @pytest.mark.parametrize("R", [3, 16, 17, 33, 64])
 def test_order4_leaf_contractions(h, dims, R):

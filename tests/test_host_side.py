@@ -559,3 +559,23 @@ def test_fused_right_node_has_no_idle_waves(on_model):
                         grid = [int(t.split("grid=")[1].split(",")[0]) for t in trace() if "k_gemm_ck_lds" in t]
                         assert grid == [((dims[1] + 63) // 64 * dims[2] + 3) // 4], (dims, grid)
         """)
+
+
+def test_loads_of_the_fp64_column_contraction(on_model):
+    """Non-temporal loads (the contraction's second-last template parameter) for FP64 tensors whose columns
+    are whole cache lines and which the last-level cache does not hold; cached ones elsewhere."""
+    on_model("""
+        for dims, storage, want in (((512, 512, 128), P.TENSOR_F64, "00"), ((512, 512, 129), P.TENSOR_F64, "11"),
+                                    ((496, 528, 140), P.TENSOR_F64, "01"), ((513, 521, 140), P.TENSOR_F64, "00"),
+                                    ((640, 640, 640), P.TENSOR_F32, "00"), ((64, 10, 10), P.TENSOR_F64, "00")):
+            with P.Handle(0) as h:
+                tensor(h, dims, storage)
+                arith = P.ARITH_F64 if storage == P.TENSOR_F64 else P.ARITH_F32_F64
+                for R in (5, 20, 40, 64):
+                    model.model_trace_clear()
+                    h.mttkrp(factors(dims, R), 0, arith=arith)
+                    h.time_contraction(0, factors(dims, R), arith=arith, iters=1)
+                    kernels = [t for t in trace() if "k_gemm_cm_f64" in t]
+                    got = [t[t.index("ELb0EEE") - 1] for t in kernels]      # mode 0, then the left node twice
+                    assert got == [want[0], want[1], want[1]], (dims, kernels)
+        """)
