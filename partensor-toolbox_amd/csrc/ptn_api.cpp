@@ -884,10 +884,11 @@ void left_node_pair(Work &w, double *cur, double *acc) {
 //     1394 / 1465 / 1481; FP32 70 x 67^2 x 64 (77 MB) 389 / 421 / 425; R = 24 FP64 332^3 (279 MB)
 //     463 / 431 / 426; R = 48 70 x 67^2 x 64 (153 MB) 1165 / 1057 / 1112.
 //   standard, R <= 16: FP64 order 3 and 4 389^3 (449 MB) 588 / 627 / 591, 426^3 714 / 746 / 711; order 5
-//     R = 6 27^5 (110 MB) 718 / 811 / 751, R = 16 16^5 (8 MB) 365 / 379 / 419, 21^5 (31 MB) 502 / 520 /
-//     469; order 6 9^6 (4 MB) 464 / 484 / 497, 10^6 548 / 569 / 498.  FP32 and BF16x3 147^3 (12 MB)
-//     263 / 283 / 263, 192^3 (27 MB) 305 / 307 / 295, 70 x 67^2 x 64 (77 MB) 563 / 572 / 526; order 5
-//     12^5 (1 MB) 354 / 385 / 370, 15^5 (3 MB) 417 / 452 / 409.
+//     R = 6 27^5 (110 MB) 718 / 811 / 751, R = 16 18^5 (14 MB) 410 / 437 / 426, 21^5 (31 MB) 502 / 520 /
+//     469; order 6 9^6 (4 MB) 464 / 484 / 497, 10^6 548 / 569 / 498.  FP32 and BF16x3, set-up aside
+//     against one stream: order 3 R = 4 128^3 (8 MB) +6%, 292^3 (95 MB) +2; R = 8 187^3 (25 MB) 0, 270^3
+//     (75 MB) -1; R = 13 128^3 +2, 161^3 (16 MB) -2, 292^3 -3; order 5 R = 4 24^5 (30 MB) +2; R = 8 14^5
+//     (2 MB) +1, 16^5 (4 MB) -1, 18^5 -3; order 6 R = 8 8^6 (1 MB) +2, 9^6 (2 MB) -5.
 //   standard, larger ranks: order 3 FP64 R = 20 257^3 (130 MB) 403 / 376 / 377, 297^3 440 / 413 / 398;
 //     R = 40 307^3 (221 MB) 781 / 634 / 703, 374^3 1055 / 905 / 883; R = 64 435^3 (628 MB) 1558 / 1352 /
 //     1516; BF16x3 R = 20 251^3 (60 MB) 395 / 370 / 380, 276^3 436 / 411 / 397, R = 64 508^3 (500 MB) 1331 /
@@ -900,8 +901,10 @@ Schedule schedule_for(int N, int R, bool tree, bool fp64, int64_t bytes) {
   int64_t one, aside;
   if (R <= 16) {
     aside = tree ? 128 : 0;
-    if (tree || N <= 4) one = fp64 ? 600 : tree ? 96 : 16;
-    else one = fp64 ? (R <= 8 ? 150 : N == 5 ? 12 : 5) : N == 5 ? 4 : 2;
+    if (tree) one = fp64 ? 600 : 96;
+    else if (N <= 4) one = fp64 ? 600 : R <= 5 ? 96 : R <= 8 ? 32 : 10;
+    else if (fp64) one = N == 5 ? (R <= 8 ? 150 : 20) : (R <= 8 ? 90 : 5);
+    else one = R <= 5 ? 32 : N == 5 ? 2 : 1;
   } else {
     one = R <= 32 && N == 3 && fp64 ? 8 : 0;
     if (tree) aside = R <= 32 ? 288 : 640;

@@ -488,8 +488,8 @@ def test_als_paired_pass_of_order_4_beside_the_set_up(h, arith):
 @pytest.mark.parametrize("dims,R", [([17, 17, 16, 17, 16], 24), ([20, 18, 18, 18, 16], 16), ([8, 7, 7, 8, 7, 6], 16),
                                     ([66, 62, 60, 40], 20)])
 def test_als_fp64_set_up_aside_at_higher_orders(h, dims, R):
-    """FP64 standard-form runs of orders 4 to 6 on both sides of the limits where the set-up goes aside
-    (9.6 and 14 MB at order 5, 1 MB at order 6, 75 MB at order 4)."""
+    """FP64 standard-form runs of orders 4 to 6 on each schedule: the contraction aside (9.6 MB of order 5 at
+    rank 24), the set-up aside (75 MB of order 4 at rank 20), one stream (orders 5 and 6 at rank 16)."""
     X, _ = o.make_tensor(dims, 5, seed=32, snr_db=25.0)
     init = o.gen_factors(dims, R, seed=33)
     h.set_tensor(X)

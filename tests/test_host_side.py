@@ -462,8 +462,10 @@ def test_schedules_of_a_sweep(on_model):
         std, tree = P.MTTKRP_STANDARD, P.MTTKRP_DIMTREE
         # order, rank, form, FP64?, limit of one stream, limit of the contraction aside (MB)
         rules = [(3, 16, std, 1, 600, 0), (3, 16, tree, 1, 600, 0), (4, 10, std, 1, 600, 0), (5, 8, std, 1, 150, 0),
-                 (5, 9, std, 1, 12, 0), (6, 16, std, 1, 5, 0), (6, 16, tree, 1, 600, 0), (3, 16, std, 0, 16, 0),
-                 (4, 5, std, 0, 16, 0), (5, 5, std, 0, 4, 0), (6, 5, std, 0, 2, 0), (4, 16, tree, 0, 96, 128),
+                 (5, 9, std, 1, 20, 0), (6, 8, std, 1, 90, 0), (6, 16, std, 1, 5, 0), (6, 16, tree, 1, 600, 0),
+                 (3, 16, std, 0, 10, 0), (3, 8, std, 0, 32, 0), (3, 5, std, 0, 96, 0), (4, 9, std, 0, 10, 0),
+                 (4, 5, std, 0, 96, 0), (5, 5, std, 0, 32, 0), (5, 6, std, 0, 2, 0), (6, 5, std, 0, 32, 0),
+                 (6, 6, std, 0, 1, 0), (4, 16, tree, 0, 96, 128),
                  (3, 17, std, 1, 8, 84), (3, 32, tree, 1, 8, 288), (3, 33, std, 1, 0, 276), (3, 64, tree, 1, 0, 640),
                  (3, 20, std, 0, 0, 63), (3, 64, std, 0, 0, 591), (4, 20, std, 1, 0, 63), (4, 20, std, 0, 0, 60),
                  (4, 24, tree, 0, 0, 288), (5, 24, std, 1, 0, 12), (5, 24, std, 0, 0, 4), (6, 25, std, 1, 0, 5),
