@@ -326,8 +326,8 @@ __global__ __launch_bounds__(256, NT >= 4 || MODE == kGemmFp32 ? 2 : 1) void k_g
 // DimTrees.hpp:668-800) in one pass, written as one partial row per (i2, i1-chunk).  The four waves
 // of a block take four consecutive chunks, whatever their i2: with a block inside one i2, I1 of 64
 // and less left three waves in four without work (13 x 50 x 7925, R = 53, FP32 139 us, with a
-// register-only kernel that packed its waves so 64, here 61; 801 x 40 x 2000 BF16x3 126 and 127,
-// 44; 800^3, R = 32 FP32 469 us, 402).
+// register-only kernel that packed its waves so 64, here 56; 801 x 40 x 2000 BF16x3 122 and 127,
+// 42; 800^3, R = 32 FP32 447 us, 389).
 // ---------------------------------------------------------------------------
 template <int MODE, int NT, bool FUSE, bool NTL>
 __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X, int64_t L, int64_t C, int64_t I1,
@@ -343,27 +343,40 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i = lane & 31, kg = lane >> 5;
   const int64_t cb = (int64_t)blockIdx.x * TF, nfb = C - cb < TF ? C - cb : TF;
-  // FUSE: chunk n of the fibers, its first index of mode 1, and its length (a chunk past the last: fiber 0)
-  const int64_t wpf = FUSE ? (I1 + 63) / 64 : 1, nchunks = FUSE ? C / I1 * wpf : 0;
-  const int64_t chunk = (int64_t)blockIdx.x * 4 + (FUSE ? __builtin_amdgcn_readfirstlane(wave) : 0);
-  auto chunk_of = [&](int64_t n, int64_t &first, int64_t &i1b, int &len) {
-    const int64_t i2 = n < nchunks ? n / wpf : 0;
-    i1b = n < nchunks ? (n - i2 * wpf) * 64 : 0;
-    first = i1b + I1 * i2;
-    len = n < nchunks ? (I1 - i1b < 64 ? (int)(I1 - i1b) : 64) : 1;
-  };
+  // FUSE: the block's four chunks (i2, r) of fibers I1 i2 + 64 r ..; a chunk past the last reads fiber 0.
+  // One 32-bit division, then steps: a 64-bit division for each chunk was 1 us of every call (34 x 21 x 22,
+  // R = 12, FP32 8.4 us, now 7.3).
+  struct Chunk {
+    uint32_t i2, r;
+  } own{0, 0};
+  const uint32_t wpf = FUSE ? (uint32_t)((I1 + 63) / 64) : 1;
   // global side: instruction q reads fiber 32 q + tid / 8, elements 4 (tid % 8) .. + 3
   const int k4 = 4 * (tid & 7);
   const float *src[8];
+  if constexpr (FUSE) {
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    const uint32_t n0 = blockIdx.x * 4;         // a grid of 2^32 threads at most: below 2^26
+    Chunk ch{n0 / wpf, 0};
+    ch.r = n0 - ch.i2 * wpf;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    if (FUSE) {
-      int64_t first, i1b;
-      int len;
-      chunk_of((int64_t)blockIdx.x * 4 + q / 2, first, i1b, len);
-      const int f = 32 * (q & 1) + (tid >> 3);
-      src[q] = X + L * (first + (f < len ? f : 0)) + k4;
-    } else {
+    for (int c = 0; c < 4; ++c) {
+      if (c == w) own = ch;
+      const bool in = (int64_t)ch.i2 * I1 < C;
+      const int64_t first = in ? I1 * ch.i2 + 64 * (int64_t)ch.r : 0;
+      const int64_t len = in ? I1 - 64 * (int64_t)ch.r : 1;
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const int f = 32 * hf + (tid >> 3);
+        src[2 * c + hf] = X + L * (first + (f < len ? f : 0)) + k4;
+      }
+      if (++ch.r == wpf) {
+        ch.r = 0;
+        ++ch.i2;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
       const int fl = 32 * q + (tid >> 3);
       src[q] = X + L * (cb + (fl < nfb ? fl : 0)) + k4;
     }
@@ -457,10 +470,9 @@ __global__ __launch_bounds__(256) void k_gemm_ck_lds(const float *__restrict__ X
       }
     return;
   }
-  if (chunk >= nchunks) return;               // wave-uniform
-  int64_t first, i1b;
-  int len;
-  chunk_of(chunk, first, i1b, len);
+  if ((int64_t)own.i2 * I1 >= C) return;      // wave-uniform
+  const int64_t i1b = 64 * (int64_t)own.r, chunk = (int64_t)own.i2 * wpf + own.r;
+  const int len = I1 - i1b < 64 ? (int)(I1 - i1b) : 64;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int col = 32 * t + i;
