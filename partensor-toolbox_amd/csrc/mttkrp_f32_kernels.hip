@@ -318,8 +318,8 @@ __global__ __launch_bounds__(256, NT >= 4 || MODE == kGemmFp32 ? 2 : 1) void k_g
 // at least 32 elements after the last) and zeroes those elements in LDS.
 // NTL: non-temporal loads where every 128 bytes are a line of their own (L a multiple of 32);
 // elsewhere a line is read by two steps, and cached loads keep it (701 x 555 x 333, R = 20: 383 us
-// when a length that is no multiple of 4 was read element by element from memory, 138 now;
-// 700 x 555 x 333 184 us with non-temporal loads, 143 with cached ones).
+// when a length that is no multiple of 4 was read element by element from memory, 124 now;
+// 700 x 555 x 333 147 us with non-temporal loads, 120 with cached ones).
 // FUSE: a wave's fibers share one index of the last mode (c = i1 + I1 * i2, 64 consecutive
 // i1) and the epilogue multiplies each fiber row by the FP64 factor row A1[i1] and
 // sums them: the right node of the order-3 dimension tree (X x_0 A_0, then the TTV with A_1,
